@@ -29,10 +29,10 @@ def _p(a: np.ndarray, t):
 
 
 def build(ref: bool | None = None) -> None:
-    """Compile liboracle.so (always) and _ref/libaffref.so (when the reference tree exists)."""
+    """Compile liboracle.so (always) and _ref/libaffref.so (where the reference's sources are)."""
     targets = ["oracle"]
     if ref is None:
-        ref = os.path.isdir(REF_TREE)
+        ref = os.path.isfile(os.path.join(REF_TREE, "src", "quant", "blockquant.cpp"))
     if ref:
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", HERE, *targets], check=True)
