@@ -66,6 +66,11 @@ constexpr int kDevCoherent = 16;
 #ifndef AFFX_LDS_PTR
 #define AFFX_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 #endif
+// Pointer to memory that no launch in flight writes, as the constant address space: a load through
+// it at a wave-uniform address is a scalar load.
+#ifndef AFFX_CONST_PTR
+#define AFFX_CONST_PTR(T, p) ((const __attribute__((address_space(4))) T*)(p))
+#endif
 __device__ __forceinline__ void pin(Unit& u) {
 #pragma unroll
   for (int i = 0; i < 20; ++i) AFFX_PIN(u.c[i]);
