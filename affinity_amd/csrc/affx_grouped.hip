@@ -12,9 +12,8 @@
 //                    input: exact for every element of at least 2^-13 of the token's largest
 //                    magnitude, where both terms are normal E4M3 numbers, and within 2^-20 of that
 //                    maximum below it; 3 when a low bf16 term is given)
-//   (each GEMM runs three times: the wide tiles, then the mid and the narrow ones, an expert's
-//   partial last tile of at most kGMid or kGNarrow column tiles of tokens, in instantiations
-//   whose MFMAs, fragment reads and direct loads cover just those columns)
+//   (each GEMM runs once per width class of its tiles, kClsCT, in an instantiation whose MFMAs,
+//   fragment reads and direct loads cover just the class's columns)
 //   grouped_gemm<0>  gate/up: (row block of 128 inter rows, token tile): 8 waves x 16 rows of
 //                    gate and the same 16 of up, K = hidden in 128-column MFMA steps, 12 column
 //                    tiles per A fragment; epilogue combines terms, applies row scales, SwiGLU,
@@ -37,11 +36,17 @@ struct Tile {
   uint32_t expert, slot0, n;
 };
 
-// Tiles of each GEMM by width class: wide (kGCT column tiles of tokens: every full tile, and a
-// partial one that needs more than kGMid), mid (an expert's partial last tile of at most kGMid) and
-// narrow (at most kGNarrow), stored in that order; each class runs in its own instantiation of the
-// GEMM.
-constexpr int kNCls = 3;
+// Tiles of each GEMM by width class, kClsCT[k] column tiles of tokens: an expert's full tiles and a
+// partial last one in the narrowest class that holds its tokens, stored widest class first; each
+// class runs in its own instantiation of the GEMM.
+constexpr int kNCls = 4;
+constexpr int kClsCT[kNCls] = {12, 8, 4, 2};
+__host__ __device__ inline uint32_t cls_ct(uint32_t k) {
+  uint32_t ct = kClsCT[0];
+  for (uint32_t q = 1; q < (uint32_t)kNCls; ++q)
+    if (q == k) ct = kClsCT[q];
+  return ct;
+}
 struct GroupedHdr {
   uint32_t n_slots;
   uint32_t tx;                     // activation terms of the gate/up input (2 or 3)
@@ -85,39 +90,47 @@ __device__ __forceinline__ void plan_scan(uint32_t (&v)[N], uint32_t* wsum, uint
   }
 }
 
-// Width class of an expert's partial last tile of r tokens (r > 0): 2 narrow, 1 mid, 0 wide; nar
-// and mid are the token capacities of the narrow and mid widths.
-__device__ __forceinline__ uint32_t tile_cls(uint32_t r, uint32_t nar, uint32_t mid) {
-  return r <= nar ? 2u : r <= mid ? 1u : 0u;
+// Width class of an expert's tile of r tokens (r > 0): the narrowest whose columns hold them; tpg
+// tokens fill one column tile.
+__device__ __forceinline__ uint32_t tile_cls(uint32_t r, uint32_t tpg) {
+  uint32_t k = 0;
+#pragma unroll
+  for (int q = 1; q < kNCls; ++q)
+    if (r <= (uint32_t)kClsCT[q] * tpg) k = q;
+  return k;
 }
-// An expert's c slots in tiles of tt tokens: how many tiles of class k it has.
-__device__ __forceinline__ uint32_t n_cls_of(uint32_t c, uint32_t tt, uint32_t nar, uint32_t mid, uint32_t k) {
+// An expert's c slots in tiles of tt tokens (the capacity of class k0, the batch's widest): how many
+// tiles of class k it has.
+__device__ __forceinline__ uint32_t n_cls_of(uint32_t c, uint32_t tt, uint32_t tpg, uint32_t k0, uint32_t k) {
   const uint32_t r = c % tt;
-  return (k == 0 ? c / tt : 0u) + (r != 0u && tile_cls(r, nar, mid) == k ? 1u : 0u);
+  return (k == k0 ? c / tt : 0u) + (r != 0u && tile_cls(r, tpg) == k ? 1u : 0u);
 }
-// Writes the tiles of one expert (slots b0 .. b0 + c - 1): the full ones from tiles[at[0]], the
-// partial one at tiles[at[its class]] (at[0] past the full ones for a wide partial tile).
-__device__ __forceinline__ void put_tiles(Tile* tiles, uint32_t e, uint32_t b0, uint32_t c, uint32_t tt, uint32_t nar,
-                                          uint32_t mid, const uint32_t (&at)[kNCls]) {
-  const uint32_t full = c / tt, r = c % tt;
-  for (uint32_t k = 0; k < full; ++k) tiles[at[0] + k] = Tile{e, b0 + k * tt, tt};
-  if (r > 0) {
-    const uint32_t k = tile_cls(r, nar, mid);
-    tiles[k == 0 ? at[0] + full : at[k]] = Tile{e, b0 + full * tt, r};
+// Writes the tiles of one expert (slots b0 .. b0 + c - 1): the full ones from tiles[at[k0]], the
+// partial one at tiles[at[its class]] (past the full ones where that is k0).
+__device__ __forceinline__ void put_tiles(Tile* tiles, uint32_t e, uint32_t b0, uint32_t c, uint32_t tt, uint32_t tpg,
+                                          uint32_t k0, const uint32_t (&at)[kNCls]) {
+  const uint32_t full = c / tt, r = c % tt, kr = r ? tile_cls(r, tpg) : kNCls;
+#pragma unroll
+  for (int k = 0; k < kNCls; ++k) {
+    if ((uint32_t)k == k0)
+      for (uint32_t i = 0; i < full; ++i) tiles[at[k] + i] = Tile{e, b0 + i * tt, tt};
+    if ((uint32_t)k == kr) tiles[at[k] + ((uint32_t)k == k0 ? full : 0u)] = Tile{e, b0 + full * tt, r};
   }
 }
 
 // start_in: a caller's slot list, expert e owning slots [start_in[e], start_in[e+1]) of n_slots_in
 // (each bound clamped to n_slots_in; a range that runs backwards is empty); null: count the routes.
 __global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
-    uint32_t* __restrict__ hist, uint32_t n_chunks, uint32_t n_experts, uint32_t tt1,
-    uint32_t tt2, uint32_t nar1, uint32_t nar2, uint32_t mid1, uint32_t mid2, uint32_t tx,
+    uint32_t* __restrict__ hist, uint32_t n_chunks, uint32_t n_experts, uint32_t k01, uint32_t k02, uint32_t tx,
     const uint32_t* __restrict__ start_in,
     uint32_t n_slots_in, uint32_t max_tiles1, uint32_t max_tiles2, GroupedHdr* __restrict__ hdr,
     uint32_t* __restrict__ offsets, Tile* __restrict__ tiles1, Tile* __restrict__ tiles2) {
   static_assert(AFFX_MAX_EXPERTS <= kPlanThreads, "one thread per expert in the scan");
   __shared__ uint32_t wsum[(1 + 2 * kNCls) * (kPlanThreads / 64)];
   const uint32_t tid = threadIdx.x;
+  // tokens per column tile, and per tile of each GEMM's widest class (k01, k02)
+  const uint32_t tpg1 = 16u / tx, tpg2 = 16u / 3u;
+  const uint32_t tt1 = cls_ct(k01) * tpg1, tt2 = cls_ct(k02) * tpg2;
   uint32_t c = 0, b0 = 0;
   if (start_in) {
     if (tid < n_experts) {
@@ -136,8 +149,8 @@ __global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
   v[0] = c;
 #pragma unroll
   for (int k = 0; k < kNCls; ++k) {
-    v[1 + k] = n_cls_of(c, tt1, nar1, mid1, k);
-    v[1 + kNCls + k] = n_cls_of(c, tt2, nar2, mid2, k);
+    v[1 + k] = n_cls_of(c, tt1, tpg1, k01, k);
+    v[1 + kNCls + k] = n_cls_of(c, tt2, tpg2, k02, k);
   }
   plan_scan<NV>(v, wsum, tot);
   if (!start_in) b0 = v[0];
@@ -166,8 +179,8 @@ __global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
       base1 += tot[1 + k];
       base2 += tot[1 + kNCls + k];
     }
-    put_tiles(tiles1, tid, b0, c, tt1, nar1, mid1, at1);
-    put_tiles(tiles2, tid, b0, c, tt2, nar2, mid2, at2);
+    put_tiles(tiles1, tid, b0, c, tt1, tpg1, k01, at1);
+    put_tiles(tiles2, tid, b0, c, tt2, tpg2, k02, at2);
   }
   if (tid == 0) {
     if (!start_in) offsets[n_experts] = tot[0];
@@ -315,7 +328,7 @@ __global__ void __launch_bounds__(256) grouped_prep_x_kernel(const uint16_t* __r
 //     the VALU, not the LDS bank conflicts, sets the pace, and fewer copies measured as fast as
 //     four or eight;
 //   - B (192 columns x 128 bytes) sits in LDS, written by direct global->LDS loads two steps at
-//     a time, two steps ahead (four buffers, one workgroup barrier per two steps), read by all
+//     a time, two steps ahead (two buffers of two steps, one workgroup barrier per two), read by all
 //     eight waves; 16-byte chunks are swizzled by column so that
 //     the fragment reads of 16 lanes hit 16 distinct bank groups;
 //   - the packed weights of the next 1024 columns stream into a register ring, each chunk
@@ -324,16 +337,29 @@ constexpr int kGW = 8;                      // waves per workgroup (two per SIMD
 constexpr int kGRT = 16 / kGW;              // 16-row tiles per wave (a workgroup covers 256 rows)
 constexpr int kGT = kGW * 64;
 constexpr int kGKC = 2;                     // codebook copies (pre-rotated tables)
-constexpr int kGCT = 12;                    // 16-column tiles of B per wave (a wide tile)
-constexpr int kGMid = 8;                    // the same for a mid tile
-constexpr int kGNarrow = 4;                 // the same for a narrow tile
-// A tile of CT column tiles (kGCT, kGMid or kGNarrow): its B columns, the bytes of one B buffer
-// (one MFMA step) and the direct-load instructions per wave per step (8 columns each).
+constexpr int kGCT = kClsCT[0];             // 16-column tiles of B per wave (a wide tile)
+// A tile of CT column tiles (one of kClsCT): its B columns, the bytes of one MFMA step of B, the
+// steps that one of the two B buffers holds, and a wave's direct-load instructions per buffer (8
+// columns of one step each).
+// Light tiles (CT = 2: at most 16 tokens of two terms, 10 of three), most tiles of a batch of a few
+// hundred tokens over 256 experts, are bound by the weights' stream and the latency around it, so
+// they run two workgroups a CU (at most 128 registers, 67 KB of LDS) instead of the four column
+// tiles' one at 165: 111 experts of one or two tokens, gate/up 196 -> 146 us (4.6 TB/s), down
+// 105 -> 79 us (hidden 4096, inter 2048; kernel trace). Per step: the products first, so that
+// the next A fragments take the registers of these; block signs and scales from the fields, not the
+// LDS table (the LDS is the busier: 1 %); the second column tile's products are passed over where
+// the tile has no token there (an instantiation of its own for one column tile took two more
+// launches and as long); four steps a buffer, so that each wave has two loads a buffer and the
+// weights have four steps to arrive (a barrier waits for the loads before it). Three column tiles
+// in this form (two registers spilled) measured the same as two, four spill 40.
 template <int CT>
 struct GTile {
+  static constexpr bool kLight = CT < 4;
   static constexpr int kCols = CT * 16;
-  static constexpr uint32_t kBuf = kCols * 128;
-  static constexpr int kDma = kCols / 8 / kGW;
+  static constexpr uint32_t kStep = kCols * 128;
+  static constexpr int kNSB = kLight ? 4 : 2;
+  static constexpr uint32_t kBuf = kNSB * kStep;
+  static constexpr int kDma = kNSB * kCols / 8 / kGW;
 };
 
 struct GemmArgs {
@@ -401,7 +427,7 @@ __device__ __forceinline__ void ring_load(Unit& u, __amdgpu_buffer_rsrc_t cr, __
 }
 
 template <int PH, int TX, int CT>
-__global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
+__global__ void __launch_bounds__(kGT, GTile<CT>::kLight ? 4 : 1) grouped_gemm_kernel(GemmArgs A) {
   constexpr int TPG = 16 / TX;  // tokens per 16-column tile
   constexpr int kHalf = kGRT / 2;  // gate/up: units [0, kHalf) gate, [kHalf, kGRT) the same rows of up
   // Persistent: workgroup b runs the items (row block, token tile) w = b, b + G, b + 2G, ... (G =
@@ -432,10 +458,13 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
 #pragma unroll
   for (int i = 0; i < kPer; ++i) cbv[i] = A.codebook[tid + (uint32_t)kGT * i];
   // this instantiation's tiles: those of its width class, stored after the wider classes' tiles
-  constexpr int cls = CT == kGCT ? 0 : CT == kGMid ? 1 : 2;
   const uint32_t* ncls = A.hdr->n_cls[PH];
-  const uint32_t n_tiles = ncls[cls];
-  const uint32_t first = (cls > 0 ? ncls[0] : 0u) + (cls > 1 ? ncls[1] : 0u);
+  uint32_t n_tiles = 0, first = 0;
+#pragma unroll
+  for (int k = 0; k < kNCls; ++k) {
+    if (kClsCT[k] > CT) first += ncls[k];
+    if (kClsCT[k] == CT) n_tiles = ncls[k];
+  }
   // (entries below max_t are allocated: read before it is known whether a tile is in use)
   const uint32_t room = A.max_tiles - min(first, A.max_tiles);
   const Tile* tiles = room ? A.tiles + first : A.tiles;
@@ -452,13 +481,13 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
   __shared__ __align__(16) uint32_t lut_s[Lut<kGKC, true>::kDwords];
   __shared__ __align__(16) uint2 blk_s[16];
   const uint8_t* btbl = reinterpret_cast<const uint8_t*>(blk_s);
-  // B of step t in buffer t % 4, written two steps at a time, two steps ahead (four separate
-  // arrays: the compiler can then tell the buffers being read from the ones being written)
+  // B of step t in buffer (t / kNSB) % 2, written kNSB steps at a time, as many steps ahead (separate
+  // arrays: the compiler can then tell the buffer being read from the one being written)
+  constexpr int NSB = GTile<CT>::kNSB;
   __shared__ __align__(16) uint8_t buf0[GTile<CT>::kBuf];
   __shared__ __align__(16) uint8_t buf1[GTile<CT>::kBuf];
-  __shared__ __align__(16) uint8_t buf2[GTile<CT>::kBuf];
-  __shared__ __align__(16) uint8_t buf3[GTile<CT>::kBuf];
-  uint32_t* rowoff = reinterpret_cast<uint32_t*>(buf3);  // set-up only, before buffer 3 is written
+  uint8_t* const buf1h = buf1 + GTile<CT>::kBuf / 2;
+  uint32_t* rowoff = reinterpret_cast<uint32_t*>(buf1h);  // set-up only, before buffer 1 is written
   __shared__ __align__(16) uint32_t rowoff_n[GTile<CT>::kCols];  // the next tile's, during the last 1024 columns
   // Staged at the start of each item by direct-to-LDS loads, so that neither the epilogue nor the
   // step to the next item waits for memory: the item's activation exponents (gate/up: one per
@@ -470,7 +499,6 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
   __shared__ __align__(16) uint32_t ep_tok[128];
   __shared__ __align__(16) uint32_t ep_tile[64];
   const uint8_t* lut = reinterpret_cast<const uint8_t*>(lut_s);
-  auto bufsel = [&](int i) -> uint8_t* { return i == 0 ? buf0 : i == 1 ? buf1 : i == 2 ? buf2 : buf3; };
 
   // ---- per-item state: the expert's planes, this wave's row tiles, the B rows -----------------
   // the wave's 16-row tiles: gate/up = gate tile rt0 (unit 0) and the same rows of up (unit 1);
@@ -531,19 +559,24 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
     if (tp < GTile<CT>::kCols)
       rowoff_n[tp] = used ? (uint32_t)A.b_off + (brow * TX + (tp & 15u) % TX) * K : (uint32_t)A.zero_off;
   };
-  // DMA lane map: instruction i of wave w writes columns 8b..8b+7 (b = GTile<CT>::kDma w + i), lane l to
-  // LDS slot l & 7 of column 8b + (l >> 3); slot p of column col holds global chunk p ^ f(col),
+  // DMA lane map: a wave's instruction i of a buffer writes columns 8b..8b+7 of one of its steps,
+  // lane l to LDS slot l & 7 of column 8b + (l >> 3) (dma_at: b and the step; light tiles spread
+  // the steps of a buffer over the waves); slot p of column col holds global chunk p ^ f(col),
   // f(col) = (c ^ (c >> 3)) & 7 with c = col & 15 (the column within its 16-column tile), that
   // is (col & 7) ^ ((col >> 3) & 1). A fragment read (lane = column c + 16 k-group) then puts lanes
   // 0-7, 8-15 (and so on) on 8 distinct 16-byte bank groups, and lanes 0-15 on 16.
   // (sized for the wide tile, a narrow one uses the first entries: with a size that depends on CT,
   // captured by the lambdas below, ROCm 7.2's hipcc emits no host stub for the kernel)
-  uint32_t roff[GTile<kGCT>::kDma];
+  constexpr int kPerStep = GTile<CT>::kLight ? GTile<CT>::kDma : GTile<CT>::kDma / 2;  // column groups of a wave
+  auto dma_b = [&](int i) -> uint32_t {  // (i < kPerStep) column group of the wave's i-th
+    return GTile<CT>::kLight ? (kPerStep * wv + (uint32_t)i) % (2u * CT) : kPerStep * wv + (uint32_t)i;
+  };
+  uint32_t roff[GTile<kGCT>::kDma / 2];
   auto roff_load = [&]() {
     const uint32_t lp = tid_now() & 63u;
 #pragma unroll
-    for (int i = 0; i < GTile<CT>::kDma; ++i) {
-      const uint32_t col = 8u * (GTile<CT>::kDma * wv + i) + (lp >> 3);
+    for (int i = 0; i < kPerStep; ++i) {
+      const uint32_t col = 8u * dma_b(i) + (lp >> 3);
       const uint32_t q = (lp & 7u) ^ ((col & 7u) ^ ((col >> 3) & 1u));
       roff[i] = rowoff[col] + (q << 4);
     }
@@ -551,18 +584,30 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
   auto roff_load_next = [&]() {
     const uint32_t lp = tid_now() & 63u;
 #pragma unroll
-    for (int i = 0; i < GTile<CT>::kDma; ++i) {
-      const uint32_t col = 8u * (GTile<CT>::kDma * wv + i) + (lp >> 3);
+    for (int i = 0; i < kPerStep; ++i) {
+      const uint32_t col = 8u * dma_b(i) + (lp >> 3);
       const uint32_t q = (lp & 7u) ^ ((col & 7u) ^ ((col >> 3) & 1u));
       roff[i] = rowoff_n[col] + (q << 4);
     }
   };
   const __amdgpu_buffer_rsrc_t wsr = buffer_rsrc(A.ws, 0xFFFFFFFFu);
-  auto dma = [&](uint8_t* buf, uint32_t step) {
+  // steps t .. t + kNSB - 1 of B into buf
+  auto dma = [&](uint8_t* buf, uint32_t t) {
+    if constexpr (GTile<CT>::kLight) {
 #pragma unroll
-    for (int i = 0; i < GTile<CT>::kDma; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wsr, AFFX_LDS_PTR(buf + (GTile<CT>::kDma * wv + i) * 1024u), 16, roff[i],
-                                               step * 128u, 0, 0);
+      for (int i = 0; i < kPerStep; ++i) {
+        const uint32_t st = (kPerStep * wv + (uint32_t)i) / (2u * CT);  // the step within the buffer
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wsr, AFFX_LDS_PTR(buf + st * GTile<CT>::kStep + dma_b(i) * 1024u), 16,
+                                                 roff[i], (t + st) * 128u, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int st = 0; st < NSB; ++st)
+#pragma unroll
+        for (int i = 0; i < kPerStep; ++i)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(wsr, AFFX_LDS_PTR(buf + st * GTile<CT>::kStep + dma_b(i) * 1024u), 16,
+                                                   roff[i], (t + st) * 128u, 0, 0);
+    }
   };
 
   // ---- set-up of the first item (B row loads first: the set-up waits for them, and loads
@@ -579,7 +624,6 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
     __syncthreads();
     roff_load();
     dma(buf0, 0);
-    dma(buf1, 1);
     __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(0));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -609,7 +653,7 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
   const __amdgpu_buffer_rsrc_t tok_r = buffer_rsrc(A.slot_tok, 4u * A.n_sl);
   const __amdgpu_buffer_rsrc_t tile_r = buffer_rsrc(tiles, (uint32_t)sizeof(Tile) * max_t);
   auto lds4 = [&](__amdgpu_buffer_rsrc_t r, uint32_t* dst, uint32_t byte_off) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, AFFX_LDS_PTR(dst), 4, lane * 4u, byte_off, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, AFFX_LDS_PTR(dst), 4, (tid_now() & 63u) * 4u, byte_off, 0, 0);
   };
   for (;;) {
     // ---- staging (one wave each; issued before the steps' loads, so the steps' exact wait
@@ -653,6 +697,7 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
     // loads there or before the epilogue was held by the memory pipeline). Needs the next item's B
     // rows staged (visible after the first barrier, so at least two sets of 1024 columns).
     const bool cont = has_next && nst >= 2u;
+    const uint32_t n_cur = tl.n;
     // the lane's table copy, fragment offsets and epilogue position (derived per item: see tid_now)
     const uint32_t lane_p = tid_now() & 63u;
     const uint32_t copy4 = (lane_p & (kGKC - 1)) * 4u;
@@ -677,21 +722,20 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
     // and the wait counts of a step are all fixed at compile time)
     auto step = [&](auto mc, uint32_t s, bool more) {
       constexpr int m = decltype(mc)::value;
-      const uint8_t* bcur = bufsel(m & 3);
-      // B of steps t + 2 and t + 3, issued at the top of even steps t into the buffers of steps
-      // t - 2 and t - 1 (read before the barrier that ended step t - 1): the workgroup then needs
-      // one barrier per two steps. Past the last step the loads repeat the last step's B into
-      // buffers nobody reads again, so the count of loads in flight is the same on every path.
-      if constexpr ((m & 1) == 0) {
-        const uint32_t t2 = s * 8u + m + 2u, t3 = t2 + 1u;
-        // (at step 6 of the last 1024 columns: the next item's steps 0 and 1, which go to buffers
-        // 0 and 1 as those of steps t + 2 and t + 3 would)
-        const bool nx = m == 6 && !more && cont;
-        if constexpr (m == 6) {
+      const uint8_t* bcur = ((m / NSB) % 2 ? buf1 : buf0) + (m % NSB) * GTile<CT>::kStep;
+      // B of the next NSB steps, issued at the top of a buffer's first step into the other buffer
+      // (read before the barrier that ended the step before): the workgroup then needs one barrier
+      // per NSB steps. Past the last step the loads repeat the last steps' B into a buffer nobody
+      // reads again, so the count of loads in flight is the same on every path.
+      if constexpr (m % NSB == 0) {
+        const uint32_t t2 = s * 8u + m + NSB;
+        // (in the last 1024 columns' last buffer: the next item's first steps, which go to buffer 0
+        // as the steps after these would)
+        const bool nx = m == 8 - NSB && !more && cont;
+        if constexpr (m == 8 - NSB) {
           if (nx) roff_load_next();
         }
-        dma(bufsel((m + 2) & 3), nx ? 0u : t2 < nsteps ? t2 : nsteps - 1u);
-        dma(bufsel((m + 3) & 3), nx ? 1u : t3 < nsteps ? t3 : nsteps - 1u);
+        dma((m / NSB) % 2 ? buf0 : buf1, nx ? 0u : t2 < nsteps ? t2 : nsteps - NSB);
       }
       __builtin_amdgcn_sched_barrier(0);
       // ring loads for the next 1024 columns; after the last ones, the same loads of tile 0 (hot
@@ -714,7 +758,7 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
       // the next 1024 columns after step 7: the ring has reloaded every register those reads use.)
       constexpr int mn = (m + 1) & 7;
       constexpr int kLook = CT >= 12 ? 4 : CT >= 8 ? 2 : 0, kFin = CT >= 12 ? 8 : CT >= 8 ? 5 : 2;
-      uint32_t rawn[kGRT][8], sxn[kGRT][4];
+      uint32_t rawn[kGRT][8], sxn[kGRT][GTile<CT>::kLight ? 2 : 4];
       v8i a_next[kGRT];
       auto bread = [&](int ct) -> v8i {
         const u32x4 lo = *reinterpret_cast<const u32x4*>(bcur + ct * 2048 + bo0);
@@ -724,6 +768,27 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
         b[4] = (int)hi[0]; b[5] = (int)hi[1]; b[6] = (int)hi[2]; b[7] = (int)hi[3];
         return b;
       };
+      if constexpr (GTile<CT>::kLight) {
+        // (four waves a SIMD: the other waves' work covers the table reads' and MFMAs' latency)
+        static_for<0, CT>([&](auto cc) {
+          constexpr int ct = decltype(cc)::value;
+          if (ct > 0 && n_cur <= (uint32_t)(ct * TPG)) return;  // no token there (the same for the whole workgroup)
+          const v8i bq = bread(ct);
+#pragma unroll
+          for (int r = 0; r < kGRT; ++r) acc[r][ct] = mfma(a_cur[r], bq, acc[r][ct]);
+        });
+        __builtin_amdgcn_sched_barrier(0);  // (the products first: their A fragments' registers are then free)
+        static_for<0, kGRT>([&](auto rc) {
+          constexpr int r = decltype(rc)::value;
+          pin_step<mn>(u[r]);
+          lut_lookup<kGKC, mn, true>(u[r], lut, btbl, copy4, rawn[r], sxn[r]);
+        });
+#pragma unroll
+        for (int r = 0; r < kGRT; ++r) {
+          a_next[r] = lut_finish(rawn[r], sxn[r]);
+          AFFX_PIN(a_next[r]);
+        }
+      } else {
       v8i bq0 = bread(0), bq1 = bread(1);
       static_for<0, CT>([&](auto cc) {
         constexpr int ct = decltype(cc)::value;
@@ -750,6 +815,7 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
         bq0 = bq1;
         if constexpr (ct + 2 < CT) bq1 = bq2;
       });
+      }
       // the accumulators are materialised here (else the compiler sinks every MFMA below all
       // eight steps' table reads and holds those in registers). They stay in VGPRs: a kernel that
       // names no AGPR gets its whole register budget as VGPRs, where one that does is split half
@@ -760,13 +826,13 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
         for (int ct = 0; ct < CT; ++ct) AFFX_PIN(acc[r][ct]);
 #pragma unroll
       for (int r = 0; r < kGRT; ++r) a_cur[r] = a_next[r];
-      // After an odd step t: the B of steps t + 1 and t + 2 (issued at the top of step t - 1) is in
-      // LDS once every wave's loads up to them have landed. Loads complete in issue order, so at
-      // most the loads issued after them may still be outstanding: the ring loads of steps t - 1
-      // and t (2 units x {0,1,1,1,1,1,1,2} by step).
-      if constexpr ((m & 1) == 1) {
+      // After a buffer's last step t: the B of the next NSB steps (issued at the top of step t - NSB + 1)
+      // is in LDS once every wave's loads up to them have landed. Loads complete in issue order, so
+      // at most the loads issued after them may still be outstanding: the ring loads of the
+      // buffer's steps (2 units x {0,1,1,1,1,1,1,2} by step).
+      if constexpr (m % NSB == NSB - 1) {
         constexpr int c[8] = {0, 1, 1, 1, 1, 1, 1, 2};
-        constexpr int k = kGRT * (c[m - 1] + c[m]);
+        constexpr int k = kGRT * (NSB == 2 ? c[m - 1] + c[m] : c[m - (NSB - 1)] + c[m - (NSB - 2)] + c[m - 1] + c[m]);
         __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(k));
         __builtin_amdgcn_s_barrier();
       }
@@ -775,7 +841,7 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
     for (uint32_t s = 0; s < nst; ++s) {
       const bool more = s + 1 < nst;
       if (!more && cont) {
-        // the next item's planes and B-row offsets (published by the barrier of step 1)
+        // the next item's planes and B-row offsets (published by the barrier of the first buffer)
         rowoff_store_next(tln, brow_staged(tln));
         set_item(tln, rbn);
       }
@@ -825,14 +891,16 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
 
     // ---- epilogue arithmetic and stores ------------------------------------------------------
     // Gate/up: the SwiGLU terms go to LDS first, term t of the tile's token j at row x of the row
-    // block (x < 128) at stg(t) + j * 128 + x (terms 0-1 in buffer 2, term 2 in buffer 3 past the
-    // B-row offsets the next item writes there; both buffers are free once the steps are done),
+    // block (x < 128) at stg(t) + j * 128 + x (terms 0-1 in the lower half of buffer 1, term 2 in its
+    // upper half past the B-row offsets the next item writes there; the buffer is free once the
+    // steps are done),
     // and then out in 16-byte pieces: each (token, term) is 128 bytes of the output row, four runs
     // of 32 at a 128-byte stride in the down GEMM's step order. (Written from the accumulator
     // lanes, two or four bytes per lane and term: 36 narrow stores per wave, whose
     // acknowledgements the next item then waited for.)
     constexpr uint32_t kTT = CT * TPG;  // tokens of a tile of this class
-    auto stg = [&](uint32_t t) -> uint8_t* { return t < 2 ? buf2 + t * kTT * 128u : buf3 + 1024u; };
+    auto stg = [&](uint32_t t) -> uint8_t* { return t < 2 ? buf1 + t * kTT * 128u : buf1h + 1024u; };
+    static_assert(2u * kTT * 128u <= GTile<CT>::kBuf / 2 && 1024u + kTT * 128u <= GTile<CT>::kBuf / 2, "");
     if constexpr (PH == 0) {
       static_for<0, kHalf>([&](auto pc) {
         constexpr int p = decltype(pc)::value;
@@ -955,7 +1023,6 @@ __global__ void __launch_bounds__(kGT, 1) grouped_gemm_kernel(GemmArgs A) {
       __syncthreads();
       roff_load();
       dma(buf0, 0);
-      dma(buf1, 1);
     }
     w += gridDim.x;
     rb = rbn;
@@ -1008,8 +1075,16 @@ struct GroupedWs {
   uint32_t max_tiles1, max_tiles2;
 };
 
-// tokens per workgroup tile: kGCT column tiles of 16 / terms tokens each
-uint32_t tile_tokens(uint32_t terms) { return kGCT * (16 / terms); }
+// The widest class a batch of T tokens needs (tokens are `terms` columns each): one of whose tiles
+// hold all tokens of an expert that every token names at most once. (An expert named more often, or
+// any slot list, is cut into more tiles of that class.) The wider classes are not launched.
+uint32_t widest_cls(uint32_t T, uint32_t terms) {
+  uint32_t k = 0;
+  for (int q = 1; q < kNCls; ++q)
+    if (T <= (uint32_t)kClsCT[q] * (16 / terms)) k = (uint32_t)q;
+  return k;
+}
+uint32_t tile_tokens(uint32_t T, uint32_t terms) { return cls_ct(widest_cls(T, terms)) * (16 / terms); }
 
 // chunks of the routes form's placement: they cover the routes and the run entries 0 .. T
 uint64_t place_chunks(uint32_t T, uint64_t P) {
@@ -1020,7 +1095,7 @@ uint64_t place_chunks(uint32_t T, uint64_t P) {
 // T tokens, room for P slots (the routes form: T * top_k)
 GroupedWs grouped_ws(uint32_t T, uint64_t P, uint32_t E, uint32_t hidden, uint32_t inter, uint32_t tx) {
   GroupedWs w;
-  const uint32_t tt1 = tile_tokens(tx), tt2 = tile_tokens(3);
+  const uint32_t tt1 = tile_tokens(T, tx), tt2 = tile_tokens(T, 3);
   w.max_tiles1 = (uint32_t)(P / tt1 + E + 1);
   w.max_tiles2 = (uint32_t)(P / tt2 + E + 1);
   uint64_t o = 0;
@@ -1096,12 +1171,8 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   A.limit = L->swiglu_limit;
   A.sigma_a = 7 - ilogbf(L->swiglu_limit * L->swiglu_limit);
 
-  const uint32_t tt1 = tile_tokens(tx), tt2 = tile_tokens(3);
+  const uint32_t k01 = widest_cls(T, tx), k02 = widest_cls(T, 3);
   const uint32_t Pp = sel ? T * K : 0u;
-  // an expert's partial last tile is narrow (mid) when its tokens fill at most kGNarrow (kGMid)
-  // column tiles
-  const uint32_t nar1 = kGNarrow * (16 / tx), nar2 = kGNarrow * (16 / 3);
-  const uint32_t mid1 = kGMid * (16 / tx), mid2 = kGMid * (16 / 3);
   const uint32_t nch = sel ? (uint32_t)place_chunks(T, Pp) : 0u;
   if (sel) {
     hipLaunchKernelGGL(grouped_hist_kernel, dim3(nch), dim3(256), 0, s, sel, Pp, T, K, L->n_experts,
@@ -1109,8 +1180,7 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
     if (int rc0 = check_launch("grouped_hist_kernel")) return rc0;
   }
   hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, (uint32_t*)(b + lay.hist), nch,
-                     L->n_experts, tt1, tt2, nar1,
-                     nar2, mid1, mid2, tx, sel ? nullptr : start, sel ? 0u : n_slots, lay.max_tiles1, lay.max_tiles2,
+                     L->n_experts, k01, k02, tx, sel ? nullptr : start, sel ? 0u : n_slots, lay.max_tiles1, lay.max_tiles2,
                      (GroupedHdr*)(b + lay.hdr), (uint32_t*)(b + lay.offsets), (Tile*)(b + lay.tiles1),
                      (Tile*)(b + lay.tiles2));
   int rc = check_launch("grouped_plan_kernel");
@@ -1135,33 +1205,33 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   if ((rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
     return rc;
   const uint32_t gmax = cus >= 8 ? (uint32_t)cus / 8u * 8u : 8u;
-  // (the mid and narrow tiles: at most one per expert)
-  auto grid = [&](uint32_t row_blocks, uint32_t tiles) {
+  // (the classes below the widest: at most one tile per expert)
+  auto grid = [&](uint32_t row_blocks, uint32_t tiles, uint32_t per_cu) {
     const uint32_t items = row_blocks * ((tiles + 7) / 8 * 8);
-    return items < gmax ? items : gmax;
+    return items < per_cu * gmax ? items : per_cu * gmax;
   };
-  const uint32_t E8 = L->n_experts < lay.max_tiles1 ? L->n_experts : lay.max_tiles1;
   A.tiles = (const Tile*)(b + lay.tiles1);
   A.max_tiles = lay.max_tiles1;
   A.b_off = lay.xq;
-  const uint32_t g1 = grid(L->inter / 128, lay.max_tiles1), gn1 = grid(L->inter / 128, E8);
-  if (tx == 2) {
-    hipLaunchKernelGGL((grouped_gemm_kernel<0, 2, kGCT>), dim3(g1), dim3(kGT), 0, s, A);
-    hipLaunchKernelGGL((grouped_gemm_kernel<0, 2, kGMid>), dim3(gn1), dim3(kGT), 0, s, A);
-    hipLaunchKernelGGL((grouped_gemm_kernel<0, 2, kGNarrow>), dim3(gn1), dim3(kGT), 0, s, A);
-  } else {
-    hipLaunchKernelGGL((grouped_gemm_kernel<0, 3, kGCT>), dim3(g1), dim3(kGT), 0, s, A);
-    hipLaunchKernelGGL((grouped_gemm_kernel<0, 3, kGMid>), dim3(gn1), dim3(kGT), 0, s, A);
-    hipLaunchKernelGGL((grouped_gemm_kernel<0, 3, kGNarrow>), dim3(gn1), dim3(kGT), 0, s, A);
-  }
+  auto each_cls = [&](auto ph, auto txc, uint32_t k0, uint32_t row_blocks, uint32_t max_tiles) {
+    constexpr int PH = decltype(ph)::value, TX = decltype(txc)::value;
+    const uint32_t part = L->n_experts < max_tiles ? L->n_experts : max_tiles;
+    static_for<0, kNCls>([&](auto kc) {
+      constexpr int k = decltype(kc)::value, CT = kClsCT[k];
+      if ((uint32_t)k < k0) return;
+      const dim3 g(grid(row_blocks, (uint32_t)k == k0 ? max_tiles : part, GTile<CT>::kLight ? 2u : 1u));
+      hipLaunchKernelGGL((grouped_gemm_kernel<PH, TX, CT>), g, dim3(kGT), 0, s, A);
+    });
+  };
+  if (tx == 2)
+    each_cls(IConst<0>{}, IConst<2>{}, k01, L->inter / 128, lay.max_tiles1);
+  else
+    each_cls(IConst<0>{}, IConst<3>{}, k01, L->inter / 128, lay.max_tiles1);
   if ((rc = check_launch("grouped_gemm_kernel (gate/up)"))) return rc;
   A.tiles = (const Tile*)(b + lay.tiles2);
   A.max_tiles = lay.max_tiles2;
   A.b_off = lay.aq;
-  const uint32_t g2 = grid(L->hidden / 256, lay.max_tiles2), gn2 = grid(L->hidden / 256, E8);
-  hipLaunchKernelGGL((grouped_gemm_kernel<1, 3, kGCT>), dim3(g2), dim3(kGT), 0, s, A);
-  hipLaunchKernelGGL((grouped_gemm_kernel<1, 3, kGMid>), dim3(gn2), dim3(kGT), 0, s, A);
-  hipLaunchKernelGGL((grouped_gemm_kernel<1, 3, kGNarrow>), dim3(gn2), dim3(kGT), 0, s, A);
+  each_cls(IConst<1>{}, IConst<3>{}, k02, L->hidden / 256, lay.max_tiles2);
   if ((rc = check_launch("grouped_gemm_kernel (down)"))) return rc;
   hipLaunchKernelGGL(grouped_combine_kernel, dim3((L->hidden / 4 + 255) / 256, T), dim3(256), 0, s,
                      (const float*)(b + lay.z), ord_d, run_d, slot_w, n_sl, L->hidden, y, accumulate);

@@ -296,7 +296,7 @@ struct IConst {
   static constexpr int value = N;
 };
 template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
+__host__ __device__ __forceinline__ void static_for(F&& f) {
   if constexpr (B < E) {
     f(IConst<B>{});
     static_for<B + 1, E>(f);

@@ -197,3 +197,34 @@ def test_engine_hook_dim_major_arenas(ax, orc, c1_codebook, layer):
 def _lib_err():
     from affinity_amd._lib import last_error
     return last_error()
+
+
+# tokens per expert at the edges of the width classes (a column tile holds 8 tokens of two terms, 5 of
+# three; classes of 2, 4, 8 and 12 column tiles) and of the batch sizes that choose the widest class
+EDGES = [[1, 5, 6, 10], [8, 9, 16, 17, 2], [11, 16, 10, 33, 1, 3], [20, 21, 32, 33, 11, 1],
+         [40, 41, 60, 61, 64, 65, 96, 97, 0, 121], [4096], [4000, 97]]
+
+
+@pytest.mark.parametrize("lo", [False, True])
+@pytest.mark.parametrize("counts", EDGES, ids=lambda c: "-".join(map(str, c)))
+def test_grouped_tile_class_edges(ax, orc, c1_codebook, layer, counts, lo):
+    """One route a token, expert e taken by counts[e] tokens in a shuffled order; one batch of 4096
+    pairs and one of 4097 (the plan in one workgroup, and in chunks). At most 64 tokens, the first and
+    last of every expert among them, against the oracle."""
+    ex, pool, hidden, inter = layer
+    rng = np.random.default_rng(sum(counts) + lo)
+    T = sum(counts)
+    sel = rng.permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.uint32).reshape(T, 1)
+    w = rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32)
+    xf = rng.standard_normal((T, hidden)).astype(np.float32)
+    hi = torch.from_numpy(xf).cuda().to(torch.bfloat16)
+    xlo = (torch.from_numpy(xf).cuda() - hi.float()).to(torch.bfloat16) if lo else None
+    xr = (hi.float() + (xlo.float() if lo else 0)).cpu().numpy()
+    y = ax.expert_ffn_grouped(pool, hi, torch.from_numpy(sel.view(np.int32)).cuda(), torch.from_numpy(w).cuda(),
+                              x_lo=xlo).cpu().numpy()
+    ends = [i for e in range(len(counts)) if counts[e] for i in np.nonzero(sel[:, 0] == e)[0][[0, -1]]]
+    pick = np.unique(np.concatenate([ends, rng.permutation(T)[:max(0, 64 - len(ends))]])).astype(int)
+    ref = _oracle(orc, ex, orc.unpack_codebook(c1_codebook), xr[pick], sel[pick], w[pick], hidden, inter)
+    assert np.isfinite(y).all()
+    for i, t in enumerate(pick):
+        assert rel_l2(y[t], ref[i]) <= TOL, (t, rel_l2(y[t], ref[i]))
