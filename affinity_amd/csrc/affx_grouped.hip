@@ -1,13 +1,15 @@
 // Prefill path: the routed experts of a whole chunk, grouped by expert (each expert's weights
 // are decoded once per tile of its tokens), on the fp8 MFMA.
 //
-//   grouped_plan     one workgroup: per-expert counts (from the routes, or from a slot list the
+//   grouped_hist     per chunk of routes: the count of each expert, and `run` (token t's routes are
+//                    entries t k .. t k + k - 1 of `ord`) and a no-slot mark in `ord` for a route
+//                    naming no expert of the layer
+//   grouped_plan     one workgroup: per-expert counts (summed over the chunks, or from a slot list the
 //                    caller built), exclusive scan, tile lists
-//   grouped_run      per route: `run` (token t's routes are entries t k .. t k + k - 1 of `ord`)
-//                    and a no-slot mark in `ord` for a route naming no expert of the layer
-//   grouped_place    one workgroup per expert: its (token, route) pairs in token order (stable),
-//                    so every slot and every output sum has a fixed order; writes the slot list
-//                    (token and weight per slot, `ord`: each token's slots in route order)
+//   grouped_place    per chunk: its (token, route) pairs in token order (stable), so every slot and
+//                    every output sum has a fixed order; writes the slot list (token, weight and
+//                    activation exponent per slot, `ord`: each token's slots in route order)
+//   grouped_plan_small  these three in one workgroup, for at most kSmallPairs routes
 //   grouped_prep_x   per token: exponent and E4M3 terms of the activation (2 terms for a bf16
 //                    input: exact for every element of at least 2^-13 of the token's largest
 //                    magnitude, where both terms are normal E4M3 numbers, and within 2^-20 of that
@@ -77,16 +79,25 @@ __device__ __forceinline__ void plan_scan(uint32_t (&v)[N], uint32_t* wsum, uint
 #pragma unroll
     for (int q = 0; q < N; ++q) wsum[q * kW + wv] = inc[q];
   __syncthreads();
+  // the waves' totals: scanned by one 16-lane run per count
+  static_assert(kW == 16 && N * kW <= kPlanThreads, "");
+  const uint32_t x = tid < N * kW ? wsum[tid] : 0u;
+  uint32_t in = x;
+#pragma unroll
+  for (int o = 1; o < (int)kW; o <<= 1) {
+    const uint32_t n = __shfl_up(in, o);
+    if ((lane & (kW - 1)) >= (uint32_t)o) in += n;
+  }
+  __syncthreads();
+  if (tid < N * kW) {
+    wsum[tid] = in - x;
+    if ((tid & (kW - 1)) == kW - 1) wsum[N * kW + tid / kW] = in;
+  }
+  __syncthreads();
 #pragma unroll
   for (int q = 0; q < N; ++q) {
-    uint32_t before = 0, all = 0;
-    for (uint32_t w = 0; w < kW; ++w) {
-      const uint32_t x = wsum[q * kW + w];
-      before += w < wv ? x : 0u;
-      all += x;
-    }
-    v[q] = before + inc[q] - v[q];
-    tot[q] = all;
+    v[q] = wsum[q * kW + wv] + inc[q] - v[q];
+    tot[q] = wsum[N * kW + q];
   }
 }
 
@@ -118,32 +129,26 @@ __device__ __forceinline__ void put_tiles(Tile* tiles, uint32_t e, uint32_t b0, 
   }
 }
 
-// start_in: a caller's slot list, expert e owning slots [start_in[e], start_in[e+1]) of n_slots_in
-// (each bound clamped to n_slots_in; a range that runs backwards is empty); null: count the routes.
-__global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
-    uint32_t* __restrict__ hist, uint32_t n_chunks, uint32_t n_experts, uint32_t k01, uint32_t k02, uint32_t tx,
-    const uint32_t* __restrict__ start_in,
-    uint32_t n_slots_in, uint32_t max_tiles1, uint32_t max_tiles2, GroupedHdr* __restrict__ hdr,
-    uint32_t* __restrict__ offsets, Tile* __restrict__ tiles1, Tile* __restrict__ tiles2) {
-  static_assert(AFFX_MAX_EXPERTS <= kPlanThreads, "one thread per expert in the scan");
-  __shared__ uint32_t wsum[(1 + 2 * kNCls) * (kPlanThreads / 64)];
+// The plan of one workgroup of kPlanThreads threads: thread e < n_experts holds expert e's count c
+// (and, with own_slots, the first slot b0 its caller chose; else the slots follow in expert order).
+// Slot and tile offsets by one exclusive scan (expert order) of the count and the tiles of each width
+// class of both GEMMs, whose widest classes are k01 and k02; writes the tiles, the header and returns
+// the expert's first slot.
+struct PlanOut {
+  GroupedHdr* hdr;
+  uint32_t* offsets;
+  Tile* tiles1;
+  Tile* tiles2;
+  uint32_t max_tiles1, max_tiles2;
+};
+constexpr uint32_t kPlanSums = (1 + 2 * kNCls) * (kPlanThreads / 64 + 1);
+__device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own_slots, uint32_t n_slots_in,
+                                               uint32_t n_experts, uint32_t k01, uint32_t k02, uint32_t tx,
+                                               uint32_t* wsum, const PlanOut& o) {
   const uint32_t tid = threadIdx.x;
-  // tokens per column tile, and per tile of each GEMM's widest class (k01, k02)
+  // tokens per column tile, and per tile of each GEMM's widest class
   const uint32_t tpg1 = 16u / tx, tpg2 = 16u / 3u;
   const uint32_t tt1 = cls_ct(k01) * tpg1, tt2 = cls_ct(k02) * tpg2;
-  uint32_t c = 0, b0 = 0;
-  if (start_in) {
-    if (tid < n_experts) {
-      const uint32_t a = min(start_in[tid], n_slots_in), b = min(start_in[tid + 1], n_slots_in);
-      c = b > a ? b - a : 0u;
-      b0 = a;
-    }
-  } else if (tid < n_experts) {
-    // an expert's count: the sum of its chunk counts (grouped_hist_kernel), in chunk order
-    for (uint32_t b = 0; b < n_chunks; ++b) c += hist[(uint64_t)b * n_experts + tid];
-  }
-  // slot offsets and tile offsets: one exclusive scan (expert order) of the count and the tiles of
-  // each width class of both GEMMs
   constexpr int NV = 1 + 2 * kNCls;
   uint32_t v[NV], tot[NV];
   v[0] = c;
@@ -153,24 +158,14 @@ __global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
     v[1 + kNCls + k] = n_cls_of(c, tt2, tpg2, k02, k);
   }
   plan_scan<NV>(v, wsum, tot);
-  if (!start_in) b0 = v[0];
+  if (!own_slots) b0 = v[0];
   uint32_t need1 = 0, need2 = 0;
 #pragma unroll
   for (int k = 0; k < kNCls; ++k) { need1 += tot[1 + k]; need2 += tot[1 + kNCls + k]; }
   // a caller's overlapping ranges could ask for more tiles than the workspace holds: then no tile
-  const bool fits = need1 <= max_tiles1 && need2 <= max_tiles2;
-  if (!start_in && tid < n_experts) {
-    // each chunk's first slot of this expert: its offset plus the counts of the chunks before
-    uint32_t at = v[0];
-    for (uint32_t b = 0; b < n_chunks; ++b) {
-      const uint64_t hi = (uint64_t)b * n_experts + tid;
-      const uint32_t cb = hist[hi];
-      hist[hi] = at;
-      at += cb;
-    }
-  }
+  const bool fits = need1 <= o.max_tiles1 && need2 <= o.max_tiles2;
   if (fits && tid < n_experts) {
-    if (!start_in) offsets[tid] = v[0];
+    if (!own_slots) o.offsets[tid] = b0;
     uint32_t at1[kNCls], at2[kNCls], base1 = 0, base2 = 0;
 #pragma unroll
     for (int k = 0; k < kNCls; ++k) {
@@ -179,19 +174,130 @@ __global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
       base1 += tot[1 + k];
       base2 += tot[1 + kNCls + k];
     }
-    put_tiles(tiles1, tid, b0, c, tt1, tpg1, k01, at1);
-    put_tiles(tiles2, tid, b0, c, tt2, tpg2, k02, at2);
+    put_tiles(o.tiles1, tid, b0, c, tt1, tpg1, k01, at1);
+    put_tiles(o.tiles2, tid, b0, c, tt2, tpg2, k02, at2);
   }
   if (tid == 0) {
-    if (!start_in) offsets[n_experts] = tot[0];
-    hdr->n_slots = start_in ? n_slots_in : tot[0];
+    if (!own_slots) o.offsets[n_experts] = tot[0];
+    o.hdr->n_slots = own_slots ? n_slots_in : tot[0];
 #pragma unroll
     for (int k = 0; k < kNCls; ++k) {
-      hdr->n_cls[0][k] = fits ? tot[1 + k] : 0u;
-      hdr->n_cls[1][k] = fits ? tot[1 + kNCls + k] : 0u;
+      o.hdr->n_cls[0][k] = fits ? tot[1 + k] : 0u;
+      o.hdr->n_cls[1][k] = fits ? tot[1 + kNCls + k] : 0u;
     }
-    hdr->tx = tx;
-    hdr->bad = fits ? 0u : 1u;
+    o.hdr->tx = tx;
+    o.hdr->bad = fits ? 0u : 1u;
+  }
+  return b0;
+}
+
+// start_in: a caller's slot list, expert e owning slots [start_in[e], start_in[e+1]) of n_slots_in
+// (each bound clamped to n_slots_in; a range that runs backwards is empty); null: the routes'
+// counts per chunk (grouped_hist_kernel), replaced by each chunk's first slot of each expert.
+__global__ void __launch_bounds__(kPlanThreads) grouped_plan_kernel(
+    uint32_t* __restrict__ hist, uint32_t n_chunks, uint32_t n_experts, uint32_t k01, uint32_t k02, uint32_t tx,
+    const uint32_t* __restrict__ start_in, uint32_t n_slots_in, PlanOut o) {
+  static_assert(AFFX_MAX_EXPERTS <= kPlanThreads, "one thread per expert in the scan");
+  __shared__ uint32_t wsum[kPlanSums];
+  const uint32_t tid = threadIdx.x;
+  const bool own = start_in != nullptr, mine = tid < n_experts;
+  uint32_t c = 0, b0 = 0;
+  // (chunks eight at a time: their loads are in flight together)
+  constexpr uint32_t kB = 8;
+  uint32_t cb[kB];
+  auto chunks = [&](uint32_t b) {
+#pragma unroll
+    for (uint32_t i = 0; i < kB; ++i) cb[i] = mine && b + i < n_chunks ? hist[(uint64_t)(b + i) * n_experts + tid] : 0u;
+  };
+  if (own) {
+    if (mine) {
+      const uint32_t a = min(start_in[tid], n_slots_in), e = min(start_in[tid + 1], n_slots_in);
+      c = e > a ? e - a : 0u;
+      b0 = a;
+    }
+  } else {
+    for (uint32_t b = 0; b < n_chunks; b += kB) {
+      chunks(b);
+#pragma unroll
+      for (uint32_t i = 0; i < kB; ++i) c += cb[i];
+    }
+  }
+  uint32_t at = plan_tiles(c, b0, own, n_slots_in, n_experts, k01, k02, tx, wsum, o);
+  if (own) return;
+  // each chunk's first slot of this expert: its offset plus the counts of the chunks before
+  for (uint32_t b = 0; b < n_chunks; b += kB) {
+    if (n_chunks > kB) chunks(b);  // (else they are still here)
+#pragma unroll
+    for (uint32_t i = 0; i < kB; ++i)
+      if (mine && b + i < n_chunks) {
+        hist[(uint64_t)(b + i) * n_experts + tid] = at;
+        at += cb[i];
+      }
+  }
+}
+
+// The whole plan of a small batch's routes in one workgroup: counts, plan and placement (see
+// grouped_hist_kernel and grouped_place_kernel for what it writes and the slot order). The pairs
+// are taken in groups of 64, a wave each.
+constexpr uint32_t kSmallPairs = 4096;
+__global__ void __launch_bounds__(kPlanThreads) grouped_plan_small_kernel(
+    const uint32_t* __restrict__ sel, const float* __restrict__ w, uint32_t n_pairs, uint32_t n_tok, uint32_t top_k,
+    uint32_t n_experts, uint32_t k01, uint32_t k02, uint32_t tx, const int32_t* __restrict__ tok_sigma,
+    uint32_t* __restrict__ slot_tok, float* __restrict__ slot_w, int32_t* __restrict__ slot_sigma,
+    uint32_t* __restrict__ ord, uint32_t* __restrict__ run, PlanOut o) {
+  static_assert(AFFX_MAX_EXPERTS <= 512, "expert ids ranked by 9 ballots");
+  constexpr uint32_t kW = kPlanThreads / 64, kR = kSmallPairs / kPlanThreads, kG = kSmallPairs / 64;
+  __shared__ uint32_t wsum[kPlanSums];
+  __shared__ uint16_t grp[kG][AFFX_MAX_EXPERTS];  // a group's count of each expert, then its first rank
+  __shared__ uint32_t off[AFFX_MAX_EXPERTS];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const uint32_t ng = (n_pairs + 63u) / 64u;
+  uint32_t ev[kR], rank[kR];
+#pragma unroll
+  for (uint32_t r = 0; r < kR; ++r) {
+    const uint32_t i = r * kPlanThreads + tid;
+    ev[r] = i < n_pairs ? sel[i] : ~0u;
+  }
+  for (uint32_t q = tid; q < ng * (AFFX_MAX_EXPERTS / 2); q += kPlanThreads) reinterpret_cast<uint32_t*>(&grp[0][0])[q] = 0u;
+  for (uint32_t i = tid; i <= n_tok; i += kPlanThreads) run[i] = i * top_k;
+  __syncthreads();
+  const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+  for (uint32_t r = 0; r < kR; ++r) {
+    const uint32_t g = r * kW + wv;
+    rank[r] = 0;
+    if (g >= ng) continue;  // (whole waves)
+    const bool ok = ev[r] < n_experts;
+    const uint64_t m = same_key_lanes<9>(ok ? ev[r] : 0u, ok);
+    rank[r] = (uint32_t)__popcll(m & below);
+    if (ok && (uint32_t)__builtin_ctzll(m) == lane) grp[g][ev[r]] = (uint16_t)__popcll(m);
+  }
+  __syncthreads();
+  uint32_t c = 0;
+  if (tid < n_experts) {
+#pragma unroll 8
+    for (uint32_t g = 0; g < ng; ++g) {
+      const uint32_t x = grp[g][tid];
+      grp[g][tid] = (uint16_t)c;
+      c += x;
+    }
+  }
+  const uint32_t b0 = plan_tiles(c, 0u, false, 0u, n_experts, k01, k02, tx, wsum, o);
+  if (tid < n_experts) off[tid] = b0;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < kR; ++r) {
+    const uint32_t i = r * kPlanThreads + tid;
+    if (i >= n_pairs) continue;
+    if (!(ev[r] < n_experts)) {
+      ord[i] = ~0u;
+      continue;
+    }
+    const uint32_t pos = off[ev[r]] + grp[r * kW + wv][ev[r]] + rank[r], t = i / top_k;
+    slot_tok[pos] = t;
+    slot_w[pos] = w[i];
+    slot_sigma[pos] = tok_sigma[t];
+    ord[i] = pos;
   }
 }
 
@@ -241,8 +347,11 @@ __global__ void __launch_bounds__(256) grouped_place_kernel(const uint32_t* __re
                                                             const float* __restrict__ w, uint32_t n_pairs,
                                                             uint32_t top_k, uint32_t n_experts,
                                                             const uint32_t* __restrict__ first,
+                                                            const int32_t* __restrict__ tok_sigma,
                                                             uint32_t* __restrict__ slot_tok,
-                                                            float* __restrict__ slot_w, uint32_t* __restrict__ ord) {
+                                                            float* __restrict__ slot_w,
+                                                            int32_t* __restrict__ slot_sigma,
+                                                            uint32_t* __restrict__ ord) {
   static_assert(AFFX_MAX_EXPERTS <= 512, "expert ids ranked by 9 ballots");
   constexpr uint32_t NR = kPlaceChunk / 256, NG = NR * 4;  // rounds, (round, wave) groups
   __shared__ uint32_t grp[NG][AFFX_MAX_EXPERTS];
@@ -280,8 +389,10 @@ __global__ void __launch_bounds__(256) grouped_place_kernel(const uint32_t* __re
     if (!(ev[r] < n_experts)) continue;
     const uint32_t i = b * kPlaceChunk + r * 256u + tid;
     const uint32_t pos = fb[ev[r]] + grp[r * 4u + wv][ev[r]] + rank[r];
-    slot_tok[pos] = i / top_k;
+    const uint32_t t = i / top_k;
+    slot_tok[pos] = t;
     slot_w[pos] = w[i];
+    slot_sigma[pos] = tok_sigma[t];
     ord[i] = pos;
   }
 }
@@ -296,6 +407,7 @@ __global__ void __launch_bounds__(256) grouped_prep_x_kernel(const uint16_t* __r
                                                              const uint32_t* __restrict__ run,
                                                              uint32_t n_slots,
                                                              int32_t* __restrict__ slot_sigma,
+                                                             int32_t* __restrict__ tok_sigma,
                                                              uint8_t* __restrict__ xq,
                                                              uint32_t* __restrict__ zeros,
                                                              uint32_t zero_words) {
@@ -305,7 +417,12 @@ __global__ void __launch_bounds__(256) grouped_prep_x_kernel(const uint16_t* __r
   __shared__ float red[4];
   const int sigma = row_terms<true>(x + (uint64_t)t * hidden, xlo ? xlo + (uint64_t)t * hidden : nullptr, hidden,
                                     tx, xq + (uint64_t)t * tx * hidden, red);
-  // the exponent goes to each of the token's slots, for the gate/up epilogue
+  // the exponent, for the gate/up epilogue: of the token (the routes form, whose placement hands it to
+  // the slots), or to each of the token's slots (a caller's slot list)
+  if (!ord) {
+    if (tid == 0) tok_sigma[t] = sigma;
+    return;
+  }
   const uint32_t r1 = min(run[t + 1], n_slots);
   for (uint32_t i = min(run[t], r1) + tid; i < r1; i += 256) {
     const uint32_t sl = ord[i];
@@ -1071,17 +1188,18 @@ namespace {
 
 
 struct GroupedWs {
-  uint64_t hdr, offsets, run, slot_tok, slot_w, ord, hist, tiles1, tiles2, sigma, zeros, xq, aq, z, total;
+  uint64_t hdr, offsets, run, slot_tok, slot_w, ord, hist, tiles1, tiles2, sigma, tok_sigma, zeros, xq, aq, z, total;
   uint32_t max_tiles1, max_tiles2;
 };
 
-// The widest class a batch of T tokens needs (tokens are `terms` columns each): one of whose tiles
-// hold all tokens of an expert that every token names at most once. (An expert named more often, or
-// any slot list, is cut into more tiles of that class.) The wider classes are not launched.
+// The widest class of a batch of T tokens (tokens are `terms` columns each): the narrowest two of whose
+// tiles hold the batch. An expert with more tokens than one tile is cut into more of them, of which
+// a batch this small has few (24 tokens over 256 experts: none at uniform routes), and the wider
+// classes, whose launches would find no tile, are not launched (4-5 us each).
 uint32_t widest_cls(uint32_t T, uint32_t terms) {
   uint32_t k = 0;
   for (int q = 1; q < kNCls; ++q)
-    if (T <= (uint32_t)kClsCT[q] * (16 / terms)) k = (uint32_t)q;
+    if (T <= 2u * (uint32_t)kClsCT[q] * (16 / terms)) k = (uint32_t)q;
   return k;
 }
 uint32_t tile_tokens(uint32_t T, uint32_t terms) { return cls_ct(widest_cls(T, terms)) * (16 / terms); }
@@ -1109,6 +1227,7 @@ GroupedWs grouped_ws(uint32_t T, uint64_t P, uint32_t E, uint32_t hidden, uint32
   w.tiles1 = o; o += a256(sizeof(Tile) * w.max_tiles1);
   w.tiles2 = o; o += a256(sizeof(Tile) * w.max_tiles2);
   w.sigma = o; o += a256(4 * P);  // per slot
+  w.tok_sigma = o; o += a256(4ull * T);
   w.zeros = o; o += a256(hidden > inter ? hidden : inter);
   w.xq = o; o += a256((uint64_t)T * tx * hidden);
   w.aq = o; o += a256(P * 3 * inter);
@@ -1173,30 +1292,41 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
 
   const uint32_t k01 = widest_cls(T, tx), k02 = widest_cls(T, 3);
   const uint32_t Pp = sel ? T * K : 0u;
-  const uint32_t nch = sel ? (uint32_t)place_chunks(T, Pp) : 0u;
-  if (sel) {
-    hipLaunchKernelGGL(grouped_hist_kernel, dim3(nch), dim3(256), 0, s, sel, Pp, T, K, L->n_experts,
-                       (uint32_t*)(b + lay.hist), (uint32_t*)(b + lay.run), (uint32_t*)(b + lay.ord));
-    if (int rc0 = check_launch("grouped_hist_kernel")) return rc0;
-  }
-  hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, (uint32_t*)(b + lay.hist), nch,
-                     L->n_experts, k01, k02, tx, sel ? nullptr : start, sel ? 0u : n_slots, lay.max_tiles1, lay.max_tiles2,
-                     (GroupedHdr*)(b + lay.hdr), (uint32_t*)(b + lay.offsets), (Tile*)(b + lay.tiles1),
-                     (Tile*)(b + lay.tiles2));
-  int rc = check_launch("grouped_plan_kernel");
-  if (rc) return rc;
-  if (sel) {
-    hipLaunchKernelGGL(grouped_place_kernel, dim3(nch), dim3(256), 0, s, sel, w, Pp, K, L->n_experts,
-                       (const uint32_t*)(b + lay.hist), (uint32_t*)(b + lay.slot_tok), (float*)(b + lay.slot_w),
-                       (uint32_t*)(b + lay.ord));
-    if ((rc = check_launch("grouped_place_kernel"))) return rc;
-  }
   const uint32_t n_sl = (uint32_t)P;  // slot indices are below this (the routes form's taken slots too)
   const uint32_t zmax = L->hidden > L->inter ? L->hidden : L->inter;
+  int32_t* tok_sigma = (int32_t*)(b + lay.tok_sigma);
   hipLaunchKernelGGL(grouped_prep_x_kernel, dim3(T), dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)x_lo,
-                     L->hidden, tx, ord_d, run_d, n_sl, (int32_t*)(b + lay.sigma), b + lay.xq,
+                     L->hidden, tx, ord, run, n_sl, (int32_t*)(b + lay.sigma), tok_sigma, b + lay.xq,
                      (uint32_t*)(b + lay.zeros), zmax / 4);
-  if ((rc = check_launch("grouped_prep_x_kernel"))) return rc;
+  int rc = check_launch("grouped_prep_x_kernel");
+  if (rc) return rc;
+  const PlanOut po{(GroupedHdr*)(b + lay.hdr), (uint32_t*)(b + lay.offsets), (Tile*)(b + lay.tiles1),
+                   (Tile*)(b + lay.tiles2), lay.max_tiles1, lay.max_tiles2};
+  uint32_t* hist = (uint32_t*)(b + lay.hist);
+  if (sel && Pp <= kSmallPairs) {
+    // one workgroup instead of three launches: 7.1 us against 5.4 + 8.2 + 5.0 at 144 pairs, 11.6 against
+    // 5.2 + 8.4 + 5.4 at 1998 (kernel trace; the gaps between launches come on top)
+    hipLaunchKernelGGL(grouped_plan_small_kernel, dim3(1), dim3(kPlanThreads), 0, s, sel, w, Pp, T, K, L->n_experts,
+                       k01, k02, tx, tok_sigma, (uint32_t*)(b + lay.slot_tok), (float*)(b + lay.slot_w),
+                       (int32_t*)(b + lay.sigma), (uint32_t*)(b + lay.ord), (uint32_t*)(b + lay.run), po);
+    if ((rc = check_launch("grouped_plan_small_kernel"))) return rc;
+  } else {
+    const uint32_t nch = sel ? (uint32_t)place_chunks(T, Pp) : 0u;
+    if (sel) {
+      hipLaunchKernelGGL(grouped_hist_kernel, dim3(nch), dim3(256), 0, s, sel, Pp, T, K, L->n_experts, hist,
+                         (uint32_t*)(b + lay.run), (uint32_t*)(b + lay.ord));
+      if ((rc = check_launch("grouped_hist_kernel"))) return rc;
+    }
+    hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, hist, nch, L->n_experts, k01, k02, tx,
+                       sel ? nullptr : start, sel ? 0u : n_slots, po);
+    if ((rc = check_launch("grouped_plan_kernel"))) return rc;
+    if (sel) {
+      hipLaunchKernelGGL(grouped_place_kernel, dim3(nch), dim3(256), 0, s, sel, w, Pp, K, L->n_experts,
+                         (const uint32_t*)hist, tok_sigma, (uint32_t*)(b + lay.slot_tok), (float*)(b + lay.slot_w),
+                         (int32_t*)(b + lay.sigma), (uint32_t*)(b + lay.ord));
+      if ((rc = check_launch("grouped_place_kernel"))) return rc;
+    }
+  }
   // gate/up: 128 gate + 128 up rows per item; down: 256 rows. Items (row block, tile), the tile
   // count rounded up to a multiple of the 8 XCDs (see the kernel's order), run by a persistent
   // grid of one workgroup per CU (a multiple of 8), or fewer when there are fewer items
