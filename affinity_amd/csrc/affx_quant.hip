@@ -1,11 +1,17 @@
 // Producer side on the GPU: the synthetic-weight generator and the codebook quantiser.
 //
 // affx_quantize_matrix is the reference's quantize_matrix for the quad format
-// (src/quant/blockquant.cpp:586-791) run per row on the GPU, bit-exact: every float operation
-// is the reference's, in its order, with no contraction into FMAs. The nearest-quad search is exhaustive (each lane scores 16 of the 1024
-// entries, then a wave reduction keeps the minimum, or the lowest index among equal minima),
-// which returns exactly what the reference's scan and its acceleration grid return
-// (src/quant/blockquant.cpp:162-174, 558-578).
+// (src/quant/blockquant.cpp:586-791) on the GPU, bit-exact: every float operation that decides an
+// output is the reference's, in its order, with no contraction into FMAs. A block's setting (variant,
+// scale, sign and rotation: up to 24, each the sum of four nearest-entry distances) is chosen in two
+// stages. First every setting's error is taken from f32 matrix products with a bound on their
+// rounding; where one setting's upper bound lies below all other lower bounds, that setting is the
+// reference's choice, whatever the last bits. The rest (a few percent of the blocks: near ties, and
+// inputs the bound does not cover) are settled by the reference's own search among the settings
+// still open, exhaustively: each lane scores 16 of the 1024 entries, then a wave reduction keeps the
+// minimum, which is exactly what the reference's scan and its acceleration grid return
+// (src/quant/blockquant.cpp:162-174, 558-578). The codes of the chosen setting are the
+// reference's scan, a quad a lane (the lowest index among equal minima).
 //
 // affx_gen_normal is the benchmark's synthetic generator: splitmix64 in counter form plus
 // Box-Muller in double (the generator of src/quant/blockquant.cpp:37-42, 862-869), rounded to
@@ -54,16 +60,6 @@ __device__ __forceinline__ float wave_min(float v) {
   return v;
 }
 
-// (value, index) minimum; equal values keep the lower index.
-__device__ __forceinline__ void wave_argmin(float& v, uint32_t& i) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o);
-    const uint32_t oi = __shfl_xor(i, o);
-    if (ov < v || (ov == v && oi < i)) { v = ov; i = oi; }
-  }
-}
-
 // Squared distance of target t to entry e, dimensions summed in order, no contraction.
 __device__ __forceinline__ float qdist(const float4 e, const float t0, const float t1,
                                        const float t2, const float t3) {
@@ -89,37 +85,94 @@ __device__ __forceinline__ float quad_min(const float4* __restrict__ ent, uint32
   return wave_min(m);
 }
 
-__device__ __forceinline__ uint32_t quad_argmin(const float4* __restrict__ ent, uint32_t lane,
-                                                float t0, float t1, float t2, float t3) {
-  float m = 3.402823466e38f;
-  uint32_t bi = 0xFFFFFFFFu;
-  for (int j = 0; j < 16; ++j) {
-    const uint32_t c = lane + 64 * j;
-    const float s = qdist(ent[c], t0, t1, t2, t3);
-    if (s < m) { m = s; bi = c; }
+// The reference's setting search of one block (blockquant.cpp:706-762) among the settings of `open`
+// (bit 12 v + 4 j + g: variant v, scale mid - 1 + j, g: bit 0 sign, bit 1 rotation), all lanes of
+// the wave on one block: the first strict minimum in the order v, scale, g.
+__device__ uint32_t search_block(const float4* ent, uint32_t lane, const float* __restrict__ blk,
+                                 const float* __restrict__ imp, float rscale, int mid, uint32_t open) {
+  float x[16], wt[4] = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+  for (int i = 0; i < 16; ++i) x[i] = blk[i];
+  if (imp) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float s = 0.f;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) s = s + imp[4 * i + p];
+      wt[i] = s / 4.0f;
+    }
   }
-  wave_argmin(m, bi);
-  return bi == 0xFFFFFFFFu ? 0u : bi;  // nothing below FLT_MAX: the scan's default, code 0
+  uint32_t best = 0;  // field: variant << 5 | g << 3 | scale
+  double best_err = 1.7976931348623157e308;
+  for (uint32_t v = 0; v < 2; ++v)
+    for (int j = 0; j < 3; ++j) {
+      const int s = mid - 1 + j;
+      if (s < 0 || s > 7) continue;
+      const float bs = rscale * (float)(1u << s);
+      if (bs <= 0.f) continue;
+      const float inv = 1.0f / bs;
+      for (uint32_t g = 0; g < 4; ++g) {
+        if (!((open >> (12u * v + 4u * j + g)) & 1u)) continue;
+        const float sg = (g & 1u) ? -inv : inv;
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float t[4];
+#pragma unroll
+          for (int p = 0; p < 4; ++p) t[p] = ((g & 2u) ? x[4 * i + (p + 2) % 4] : x[4 * i + p]) * sg;
+          const float d = quad_min(ent + v * kLut, lane, t[0], t[1], t[2], t[3]);
+          acc = acc + d * wt[i];
+        }
+        const double e = (double)acc * (double)bs * (double)bs;
+        if (e < best_err) { best_err = e; best = (v << 5) | (g << 3) | (uint32_t)s; }
+      }
+    }
+  return best;
 }
 
-// One workgroup per row: 4 waves split the row's 16-blocks; the row's bit streams are built in
-// LDS with atomicOr (disjoint bits) and written out as whole bytes.
+// ---- the search in matrix products -----------------------------------------------------------------
+// Bound by VALU issue: the exhaustive search took 12 operations for every (entry, target) pair, 96
+// targets a block; here a product and 8 minimum operations serve 512 of them, and the codes' scan
+// is the only exhaustive one left. 2048 x 4096: 16.0 -> 3.05 ms (8.4M weights).
+// A workgroup takes 1024 columns of a row, a wave 16 blocks of them. With t a quad's target, the
+// distance to entry e is 2 (|e|^2 / 2 - e.t) + |t|^2: a 16x16x4 f32 product of 16 entries (A, row =
+// entry) with the 16 blocks' targets (B, column = block, K = the quad's four dimensions) on top of
+// C = |e|^2 / 2. The targets of the opposite sign are its negation, |e|^2 / 2 + e.t = |e|^2 - D, so 24
+// products (3 scales x 2 rotations x 4 quads) an entry tile serve 48 of the 96 (setting, quad)
+// pairs of a variant.
+// Bound: u = 2^-24. The reference's float distance is within 6u of the true one; |e|^2 / 2 in f32,
+// four products and four sums, each with one rounding of a value of at most |e|^2 / 2 + |e| |t| <=
+// (E + |t|^2) (E = the largest |e|^2), are within 12u of that, twice it 24u; |t|^2 in f32 within 8u |t|^2;
+// the sums over four quads with their weights (>= 0, else the block is searched in full) within
+// 16u of themselves on either side. The code takes 44u (E + |t|^2) a quad and 64u of the sum.
 constexpr int kQuantMaxCols = 8192;
+constexpr uint32_t kQuantChunk = 1024;
+constexpr float kU = 5.9604645e-8f;
+typedef float qv4f __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(256) quantize_rows_kernel(
-    const float* __restrict__ w, uint32_t rows, uint32_t cols, const float4* __restrict__ cb,
+__device__ __forceinline__ float low_of(float a, float b) { return __builtin_fminf(a, b); }
+
+__global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
+    const float* __restrict__ w, uint32_t cols, uint32_t chunks, const float4* __restrict__ cb,
     const float* __restrict__ imp, uint8_t* __restrict__ codes, uint8_t* __restrict__ fields,
     uint16_t* __restrict__ rscales) {
-  const uint32_t r = blockIdx.x;
+  const uint32_t r = blockIdx.x / chunks, ch = blockIdx.x - r * chunks;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   __shared__ float4 ent[kVariants * kLut];                      // 32 KiB
-  __shared__ uint32_t cbits[kQuantMaxCols * 10 / 128];          // row code stream
-  __shared__ uint32_t fbits[kQuantMaxCols * 6 / 512 + 1];       // row field stream
-  __shared__ float red[4];
-  for (uint32_t i = tid; i < kVariants * kLut; i += 256) ent[i] = cb[i];
-  const uint32_t ncw = cols * 10 / 128, nfw = (cols * 6 / 16 + 31) / 32;
-  for (uint32_t i = tid; i < ncw; i += 256) cbits[i] = 0;
-  for (uint32_t i = tid; i < nfw; i += 256) fbits[i] = 0;
+  __shared__ __align__(16) float half[kVariants * kLut];        // |e|^2 / 2
+  __shared__ uint32_t cbits[kQuantChunk * 10 / 128];            // the chunk's code stream
+  __shared__ uint32_t fbits[kQuantChunk * 6 / 512 + 1];         // the chunk's field stream
+  __shared__ float red[8];
+  float e2max = 0.f;
+  for (uint32_t i = tid; i < kVariants * kLut; i += 256) {
+    const float4 e = cb[i];
+    ent[i] = e;
+    const float n = ((e.x * e.x + e.y * e.y) + e.z * e.z) + e.w * e.w;
+    half[i] = 0.5f * n;
+    e2max = e2max >= n ? e2max : n;  // (a NaN is kept)
+  }
+  for (uint32_t i = tid; i < kQuantChunk * 10 / 128; i += 256) cbits[i] = 0;
+  if (tid < kQuantChunk * 6 / 512 + 1) fbits[tid] = 0;
 
   const float* row = w + (uint64_t)r * cols;
   float rmax = 0.f;
@@ -128,101 +181,190 @@ __global__ void __launch_bounds__(256) quantize_rows_kernel(
     rmax = rmax < a ? a : rmax;
   }
   rmax = -wave_min(-rmax);
-  if (lane == 0) red[wv] = rmax;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float x = __shfl_xor(e2max, o);
+    e2max = e2max >= x ? e2max : x;
+  }
+  if (lane == 0) { red[wv] = rmax; red[4 + wv] = e2max; }
   __syncthreads();
   rmax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+  for (int q = 0; q < 4; ++q) e2max = e2max >= red[4 + q] ? e2max : red[4 + q];
   float rscale = rmax > 0.f ? ldexpf(rmax, -7) : 0.f;
   const uint16_t h = f32_to_bf16_rne(rscale);
   rscale = __uint_as_float((uint32_t)h << 16);
-  if (tid == 0) rscales[r] = h;
+  if (ch == 0 && tid == 0) rscales[r] = h;
 
-  const uint32_t nblk = cols / kBlock;
-  for (uint32_t b = wv; b < nblk; b += 4) {
-    float blk[16];
+  // ---- this wave's 16 blocks: lane (c, kg) holds dimension kg of block c's quads ---------------------
+  const uint32_t c0 = ch * kQuantChunk, nblk = min(cols - c0, kQuantChunk) / kBlock;
+  const uint32_t c = lane & 15, kg = lane >> 4, b = 16u * wv + c;
+  const bool live = b < nblk;
+  const float* blk = row + c0 + (uint64_t)(live ? b : 0u) * kBlock;
+  const float* bimp = imp ? imp + c0 + (live ? b : 0u) * kBlock : nullptr;
+  float wq[4], wr[4], S[4], wt[4] = {1.f, 1.f, 1.f, 1.f}, bmax = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) blk[i] = row[b * 16 + i];
-    float bmax = 0.f;
+  for (int q = 0; q < 4; ++q) {
+    wq[q] = live ? blk[4 * q + kg] : 0.f;
+    wr[q] = __shfl_xor(wq[q], 32);  // dimension (kg + 2) % 4
+    const float a = fabsf(wq[q]);
+    bmax = bmax < a ? a : bmax;
+    S[q] = wq[q] * wq[q];
+    if (bimp) wt[q] = (((bimp[4 * q] + bimp[4 * q + 1]) + bimp[4 * q + 2]) + bimp[4 * q + 3]) * 0.25f;
+  }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) { const float a = fabsf(blk[i]); bmax = bmax < a ? a : bmax; }
-    float wt[4] = {1.f, 1.f, 1.f, 1.f};
-    if (imp) {
+  for (int o = 16; o <= 32; o <<= 1) {
+    const float a = __shfl_xor(bmax, o);
+    bmax = bmax < a ? a : bmax;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float s = 0.f;
-#pragma unroll
-        for (int p = 0; p < 4; ++p) s = s + imp[b * 16 + 4 * i + p];
-        wt[i] = s / 4.0f;
-      }
+    for (int q = 0; q < 4; ++q) S[q] = S[q] + __shfl_xor(S[q], o);
+  }
+  const bool need = live && bmax > 0.f && rscale > 0.f;
+  int mid = 0;
+  if (need) {
+    const double ideal = (double)bmax / (double)rscale;
+    double bd = 1.7976931348623157e308;
+    for (int s = 0; s <= 7; ++s) {
+      const double d = fabs((double)(float)(1u << s) - ideal);
+      if (d < bd) { bd = d; mid = s; }
     }
-    uint32_t best_s = 0, best_v = 0, best_g = 0;
-    double best_err = 1.7976931348623157e308;
-    if (bmax > 0.f && rscale > 0.f) {
-      const double ideal = (double)bmax / (double)rscale;
-      uint32_t mid = 0;
-      double bd = 1.7976931348623157e308;
-      for (uint32_t s = 0; s <= 7; ++s) {
-        const double d = fabs((double)(float)(1u << s) - ideal);
-        if (d < bd) { bd = d; mid = s; }
-      }
-      const int lo = (int)mid - 1 > 0 ? (int)mid - 1 : 0;
-      const int hi = (int)mid + 1 < 7 ? (int)mid + 1 : 7;
-      for (uint32_t v = 0; v < 2; ++v) {
-        const float4* ev = ent + v * kLut;
-        for (int s = lo; s <= hi; ++s) {
-          const float bs = rscale * (float)(1u << s);
-          if (bs <= 0.f) continue;
-          const float inv = 1.0f / bs;
-          for (uint32_t g = 0; g < 4; ++g) {
-            const float sg = (g & 1u) ? -inv : inv;
-            const uint32_t rh = (g & 2u) ? 2u : 0u;
-            float acc = 0.f;
-            for (int i = 0; i < 4; ++i) {
-              const float t0 = blk[4 * i + (0 + rh) % 4] * sg;
-              const float t1 = blk[4 * i + (1 + rh) % 4] * sg;
-              const float t2 = blk[4 * i + (2 + rh) % 4] * sg;
-              const float t3 = blk[4 * i + (3 + rh) % 4] * sg;
-              const float d = quad_min(ev, lane, t0, t1, t2, t3);
-              acc = acc + d * wt[i];
-            }
-            const double e = (double)acc * (double)bs * (double)bs;
-            if (e < best_err) { best_err = e; best_s = (uint32_t)s; best_v = v; best_g = g; }
-          }
+  }
+  float inv[3], er[3];
+  uint32_t valid = 0;  // settings there are (scale 0..7), as in search_block
+  bool sane = e2max < 1e30f;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int s = mid - 1 + j;
+    const bool in = s >= 0 && s <= 7;
+    const float bs = rscale * (float)(1u << (in ? s : 0));
+    inv[j] = in && need ? 1.0f / bs : 0.f;
+    if (in) valid |= 0xF00Fu << (4 * j);
+    er[j] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) er[j] = er[j] + wt[q] * (44.f * kU * (e2max + S[q] * inv[j] * inv[j]));
+    er[j] = er[j] * (float)(1u << (2 * j));
+    sane = sane && (!in || (bs > 1e-30f && bs < 1e30f)) && er[j] < 1e30f;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) sane = sane && wt[q] >= 0.f;
+
+  uint32_t open = 0;
+  if (__ballot(need && sane)) {  // (the whole wave)
+    float ea[24];  // errors of the settings over bs(j = 0)^2
+    for (uint32_t v = 0; v < 2; ++v) {
+      float m[24][2];
+#pragma unroll
+      for (int k = 0; k < 24; ++k) m[k][0] = m[k][1] = 3.402823466e38f;
+      const float* A = reinterpret_cast<const float*>(ent + v * kLut) + 4u * c + kg;
+      const float* Hf = half + v * kLut + 4u * kg;
+#pragma unroll 1
+      for (int i = 0; i < kLut / 16; ++i) {
+        const float a = A[64 * i];
+        const qv4f C = *reinterpret_cast<const qv4f*>(Hf + 16 * i);
+        const qv4f n = C + C;
+        auto product = [&](int k) -> qv4f {
+          const float t = ((k / 4) % 2 ? wr[k % 4] : wq[k % 4]) * inv[k / 8];
+          return __builtin_amdgcn_mfma_f32_16x16x4f32(a, -t, C, 0, 0, 0);
+        };
+        // (two products in flight: the minima of one run behind the next two)
+        qv4f D0 = product(0), D1 = product(1);
+#pragma unroll
+        for (int k = 0; k < 24; ++k) {
+          const qv4f D = D0;
+          D0 = D1;
+          if (k + 2 < 24) D1 = product(k + 2);
+          __builtin_amdgcn_sched_barrier(0);
+          m[k][0] = low_of(low_of(m[k][0], D[0]), D[1]);
+          m[k][0] = low_of(low_of(m[k][0], D[2]), D[3]);
+          m[k][1] = low_of(low_of(m[k][1], n[0] - D[0]), n[1] - D[1]);
+          m[k][1] = low_of(low_of(m[k][1], n[2] - D[2]), n[3] - D[3]);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
+#pragma unroll
+      for (int k = 0; k < 24; ++k)
+#pragma unroll
+        for (int sg = 0; sg < 2; ++sg) {
+          float x = m[k][sg];
+          x = low_of(x, __shfl_xor(x, 16));
+          m[k][sg] = low_of(x, __shfl_xor(x, 32));
+        }
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          float e = 0.f;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            e = e + wt[q] * (2.f * m[8 * j + 4 * (g >> 1) + q][g & 1] + S[q] * inv[j] * inv[j]);
+          e = e * (float)(1u << (2 * j));
+          if (v == 0) ea[4 * j + g] = e;
+          else ea[12 + 4 * j + g] = e;
+        }
     }
-    const uint32_t field = (best_v << 5) | (best_g << 3) | best_s;
-    const float mag = rscale * (float)(1u << best_s);
-    const float bs = (best_g & 1u) ? -mag : mag;
-    const uint32_t rh = (best_g & 2u) ? 2u : 0u;
-    uint32_t code[4] = {0, 0, 0, 0};
+    float hi = 3.402823466e38f;
+#pragma unroll
+    for (int k = 0; k < 24; ++k)
+      if ((valid >> k) & 1u) hi = low_of(hi, ea[k] + er[(k / 4) % 3] + 64.f * kU * fabsf(ea[k]));
+#pragma unroll
+    for (int k = 0; k < 24; ++k)
+      if (((valid >> k) & 1u) && !(ea[k] - er[(k / 4) % 3] - 64.f * kU * fabsf(ea[k]) > hi)) open |= 1u << k;
+  }
+  if (!sane) open = valid;
+  uint32_t field = 0;
+  if (need && (open & (open - 1u)) == 0u && open != 0u) {
+    const uint32_t k = (uint32_t)__builtin_ctz(open), j = (k % 12u) / 4u;
+    field = ((k / 12u) << 5) | ((k & 3u) << 3) | (uint32_t)(mid - 1 + (int)j);
+  }
+  // the blocks left open, one at a time
+  uint64_t todo = __ballot(need && kg == 0u && (open & (open - 1u)) != 0u);
+  while (todo) {
+    const uint32_t src = (uint32_t)__builtin_ctzll(todo);
+    todo &= todo - 1;
+    const uint32_t bb = (16u * wv + src) * kBlock;
+    const uint32_t f = search_block(ent, lane, row + c0 + bb, imp ? imp + c0 + bb : nullptr, rscale,
+                                    __shfl(mid, (int)src), __shfl(open, (int)src));
+    if (c == src) field = f;
+  }
+
+  // ---- the codes: lane (c, kg) takes quad kg of block c --------------------------------------------
+  if (live) {
+    const float mag = rscale * (float)(1u << (field & 7u));
+    const float bs = (field & 8u) ? -mag : mag;
+    const bool rot = (field & 16u) != 0u;
+    uint32_t code = 0;
     if (mag > 0.f) {
-      for (int i = 0; i < 4; ++i) {
-        const float t0 = blk[4 * i + (0 + rh) % 4] / bs;
-        const float t1 = blk[4 * i + (1 + rh) % 4] / bs;
-        const float t2 = blk[4 * i + (2 + rh) % 4] / bs;
-        const float t3 = blk[4 * i + (3 + rh) % 4] / bs;
-        code[i] = quad_argmin(ent + best_v * kLut, lane, t0, t1, t2, t3);
+      float x[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) x[p] = blk[4 * kg + p];
+      const float t0 = (rot ? x[2] : x[0]) / bs, t1 = (rot ? x[3] : x[1]) / bs;
+      const float t2 = (rot ? x[0] : x[2]) / bs, t3 = (rot ? x[1] : x[3]) / bs;
+      const float4* ev = ent + (field >> 5) * kLut;
+      float m = 3.402823466e38f;
+#pragma unroll 8
+      for (uint32_t e = 0; e < (uint32_t)kLut; ++e) {
+        const float d = qdist(ev[e], t0, t1, t2, t3);
+        if (d < m) { m = d; code = e; }
       }
     }
-    if (lane == 0) {
+    if (kg == 0u) {
       const uint32_t fpos = b * 6;
       atomicOr(&fbits[fpos >> 5], field << (fpos & 31));
       if ((fpos & 31) > 26) atomicOr(&fbits[(fpos >> 5) + 1], field >> (32 - (fpos & 31)));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t cpos = (b * 4 + i) * 10;
-        atomicOr(&cbits[cpos >> 5], code[i] << (cpos & 31));
-        if ((cpos & 31) > 22) atomicOr(&cbits[(cpos >> 5) + 1], code[i] >> (32 - (cpos & 31)));
-      }
     }
+    const uint32_t cpos = (b * 4 + kg) * 10;
+    atomicOr(&cbits[cpos >> 5], code << (cpos & 31));
+    if ((cpos & 31) > 22) atomicOr(&cbits[(cpos >> 5) + 1], code >> (32 - (cpos & 31)));
   }
   __syncthreads();
-  // a row's streams are whole bytes (cols % 64 == 0): 5*cols/16 code bytes, 3*cols/64 field bytes
-  const uint32_t ncb = cols * 10 / 32, nfb = cols * 6 / 128;
+  // 64 columns are whole bytes of both streams (20 and 3), and cols % 64 == 0
+  const uint32_t ncb = nblk * 5, nfb = nblk * 3 / 4;
   const uint8_t* cs = reinterpret_cast<const uint8_t*>(cbits);
   const uint8_t* fs = reinterpret_cast<const uint8_t*>(fbits);
-  for (uint32_t i = tid; i < ncb; i += 256) codes[(uint64_t)r * ncb + i] = cs[i];
-  for (uint32_t i = tid; i < nfb; i += 256) fields[(uint64_t)r * nfb + i] = fs[i];
+  uint8_t* co = codes + (uint64_t)r * (cols * 10 / 32) + ch * (kQuantChunk * 10 / 32);
+  uint8_t* fo = fields + (uint64_t)r * (cols * 6 / 128) + ch * (kQuantChunk * 6 / 128);
+  for (uint32_t i = tid; i < ncb; i += 256) co[i] = cs[i];
+  for (uint32_t i = tid; i < nfb; i += 256) fo[i] = fs[i];
 }
 
 }  // namespace affx
@@ -250,8 +392,10 @@ int affx_quantize_matrix(const void* w, uint32_t rows, uint32_t cols, const void
   if (rows == 0 || cols == 0 || cols % 64 || cols > kQuantMaxCols)
     return set_error(AFFX_ERR_ARG, "quantize_matrix: cols must be a multiple of 64 and <= %d",
                      kQuantMaxCols);
-  hipLaunchKernelGGL(quantize_rows_kernel, dim3(rows), dim3(256), 0, (hipStream_t)stream,
-                     (const float*)w, rows, cols, (const float4*)codebook_f32,
+  const uint32_t chunks = (cols + kQuantChunk - 1) / kQuantChunk;
+  if (rows > 0x7FFFFFFFu / chunks) return set_error(AFFX_ERR_ARG, "quantize_matrix: too many rows");
+  hipLaunchKernelGGL(quantize_rows_kernel, dim3(rows * chunks), dim3(256), 0, (hipStream_t)stream,
+                     (const float*)w, cols, chunks, (const float4*)codebook_f32,
                      (const float*)importance, (uint8_t*)codes, (uint8_t*)fields,
                      (uint16_t*)rscales);
   return check_launch("quantize_rows_kernel");

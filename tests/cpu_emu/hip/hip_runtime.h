@@ -283,6 +283,20 @@ inline emu_v4f __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(emu_v8i a, emu_v
   return d;
 }
 
+// ---- MFMA 16x16x4 f32: A row l % 16 and B column l % 16 of K = l / 16; D row 4 (l / 16) + v ----
+inline emu_v4f __builtin_amdgcn_mfma_f32_16x16x4f32(float a, float b, emu_v4f c, int, int, int) {
+  uint32_t w = emu_wave(), l = emu_lane();
+  emu_blk->xfer[w][l][0] = __float_as_uint(a) | ((uint64_t)__float_as_uint(b) << 32);
+  emu_wave_sync();
+  emu_v4f d = c;
+  for (int v = 0; v < 4; ++v)
+    for (int k = 0; k < 4; ++k)
+      d[v] = fmaf(__uint_as_float((uint32_t)emu_blk->xfer[w][4 * (l / 16) + v + 16 * k][0]),
+                  __uint_as_float((uint32_t)(emu_blk->xfer[w][l % 16 + 16 * k][0] >> 32)), d[v]);
+  emu_wave_sync();
+  return d;
+}
+
 // ---- launch ----
 // Sequential: one block at a time, blockDim.x threads created once per launch.
 template <typename F, typename... Args>

@@ -62,3 +62,40 @@ def test_quantizer_matches_reference_config1(ax, c1_codebook):
         assert sha(codes.cpu().numpy()) == man["planes"][name]["codes"], name
         assert sha(fields.cpu().numpy()) == man["planes"][name]["fields"], name
         assert sha(rs.cpu().numpy().view(np.uint16)) == man["planes"][name]["rscales"], name
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 64), (2, 448), (5, 1088), (2, 8192)])
+@pytest.mark.parametrize("kind", ["normal", "ties", "scales", "importance", "nonfinite"])
+def test_quantizer_edges_match_oracle(ax, orc, c1_codebook, rows, cols, kind):
+    """Bit for bit against the oracle where the setting's choice is hard: a codebook whose settings tie
+    (its second variant the first one negated, entries repeated), rows from 1e-42 to 1e38 with zero
+    blocks, importances that are zero or negative, infinities and NaN; partial chunks and a whole row of
+    8192."""
+    rng = np.random.default_rng(rows * cols + len(kind))
+    w = (0.02 * rng.standard_normal((rows, cols))).astype(np.float32)
+    cb = ax.codebook_floats(c1_codebook).copy()
+    imp = None
+    if kind == "ties":
+        cb[1] = -cb[0]
+        cb[:, 512:] = cb[:, :512]
+        w[:, ::2] = np.sign(w[:, ::2]) * np.float32(0.0078125)
+    elif kind == "scales":
+        w[0] *= np.float32(1e-40)
+        w[-1] *= np.float32(4e38 / 100)
+        w[0, 16:32] = 0
+        w[rows // 2, :64] = 0
+        w[rows // 2, 5] = np.float32(3e3)
+    elif kind == "importance":
+        imp = rng.uniform(-0.2, 1.0, cols).astype(np.float32)
+        imp[:32] = 0
+        imp[32:64] = np.abs(imp[32:64])
+    elif kind == "nonfinite":
+        w[0, 7] = np.inf
+        w[1, 20] = np.nan
+        w[-1, 33] = -np.inf
+    want = orc.quantize(w, cb.reshape(-1), imp)
+    codes, fields, rs = ax.quantize_matrix(torch.from_numpy(w).cuda(), torch.from_numpy(cb).cuda(),
+                                           None if imp is None else torch.from_numpy(imp).cuda())
+    np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
+    np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
+    np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
