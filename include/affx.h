@@ -457,7 +457,7 @@ int affx_expert_gemm_w8a8(const affx_expert_tile* tiles, uint32_t n_tiles, uint3
  * else 1. The scores are within an ulp of the host's float libm (so the weights within a few).
  * AFFX_ROUTE_SOFTMAX: the top_k largest logits (ties to the lower id), weights the softmax over
  * those k in double (bias, norm_topk_prob and routed_scaling unused).
- * top_k <= min(16, n_expert), n_expert <= 512. One wave per token; no synchronisation. */
+ * top_k <= min(16, n_expert), n_expert <= 512. No synchronisation. */
 int affx_route_topk(const float* logits, uint64_t tok_stride, uint64_t expert_stride,
                     const float* bias, uint32_t n_tok, uint32_t n_expert, uint32_t top_k, int rule,
                     int norm_topk_prob, float routed_scaling, uint32_t* sel, float* w, void* stream);

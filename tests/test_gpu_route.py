@@ -177,3 +177,24 @@ def test_router_feeds_decode_and_grouped_without_host(ax, orc, c1_codebook):
     err = rel_l2(yg, ref)
     print(f"router -> grouped rel_l2={err:.3e}")
     assert err <= 1e-3
+
+
+@pytest.mark.parametrize("T", [1, 5, 2047, 2048, 2051])
+@pytest.mark.parametrize("E,k", [(1, 1), (63, 6), (64, 16), (257, 8), (512, 16)])
+def test_route_forms_and_edges(ax, orc, T, E, k):
+    """Both forms (a workgroup a token below 2048 tokens, a wave a token from there on) at expert counts
+    around the wave's and the largest, with ties, zeros of both signs and infinities among the logits: ids
+    as the oracle's, softmax weights within an ulp (a sample of the tokens)."""
+    from affinity_amd._lib import AFFX_ROUTE_ENGINE, AFFX_ROUTE_SOFTMAX
+    rng = np.random.default_rng(T + E)
+    lg = np.round(rng.standard_normal((T, E)) * 2).astype(np.float32)   # ties, and -0.0 beside 0.0
+    lg[0] = np.where(rng.random(E) < 0.5, np.float32(0.0), np.float32(-0.0))
+    lg[T // 2, 0] = np.float32(25.0)
+    lg[T - 1, E - 1] = -np.inf
+    for rule in (AFFX_ROUTE_ENGINE, AFFX_ROUTE_SOFTMAX):
+        sel, w = _route(torch.from_numpy(lg).cuda(), k, rule, None, True, 1.5)
+        sel, w = sel.cpu().numpy(), w.cpu().numpy()
+        for t in np.unique(np.concatenate([[0, T // 2, T - 1], rng.integers(0, T, 40)])):
+            rs, rw = orc.route_topk(lg[t], None, k, True, 1.5) if rule == AFFX_ROUTE_ENGINE else orc.route(lg[t], k)
+            np.testing.assert_array_equal(sel[t], rs, err_msg=f"token {t} rule {rule}")
+            assert ulps(w[t], rw) <= (2 if rule == AFFX_ROUTE_ENGINE else 1)
