@@ -9,25 +9,28 @@
 // (token, 128-column block).
 //
 // A wave decodes the column tiles of a 16-row wave tile into MFMA A fragments (the decode's LDS
-// codebook and step order). One MFMA step's 128 K values span four 128-column blocks (lane group g
-// holds 32 columns of the tile's segment g), so to keep the blocks' sums apart the B operand places
-// the columns of group g of a token in B column 4 (token of the quad) + g and zeros elsewhere: one
-// MFMA gives, for four tokens, each group's partial, steps 0-3 completing block 2g of the tile and
-// steps 4-7 block 2g + 1. A (row, token)'s eight partials then sit in one lane quad, and every lane
-// of the quad folds them in block order (DPP quad broadcasts).
+// codebook and step order). In a fragment of the wave tile lane group g holds 32 columns of segment g,
+// so one MFMA's 128 values of K would span four 128-column blocks, whose sums must stay apart. Four
+// steps' fragments are a 4 x 4 matrix of (segment, 32 columns) over (lane group, fragment): transposed
+// by lane-row swaps (32 VALU operations for 4 fragments), lane group j of fragment g holds
+// columns 32 j .. of segment g's block, and an MFMA is one block of 16 tokens. Its sums are
+// folded into the outputs in block order, one fma each. (Without the transposition each MFMA took a
+// quad of tokens, its B zero outside the group: four times the MFMAs, and a fold through DPP quad
+// broadcasts: 256 tokens' steps over 256 experts 1092 us, now 672.)
 //
-// Tiles run in two persistent kernels by their token count, which only the device knows: each
-// kernel's workgroups walk the whole list and pass over the other's tiles (a scalar load each).
-//  * light tiles (at most 8 tokens; most tiles of a batch of a few hundred tokens over 256
-//    experts): bound by the weights' stream, so 16 waves a CU keep two units a wave in flight, and
-//    a workgroup's next column tile or next item is requested before the current one is decoded;
-//  * heavy tiles: bound by the MFMAs (each issued for one column group of a token quad), so a
-//    tile's decode is kept for all its quads, as many as its tokens fill.
+// An item is 128 rows by at most 16 tokens (one MFMA column tile) of a tile, eight waves: most tiles of
+// a batch of a few hundred tokens over 256 experts have no more, and the weights' stream and the
+// decode are the bound, so a persistent workgroup requests its next column tile's or next item's
+// weights and token rows before it decodes the current ones, two workgroups (16 waves) a CU. A tile
+// of more tokens is several items, which decode the same weights again. (A second kernel for the tiles
+// of more than 16 tokens, one decode held for all their products at half the waves a CU, made the
+// 256-token steps 755 us against 672: a handful of such tiles fills a launch of its own badly.)
+// Full tiles: 384 of 64 tokens, 2048 x 4096, 1.69 -> 1.23 ms (334 TFLOP/s); 256 of one token 987 -> 191 us.
 #include "affx_lut.h"
 
 namespace affx {
 
-constexpr int kW8Waves = 4;
+constexpr int kW8Waves = 8;
 constexpr int kW8T = kW8Waves * 64;
 constexpr int kW8KC = 2;              // codebook copies
 constexpr uint32_t kW8MaxTok = 64;    // the reference's kExpertWmmaTok (expert_kernel_hip.h:195)
@@ -38,7 +41,7 @@ struct W8a8Args {
   const uint8_t* x8;
   const float* xs;
   const uint32_t* codebook;
-  uint32_t rows, cols, n_tiles, cap;
+  uint32_t rows, cols, cap, items;  // (items: tiles x row blocks x token groups of the cap)
   float wscale;
   int y_bf16;
 };
@@ -47,12 +50,6 @@ __device__ __forceinline__ uint16_t w8_bf16(float f) {
   const uint32_t u = __float_as_uint(f);
   if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x007FFFFFu)) return (uint16_t)((u >> 16) | 0x40u);  // quiet NaN
   return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
-
-// value of lane G of this lane's quad (DPP quad_perm [G, G, G, G])
-template <int G>
-__device__ __forceinline__ float quad_lane(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), G * 0x55, 0xF, 0xF, false));
 }
 
 // A tile's tokens: at most `cap` (the launch's max_nt rounded up to a power of two of quads; a tile
@@ -66,27 +63,50 @@ __device__ __forceinline__ uint32_t w8_row(const uint32_t* tok, uint32_t j) {
   return tok ? *AFFX_CONST_PTR(uint32_t, tok + j) : j;
 }
 
-// Folds one quad's partials of a column tile into out, block 2g + h of the tile: group g's partial
-// (lane g of the quad, a DPP quad broadcast), half h; sc: the token's scales of the eight blocks.
-__device__ __forceinline__ void w8_fold(const v4f& acc0, const v4f& acc1, const float* sc, float (&out)[4]) {
-  const float4 s0 = *reinterpret_cast<const float4*>(sc);
-  const float4 s1 = *reinterpret_cast<const float4*>(sc + 4);
+// Transposes four steps' fragments of a half (steps 4h .. 4h + 3): f[j] of lane group g, the half's
+// columns 32 j .. of segment g, becomes f[g] of lane group j.
+__device__ __forceinline__ void w8_transpose(v8i (&f)[4]) {
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    float o = out[v];
-    o = __builtin_fmaf(quad_lane<0>(acc0[v]), s0.x, o);
-    o = __builtin_fmaf(quad_lane<0>(acc1[v]), s0.y, o);
-    o = __builtin_fmaf(quad_lane<1>(acc0[v]), s0.z, o);
-    o = __builtin_fmaf(quad_lane<1>(acc1[v]), s0.w, o);
-    o = __builtin_fmaf(quad_lane<2>(acc0[v]), s1.x, o);
-    o = __builtin_fmaf(quad_lane<2>(acc1[v]), s1.y, o);
-    o = __builtin_fmaf(quad_lane<3>(acc0[v]), s1.z, o);
-    o = __builtin_fmaf(quad_lane<3>(acc1[v]), s1.w, o);
-    out[v] = o;
+  for (int d = 0; d < 8; ++d) {
+    const auto p = __builtin_amdgcn_permlane32_swap((uint32_t)f[0][d], (uint32_t)f[2][d], false, false);
+    const auto q = __builtin_amdgcn_permlane32_swap((uint32_t)f[1][d], (uint32_t)f[3][d], false, false);
+    const auto r = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    const auto t = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    f[0][d] = (int)r[0];
+    f[1][d] = (int)r[1];
+    f[2][d] = (int)t[0];
+    f[3][d] = (int)t[1];
   }
 }
+// The four fragments of half h of the unit, one block of 128 columns each.
+__device__ __forceinline__ void w8_half(Unit& u, const uint8_t* lut, uint32_t copy4, int h, v8i (&f)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    uint32_t raw[8], bv[2];
+    pin_step(u, 4 * h + j);
+    lut_lookup_step<kW8KC, true>(u, lut, nullptr, copy4, 4 * h + j, raw, bv);
+    f[j] = lut_finish(raw, bv);
+    asm volatile("" ::: "memory");  // (one step's table reads in flight at a time: registers)
+  }
+  w8_transpose(f);
+}
+// B of block kb (of the column tile's eight) for the lane's token, whose staged row this is.
+__device__ __forceinline__ v8i w8_b(const uint8_t* row, uint32_t kg, int kb) {
+  return b_step(reinterpret_cast<const u32x4*>(row + kg * 32u + 128u * kb), 0);
+}
+// Folds the eight blocks' sums of a column tile, res[h][g] of block 2 g + h, in block order; sc: the
+// lane's token's scales of the eight blocks.
+__device__ __forceinline__ void w8_fold(const v4f (&res)[2][4], const float* sc, float (&out)[4]) {
+  const float4 s0 = *reinterpret_cast<const float4*>(sc);
+  const float4 s1 = *reinterpret_cast<const float4*>(sc + 4);
+  const float s[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+  for (int kb = 0; kb < 8; ++kb)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) out[v] = __builtin_fmaf(res[kb & 1][kb >> 1][v], s[kb], out[v]);
+}
 
-// Writes one quad's results (the lanes of c % 4 == 0): y[row][j] for the lane's four rows.
+// Writes the lane's results of token column j: y[row][j] for its four rows.
 __device__ __forceinline__ void w8_store(const W8a8Args& A, void* y, uint32_t ld, uint32_t row0, uint32_t j,
                                          const float (&out)[4], uint2 rsv) {
   const float rs[4] = {__uint_as_float(rsv.x << 16) * A.wscale, __uint_as_float(rsv.x & 0xFFFF0000u) * A.wscale,
@@ -102,73 +122,95 @@ __device__ __forceinline__ void w8_store(const W8a8Args& A, void* y, uint32_t ld
   }
 }
 
-// ---- light tiles: at most kW8Light tokens -------------------------------------------------------
-// Eight waves, 128 rows of a tile an item; LDS: the codebook and two buffers of a column tile's
-// token rows and scales, so two workgroups a CU (at most 128 registers a wave). The steps of a
-// workgroup are (item, column tile) pairs in order; each step first requests the next step's unit
-// and token rows, then decodes and multiplies its own, and ends in one barrier.
-constexpr uint32_t kW8Light = 8;
-constexpr int kW8LWaves = 8;
-constexpr int kW8LT = kW8LWaves * 64;
-static_assert(kW8Light == (uint32_t)kW8LWaves, "wave w stages token row w");
-
-__global__ void __launch_bounds__(kW8LT, 4) w8a8_light_kernel(W8a8Args A) {
-  __shared__ __align__(16) uint32_t lut_s[Lut<kW8KC, true>::kDwords];
-  // (two arrays a kind: the compiler can tell the buffer being read from the one being written)
-  __shared__ __align__(16) uint8_t xb0[kW8Light * kW8Row], xb1[kW8Light * kW8Row];
-  __shared__ __align__(16) float xs0[kW8Light * 8], xs1[kW8Light * 8];
-  __shared__ __align__(16) uint8_t zero_s[kSegCols];  // B of the lanes outside a token's column group
-  const uint8_t* lut = reinterpret_cast<const uint8_t*>(lut_s);
-  const uint32_t tid = threadIdx.x;
-  const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // (the lane is counted where it is used: lane values held across the steps were spilled, and a
-  // reload, a vector memory load, waits for every load in flight)
-  auto lane_now = [&]() -> uint32_t {
-    uint32_t z = 0u;
-    AFFX_PIN(z);
-    return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
-  };
-  const uint32_t nct = A.cols / kTileCols, nkb = A.cols / 128u, nrt = A.rows / kTileRows;
-  const uint32_t nrb = (nrt + kW8LWaves - 1) / kW8LWaves, items = A.n_tiles * nrb;
-  auto seek = [&](uint32_t it) -> uint32_t {
-    for (; it < items; it += gridDim.x) {
-      const uint32_t nt = w8_tokens(A.tiles, it / nrb, A.cap);
-      if (nt != 0 && nt <= kW8Light) break;
-    }
-    return __builtin_amdgcn_readfirstlane(it);
-  };
-  struct Item {
-    const uint8_t* codes;
-    const uint8_t* fields;
-    const uint32_t* tok;
-    uint32_t tile, n, rt;
-  };
-  auto open = [&](uint32_t it) -> Item {
-    Item I;
-    I.tile = __builtin_amdgcn_readfirstlane(it / nrb);
+// An item: eight row tiles (one a wave) of a tile's tokens j0 .. j0 + n - 1.
+struct W8Item {
+  const uint8_t* codes;
+  const uint8_t* fields;
+  const uint32_t* tok;
+  uint32_t tile, j0, n, rt;
+};
+// Item order: tile, row block, token group (nch groups of kW8Cols tokens; adjacent items, which run at
+// the same time, read the same weights). Most tiles fill the first group only, so workgroup b takes
+// item r G + (b + r) % G in round r (G the grid): its items go through the groups in turn, not
+// through one (G is a multiple of nch).
+constexpr uint32_t kW8Cols = 16;
+struct W8Order {
+  uint32_t nrb, nch, items;
+};
+// The first item in use from round r on (advanced); false past the last.
+__device__ __forceinline__ bool w8_seek(const W8a8Args& A, const W8Order& o, uint32_t& r, uint32_t wv, W8Item& I) {
+  for (; (uint64_t)r * gridDim.x < o.items; ++r) {
+    const uint32_t it = r * gridDim.x + (blockIdx.x + r) % gridDim.x;
+    if (it >= o.items) continue;
+    const uint32_t q = it / o.nch, j0 = (it - q * o.nch) * kW8Cols, tile = q / o.nrb;
+    const uint32_t nt = w8_tokens(A.tiles, tile, A.cap);
+    if (j0 >= nt) continue;
+    r = __builtin_amdgcn_readfirstlane(r);
+    I.tile = __builtin_amdgcn_readfirstlane(tile);
+    I.j0 = __builtin_amdgcn_readfirstlane(j0);
     const affx_expert_tile* T = A.tiles + I.tile;
     I.codes = reinterpret_cast<const uint8_t*>(*AFFX_CONST_PTR(uint64_t, &T->codes));
     I.fields = reinterpret_cast<const uint8_t*>(*AFFX_CONST_PTR(uint64_t, &T->fields));
     I.tok = reinterpret_cast<const uint32_t*>(*AFFX_CONST_PTR(uint64_t, &T->tok));
-    I.n = __builtin_amdgcn_readfirstlane(w8_tokens(A.tiles, I.tile, A.cap));
-    I.rt = __builtin_amdgcn_readfirstlane((it - I.tile * nrb) * kW8LWaves + wv);
-    return I;
+    I.n = __builtin_amdgcn_readfirstlane(min(nt - j0, kW8Cols));
+    I.rt = __builtin_amdgcn_readfirstlane((q - tile * o.nrb) * kW8Waves + wv);
+    return true;
+  }
+  return false;
+}
+// The lane's four accumulator rows' scales.
+__device__ __forceinline__ uint2 w8_rscales(const W8a8Args& A, const W8Item& I, uint32_t kg) {
+  return *reinterpret_cast<const uint2*>(
+      reinterpret_cast<const uint16_t*>(*AFFX_CONST_PTR(uint64_t, &A.tiles[I.tile].rscales)) + I.rt * 16u + 4u * kg);
+}
+__device__ __forceinline__ void* w8_y(const W8a8Args& A, const W8Item& I, uint32_t& ld) {
+  const affx_expert_tile* T = A.tiles + I.tile;
+  const uint32_t l = *AFFX_CONST_PTR(uint32_t, &T->ld);
+  ld = l ? l : *AFFX_CONST_PTR(uint32_t, &T->nt);
+  return reinterpret_cast<void*>(*AFFX_CONST_PTR(uint64_t, &T->y));
+}
+// Stages one token of a column tile: its 1 KiB of activations (one direct-to-LDS instruction) and its
+// eight scales.
+__device__ __forceinline__ void w8_stage(const W8a8Args& A, const W8Item& I, uint32_t ct, uint32_t j, uint32_t lane,
+                                         uint8_t* row, float* sc) {
+  const uint32_t t = w8_row(I.tok, j);
+  const __amdgpu_buffer_rsrc_t r = buffer_rsrc(A.x8 + (uint64_t)t * A.cols + (uint64_t)ct * kTileCols, kTileCols);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, AFFX_LDS_PTR(row), 16, lane * 16u, 0, 0, 0);
+  const __amdgpu_buffer_rsrc_t q = buffer_rsrc(A.xs + (uint64_t)t * (A.cols / 128u) + ct * 8u, 32u);
+  if (lane < 8u) __builtin_amdgcn_raw_ptr_buffer_load_lds(q, AFFX_LDS_PTR(sc), 4, lane * 4u, 0, 0, 0);
+}
+// (the lane is counted where it is used: lane values held across the steps were spilled, and a
+// reload, a vector memory load, waits for every load in flight)
+__device__ __forceinline__ uint32_t w8_lane() {
+  uint32_t z = 0u;
+  AFFX_PIN(z);
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
+}
+
+// LDS: the codebook and two buffers of a column tile's token rows and scales, so two workgroups a CU (at
+// most 128 registers a wave). The steps of a workgroup are (item, column tile) pairs in order; each
+// step first requests the next step's unit and token rows, then decodes and multiplies its own, and
+// ends in one barrier.
+__global__ void __launch_bounds__(kW8T, 4) w8a8_gemm_kernel(W8a8Args A) {
+  __shared__ __align__(16) uint32_t lut_s[Lut<kW8KC, true>::kDwords];
+  // (two arrays a kind: the compiler can tell the buffer being read from the one being written)
+  __shared__ __align__(16) uint8_t xb0[kW8Cols * kW8Row], xb1[kW8Cols * kW8Row];
+  __shared__ __align__(16) float xs0[kW8Cols * 8], xs1[kW8Cols * 8];
+  const uint8_t* lut = reinterpret_cast<const uint8_t*>(lut_s);
+  const uint32_t tid = threadIdx.x;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t nct = A.cols / kTileCols, nrt = A.rows / kTileRows;
+  const W8Order o{(nrt + kW8Waves - 1) / kW8Waves, A.cap > kW8Cols ? A.cap / kW8Cols : 1u, A.items};
+  uint32_t r = 0;
+  W8Item I;
+  if (!w8_seek(A, o, r, wv, I)) return;  // (the whole workgroup)
+  auto stage = [&](const W8Item& J, uint32_t ct, uint8_t* xb, float* xs) {
+#pragma unroll
+    for (uint32_t j = wv; j < kW8Cols; j += kW8Waves)
+      if (j < J.n) w8_stage(A, J, ct, J.j0 + j, w8_lane(), xb + j * kW8Row, xs + j * 8u);
   };
-  uint32_t it = seek(blockIdx.x);
-  if (it >= items) return;  // (the whole workgroup)
-  Item I = open(it);
-  // token row wv of a column tile (1 KiB, one direct-to-LDS instruction) and its eight scales
-  auto stage = [&](const Item& J, uint32_t ct, uint8_t* xb, float* xs) {
-    if (wv >= J.n) return;
-    const uint32_t lane = lane_now();
-    const uint32_t t = w8_row(J.tok, wv);
-    const __amdgpu_buffer_rsrc_t r = buffer_rsrc(A.x8 + (uint64_t)t * A.cols + (uint64_t)ct * kTileCols, kTileCols);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, AFFX_LDS_PTR(xb + wv * kW8Row), 16, lane * 16u, 0, 0, 0);
-    const __amdgpu_buffer_rsrc_t q = buffer_rsrc(A.xs + (uint64_t)t * nkb + ct * 8u, 32u);
-    if (lane < 8u) __builtin_amdgcn_raw_ptr_buffer_load_lds(q, AFFX_LDS_PTR(xs + wv * 8u), 4, lane * 4u, 0, 0, 0);
-  };
-  auto load = [&](Unit& u, const Item& J, uint32_t ct) {
-    if (J.rt < nrt) load_unit_ordered(u, J.codes, J.fields, (uint64_t)J.rt * nct + ct, lane_now());
+  auto load = [&](Unit& u, const W8Item& J, uint32_t ct) {
+    if (J.rt < nrt) load_unit_ordered(u, J.codes, J.fields, (uint64_t)J.rt * nct + ct, w8_lane());
   };
 
   Unit ua, ub;
@@ -177,85 +219,57 @@ __global__ void __launch_bounds__(kW8LT, 4) w8a8_light_kernel(W8a8Args A) {
   {
     uint32_t cbv[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8LT];
-    build_lut<kW8KC, kW8LT, 4, true>(lut_s, cbv, tid);
-    if (tid < kSegCols / 4) reinterpret_cast<uint32_t*>(zero_s)[tid] = 0u;
+    for (int i = 0; i < 4; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8T];
+    build_lut<kW8KC, kW8T, 4, true>(lut_s, cbv, tid);
   }
   __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(0));
   __syncthreads();
 
-  constexpr int NQ = kW8Light / 4;
-  float out[NQ][4] = {};
+  float out[4] = {};
   uint32_t ct = 0;
-  // multiplies the unit by the tile's quads; Q of them (a template of the quad count: no branch
-  // between a step's table reads and its MFMAs)
-  auto mult = [&](auto qc, Unit& u, const uint8_t* xb, const float* xs) {
-    constexpr int Q = decltype(qc)::value;
-    const uint32_t lane = lane_now(), c = lane & 15, kg = lane >> 4, copy4 = ((lane >> 1) & (kW8KC - 1)) * 4u;
-    v4f acc[Q][2];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) acc[q][0] = acc[q][1] = v4f{0.f, 0.f, 0.f, 0.f};
-    const uint8_t* src[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const uint32_t jl = 4u * (uint32_t)q + (c >> 2);
-      src[q] = (c & 3u) == kg && jl < I.n ? xb + jl * kW8Row + kg * (uint32_t)kSegCols : zero_s;
-    }
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      uint32_t raw[8], bv[2];
-      pin_step(u, m);
-      lut_lookup_step<kW8KC, true>(u, lut, nullptr, copy4, m, raw, bv);
-      const v8i a = lut_finish(raw, bv);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        const v8i b = b_step(reinterpret_cast<const u32x4*>(src[q]), m);
-        acc[q][m / 4] = mfma(a, b, acc[q][m / 4]);
-      }
-      asm volatile("" ::: "memory");  // (one step's reads in flight at a time: registers)
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int q = 0; q < Q; ++q) w8_fold(acc[q][0], acc[q][1], xs + (4u * q + (c >> 2)) * 8u, out[q]);
-  };
-  // one step, of unit u from buffers (xb, xs), with the next step's going to un and (yb, ys); false after the last
+  // one step, of unit u from buffers (xb, xs), with the next step's going to un and (yb, ys); false
+  // after the last
   auto step = [&](Unit& u, Unit& un, const uint8_t* xb, const float* xs, uint8_t* yb, float* ys) -> bool {
     const bool last = ct + 1 == nct;
-    const uint32_t itn = last ? seek(it + gridDim.x) : it;
-    const bool more = itn < items;
-    Item N = I;
-    if (last && more) N = open(itn);
+    W8Item N = I;
+    bool more = true;
+    if (last) more = w8_seek(A, o, ++r, wv, N);
     const bool rows_ok = I.rt < nrt;
-    const uint32_t lane = lane_now(), c = lane & 15, kg = lane >> 4;
+    const uint32_t lane = w8_lane(), c = lane & 15, kg = lane >> 4, copy4 = ((lane >> 1) & (kW8KC - 1)) * 4u;
     // (requested here, used after the last column tile's products)
     uint2 rsv = {0u, 0u};
-    if (last && rows_ok)
-      rsv = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(*AFFX_CONST_PTR(uint64_t, &A.tiles[I.tile].rscales)) +
-                                            I.rt * 16u + 4u * kg);
+    if (last && rows_ok) rsv = w8_rscales(A, I, kg);
     if (more) {
       load(un, N, last ? 0u : ct + 1u);
       stage(N, last ? 0u : ct + 1u, yb, ys);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (rows_ok) {
-      if (I.n > 4u) mult(IConst<2>{}, u, xb, xs);
-      else mult(IConst<1>{}, u, xb, xs);
+      // (a column past the item's tokens multiplies what its row of the LDS holds and is not stored)
+      v4f res[2][4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        v8i f[4];
+        w8_half(u, lut, copy4, h, f);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          res[h][g] = mfma(f[g], w8_b(xb + c * kW8Row, kg, 2 * g + h), v4f{0.f, 0.f, 0.f, 0.f});
+          asm volatile("" ::: "memory");
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      w8_fold(res, xs + c * 8u, out);
     }
     if (last) {
-      if (rows_ok && (c & 3u) == 0u) {
-        void* y = reinterpret_cast<void*>(*AFFX_CONST_PTR(uint64_t, &A.tiles[I.tile].y));
-        const uint32_t ldt = *AFFX_CONST_PTR(uint32_t, &A.tiles[I.tile].ld), ntt = *AFFX_CONST_PTR(uint32_t, &A.tiles[I.tile].nt);
-#pragma unroll
-        for (int q = 0; q < NQ; ++q)
-          if (4u * q + (c >> 2) < I.n) w8_store(A, y, ldt ? ldt : ntt, I.rt * 16u + 4u * kg, 4u * q + (c >> 2), out[q], rsv);
+      if (rows_ok && c < I.n) {
+        uint32_t ld;
+        void* y = w8_y(A, I, ld);
+        w8_store(A, y, ld, I.rt * 16u + 4u * kg, I.j0 + c, out, rsv);
       }
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) out[q][v] = 0.f;
+      for (int v = 0; v < 4; ++v) out[v] = 0.f;
     }
     if (!more) return false;
-    it = itn;
     I = N;
     ct = last ? 0u : ct + 1u;
     __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(0));
@@ -266,167 +280,9 @@ __global__ void __launch_bounds__(kW8LT, 4) w8a8_light_kernel(W8a8Args A) {
   }
 }
 
-// ---- heavy tiles --------------------------------------------------------------------------------
-// Four waves, 64 rows of a tile an item. NQ: the most quads of the launch's tiles; a tile runs the
-// passes and quads that its tokens fill. The tokens are staged in passes of at most kW8Pass.
-constexpr uint32_t kW8Pass = 32;
-
-template <int NQ>
-__global__ void __launch_bounds__(kW8T) w8a8_gemm_kernel(W8a8Args A) {
-  constexpr int NP = (4 * NQ + (int)kW8Pass - 1) / (int)kW8Pass;  // passes
-  constexpr int QP = NQ / NP;                                        // quads a pass
-  AFFX_DYN_LDS(lds);  // xb [4 QP][kW8Row] activation rows of the pass, then xsl [4 x 64] f32 scales
-  uint8_t* xb = lds;
-  float* xsl = reinterpret_cast<float*>(lds + 4u * QP * kW8Row);
-  __shared__ __align__(16) uint32_t lut_s[Lut<kW8KC, true>::kDwords];
-  const uint8_t* lut = reinterpret_cast<const uint8_t*>(lut_s);
-  // items tile-major, then 64-row blocks
-  const uint32_t nrb = (A.rows / kTileRows + kW8Waves - 1) / kW8Waves, items = A.n_tiles * nrb;
-  const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t c = lane & 15, kg = lane >> 4, copy4 = ((lane >> 1) & (kW8KC - 1)) * 4u;
-  const uint32_t nct = A.cols / kTileCols, nkb = A.cols / 128u;
-  auto seek = [&](uint32_t it) -> uint32_t {
-    for (; it < items; it += gridDim.x)
-      if (w8_tokens(A.tiles, it / nrb, A.cap) > kW8Light) break;
-    return it;
-  };
-  uint32_t it = seek(blockIdx.x);
-  if (it >= items) return;  // (the whole workgroup)
-  {
-    uint32_t cbv[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8T];
-    build_lut<kW8KC, kW8T, 8, true>(lut_s, cbv, tid);
-  }
-  const __amdgpu_buffer_rsrc_t xs_r = buffer_rsrc(A.xs, 0x7FFFFFF0u);
-
-  for (; it < items; it = seek(it + gridDim.x)) {
-    const uint32_t tile = it / nrb, rb = it - tile * nrb;
-    const affx_expert_tile* T = A.tiles + tile;
-    const uint32_t ntok = w8_tokens(A.tiles, tile, A.cap);
-    const uint32_t rt = rb * kW8Waves + wv;
-    const bool rows_ok = rt * kTileRows < A.rows;
-    const uint32_t* tok = reinterpret_cast<const uint32_t*>(*AFFX_CONST_PTR(uint64_t, &T->tok));
-    const uint8_t* codes = reinterpret_cast<const uint8_t*>(*AFFX_CONST_PTR(uint64_t, &T->codes));
-    const uint8_t* fields = reinterpret_cast<const uint8_t*>(*AFFX_CONST_PTR(uint64_t, &T->fields));
-    // the lane's four accumulator rows' scales
-    uint2 rsv = {0u, 0u};
-    if (rows_ok)
-      rsv = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(*AFFX_CONST_PTR(uint64_t, &T->rscales)) +
-                                            rt * 16u + 4u * kg);
-    // the lane's scale dword of each pass (token pass * 4 QP + d / 8, block 8 ct + d % 8 for
-    // d = 64 wave + lane; past the pass's tokens: out of the buffer's range, zero)
-    uint32_t xs_off[NP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const uint32_t d = 64u * wv + lane, jj = (uint32_t)p * 4u * QP + d / 8u;
-      xs_off[p] = (d < 32u * QP && jj < ntok) ? ((tok ? tok[jj] : jj) * nkb + d % 8u) * 4u : 0x7FFFFFF0u;
-    }
-
-    float out[NQ][4];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) out[q][v] = 0.f;
-
-    // a pass's LDS: the pass's token rows, QP per wave at most (1 KiB each, one direct-to-LDS load
-    // instruction), and one scale instruction per wave
-    auto stage = [&](int p, uint32_t ct) {
-#pragma unroll
-      for (int i = 0; i < QP; ++i) {
-        const uint32_t jl = wv + 4u * (uint32_t)i, j = (uint32_t)p * 4u * QP + jl;
-        if (j >= ntok) break;  // (rows past the tile's tokens are not read)
-        const __amdgpu_buffer_rsrc_t r =
-            buffer_rsrc(A.x8 + (uint64_t)w8_row(tok, j) * A.cols + (uint64_t)ct * kTileCols, kTileCols);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, AFFX_LDS_PTR(xb + jl * kW8Row), 16, lane * 16u, 0, 0, 0);
-      }
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xs_r, AFFX_LDS_PTR(xsl + 64u * wv), 4, xs_off[p] + ct * 32u, 0, 0, 0);
-    };
-
-    for (uint32_t ct = 0; ct < nct; ++ct) {
-      // this wave's unit of the column tile first (loads complete in issue order)
-      Unit u;
-      load_unit_ordered(u, codes, fields, (uint64_t)(rows_ok ? rt : 0u) * nct + ct, lane);
-      v8i a[8];
-#pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        if ((uint32_t)p * 4u * QP >= ntok) break;  // (the same for the whole workgroup)
-        __syncthreads();  // the previous pass's reads of the LDS are done
-        stage(p, ct);
-        if (p == 0) {
-          // the wave tile's eight A fragments, while the pass's rows arrive
-#pragma unroll
-          for (int m = 0; m < 8; ++m) {
-            uint32_t raw[8], bv[2];
-            pin_step(u, m);
-            lut_lookup_step<kW8KC, true>(u, lut, nullptr, copy4, m, raw, bv);
-            a[m] = lut_finish(raw, bv);
-            asm volatile("" ::: "memory");  // one step's table reads in flight at a time (registers)
-          }
-        }
-        __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(0));
-        __syncthreads();
-        if (!rows_ok) continue;
-#pragma unroll
-        for (int ql = 0; ql < QP; ++ql) {
-          const int q = p * QP + ql;
-          if (4u * (uint32_t)q >= ntok) break;
-          const uint32_t jl = 4u * (uint32_t)ql + (c >> 2);
-          const bool live = (c & 3u) == kg && (uint32_t)p * 4u * QP + jl < ntok;
-          const uint8_t* bsrc = xb + jl * kW8Row + kg * (uint32_t)kSegCols;
-          v4f acc0 = v4f{0.f, 0.f, 0.f, 0.f}, acc1 = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int m = 0; m < 8; ++m) {
-            v8i b = v8i{0, 0, 0, 0, 0, 0, 0, 0};
-            if (live) b = b_step(reinterpret_cast<const u32x4*>(bsrc), m);
-            if (m < 4)
-              acc0 = mfma(a[m], b, acc0);
-            else
-              acc1 = mfma(a[m], b, acc1);
-          }
-          w8_fold(acc0, acc1, xsl + jl * 8u, out[q]);
-          // one quad at a time: the next quad's B reads are not hoisted over this one's MFMAs (a
-          // compiler memory barrier; the registers of every quad's operands at once would cut the
-          // waves a SIMD holds to one)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) AFFX_PIN(out[q][v]);
-          asm volatile("" ::: "memory");
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    }
-    if (!rows_ok || (c & 3u) != 0u) continue;
-    void* y = reinterpret_cast<void*>(*AFFX_CONST_PTR(uint64_t, &T->y));
-    const uint32_t ldt = *AFFX_CONST_PTR(uint32_t, &T->ld), ld = ldt ? ldt : *AFFX_CONST_PTR(uint32_t, &T->nt);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const uint32_t j = 4u * q + (c >> 2);
-      if (j < ntok) w8_store(A, y, ld, rt * 16u + 4u * kg, j, out[q], rsv);
-    }
-  }
-}
-
 }  // namespace affx
 
 using namespace affx;
-
-namespace {
-
-// persistent grids: as many workgroups as the device holds at once (two a CU in either kernel)
-template <int NQ>
-int w8a8_launch(const W8a8Args& A, uint32_t grid, hipStream_t s) {
-  constexpr int NP = (4 * NQ + (int)kW8Pass - 1) / (int)kW8Pass, QP = NQ / NP;
-  const uint32_t lds = 4u * QP * kW8Row + 4u * 64u * 4u;
-  int rc = check_hip(hipFuncSetAttribute((const void*)w8a8_gemm_kernel<NQ>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)lds),
-                     "hipFuncSetAttribute(w8a8)");
-  if (rc) return rc;
-  hipLaunchKernelGGL((w8a8_gemm_kernel<NQ>), dim3(grid), dim3(kW8T), lds, s, A);
-  return check_launch("w8a8_gemm_kernel");
-}
-
-}  // namespace
 
 extern "C" int affx_expert_gemm_w8a8(const affx_expert_tile* tiles, uint32_t n_tiles, uint32_t max_nt, const void* x8,
                                      const float* xs, const uint32_t* codebook, uint32_t rows, uint32_t cols,
@@ -449,24 +305,24 @@ extern "C" int affx_expert_gemm_w8a8(const affx_expert_tile* tiles, uint32_t n_t
   A.cols = cols;
   A.wscale = wscale;
   A.y_bf16 = y_bf16 ? 1 : 0;
-  hipStream_t s = (hipStream_t)stream;
-  A.n_tiles = n_tiles;
   const uint32_t nq = (max_nt + 3u) / 4u;
   A.cap = nq <= 1 ? 4u : nq <= 2 ? 8u : nq <= 4 ? 16u : nq <= 8 ? 32u : 64u;
+  const uint32_t nch = A.cap > kW8Cols ? A.cap / kW8Cols : 1u;
+  const uint64_t items = (uint64_t)n_tiles * ((rows / kTileRows + kW8Waves - 1) / kW8Waves) * nch;
+  if (items > 0x7FFFFFFFull) {
+    // (a matrix of over a million rows: half the tiles at a time)
+    int rc = affx_expert_gemm_w8a8(tiles, n_tiles / 2, max_nt, x8, xs, codebook, rows, cols, wscale, y_bf16, stream);
+    return rc ? rc : affx_expert_gemm_w8a8(tiles + n_tiles / 2, n_tiles - n_tiles / 2, max_nt, x8, xs, codebook, rows,
+                                           cols, wscale, y_bf16, stream);
+  }
+  A.items = (uint32_t)items;
   int dev = 0, cus = 0, rc;
   if ((rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) ||
       (rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
     return rc;
-  auto grid = [&](uint32_t waves) {
-    const uint64_t items = (uint64_t)n_tiles * ((rows / kTileRows + waves - 1) / waves), most = 2ull * (uint32_t)(cus > 0 ? cus : 1);
-    return (uint32_t)(items < most ? items : most);
-  };
-  // the heavy tiles first: their items are the longer ones
-  if (A.cap > kW8Light) {
-    const uint32_t g = grid(kW8Waves);
-    rc = nq <= 4 ? w8a8_launch<4>(A, g, s) : nq <= 8 ? w8a8_launch<8>(A, g, s) : w8a8_launch<16>(A, g, s);
-    if (rc) return rc;
-  }
-  hipLaunchKernelGGL(w8a8_light_kernel, dim3(grid(kW8LWaves)), dim3(kW8LT), 0, s, A);
-  return check_launch("w8a8_light_kernel");
+  // persistent: as many workgroups as the device holds at once, a multiple of the token groups
+  const uint32_t most = 2u * (uint32_t)(cus > 1 ? cus / 2 * 2 : 2);
+  const uint32_t grid = A.items < most ? A.items : most;
+  hipLaunchKernelGGL(w8a8_gemm_kernel, dim3(grid), dim3(kW8T), 0, (hipStream_t)stream, A);
+  return check_launch("w8a8_gemm_kernel");
 }

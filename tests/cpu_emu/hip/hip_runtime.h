@@ -171,6 +171,17 @@ inline int __builtin_amdgcn_update_dpp(int old, int src, int ctrl, int, int, boo
   const int v = emu_exchange(src, from < 0 ? l : (uint32_t)from);
   return from < 0 ? (bound_ctrl ? 0 : old) : v;
 }
+// lane-row swaps (rows of 16 lanes): 32: the upper half of a with the lower half of b; 16: the odd
+// rows of a with the even rows of b
+typedef uint32_t emu_v2u __attribute__((ext_vector_type(2)));
+inline emu_v2u emu_swap(uint32_t a, uint32_t b, uint32_t half) {
+  const uint32_t l = emu_lane();
+  const bool up = (l & half) != 0;  // this lane is of the upper half / an odd row
+  const uint32_t xa = emu_exchange(a, up ? l : l + half), xb = emu_exchange(b, up ? l - half : l);
+  return emu_v2u{up ? xb : a, up ? b : xa};
+}
+inline emu_v2u __builtin_amdgcn_permlane32_swap(uint32_t a, uint32_t b, bool, bool) { return emu_swap(a, b, 32); }
+inline emu_v2u __builtin_amdgcn_permlane16_swap(uint32_t a, uint32_t b, bool, bool) { return emu_swap(a, b, 16); }
 inline uint64_t __ballot(int pred) {
   emu_blk->xfer[emu_wave()][emu_lane()][0] = pred ? 1 : 0;
   emu_wave_sync();

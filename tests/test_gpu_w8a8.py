@@ -113,3 +113,48 @@ def test_expert_gemm_w8a8_refusals(ax):
     assert f(t.data_ptr(), 1, 4, x8.data_ptr(), xs.data_ptr(), cb.data_ptr(), 24, 1024, 1.0, 0, None) == AFFX_DECLINED
     assert f(t.data_ptr(), 1, 4, x8.data_ptr(), xs.data_ptr(), cb.data_ptr(), 16, 1000, 1.0, 0, None) == AFFX_DECLINED
     assert f(t.data_ptr(), 1, 4, x8.data_ptr() + 4, xs.data_ptr(), cb.data_ptr(), 16, 1024, 1.0, 0, None) < 0
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 1024), (144, 1024), (128, 3072)])
+@pytest.mark.parametrize("max_nt", [1, 4, 5, 8, 16, 17, 32, 33, 64])
+def test_expert_gemm_w8a8_tile_edges(ax, orc, c1_codebook, rows, cols, max_nt):
+    """Tiles at the edges of the 16-token groups and of the row blocks (one row tile; nine; whole), odd
+    and even counts of column tiles, pads among them, in one launch: every output against the oracle at
+    the bound of the test above, columns beyond a tile's tokens untouched."""
+    from affinity_amd._lib import AffxExpertTile, check, lib
+    rng = np.random.default_rng(rows + cols + max_nt)
+    cbf = orc.unpack_codebook(c1_codebook)
+    x8 = rng.integers(0, 256, (80, cols), dtype=np.uint8)
+    x8[(x8 & 0x7F) == 0x7F] ^= 1
+    xs = rng.uniform(0.01, 2.0, (80, cols // 128)).astype(np.float32)
+    counts = [n for n in (1, 4, 5, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64) if n <= max_nt]
+    counts = counts + [0, max_nt]
+    tiles = (AffxExpertTile * len(counts))()
+    keep, host = [], []
+    for q, nt in enumerate(counts):
+        c = rng.integers(0, 256, rows * cols * 10 // 32, dtype=np.uint8)
+        f = rng.integers(0, 256, rows * cols * 6 // 128, dtype=np.uint8)
+        r = (rng.uniform(4e-4, 2e-3, rows).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        dc, df = np.zeros_like(c), np.zeros_like(f)
+        check(lib().affx_matrix_to_device_layout(c.ctypes.data, f.ctypes.data, dc.ctypes.data, df.ctypes.data, rows,
+                                                 cols), "layout")
+        tok = rng.integers(0, 80, max(nt, 1)).astype(np.uint32) if q % 2 else None
+        d = [torch.from_numpy(a).cuda() for a in (dc, df, r.view(np.int16))]
+        td = None if tok is None else torch.from_numpy(tok.view(np.int32)).cuda()
+        y = torch.full((rows, 70), 7.0, device="cuda")
+        keep += [d, td, y]
+        host.append((c, f, r, tok, y))
+        tiles[q] = AffxExpertTile(d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(),
+                                  None if td is None else td.data_ptr(), y.data_ptr(), nt, 70)
+    t = torch.from_numpy(np.frombuffer(bytes(tiles), np.uint8).copy()).cuda()
+    gx, gs = torch.from_numpy(x8).cuda(), torch.from_numpy(xs).cuda()
+    cb = torch.from_numpy(c1_codebook.view(np.int32)).cuda()
+    check(lib().affx_expert_gemm_w8a8(t.data_ptr(), len(counts), max_nt, gx.data_ptr(), gs.data_ptr(), cb.data_ptr(),
+                                      rows, cols, 0.5, 0, None), "gemm_w8a8")
+    torch.cuda.synchronize()
+    for nt, (c, f, r, tok, y) in zip(counts, host):
+        y = y.cpu().numpy()
+        assert (y[:, nt:] == 7.0).all()
+        if nt:
+            ref = orc.expert_gemm_w8a8(c, f, r, tok, nt, x8, xs, cbf, rows, cols, 0.5, y_bf16=False)
+            assert rel_l2(y[:, :nt], ref) <= 2e-4, nt
