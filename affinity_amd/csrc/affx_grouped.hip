@@ -828,6 +828,9 @@ __global__ void __launch_bounds__(kGT, GTile<CT>::kLight ? 4 : 1) grouped_gemm_k
       lut_lookup_step<kGKC, true>(u[r], lut, btbl, copy4, 0, raw, sx);
       a_cur[r] = lut_finish(raw, sx);
     }
+    uint32_t raw_c[4];  // the table reads in flight from one quarter of a step to the next (heavy tiles)
+    uint2 sx_c;
+    if constexpr (!GTile<CT>::kLight) lut_lookup_block<kGKC, 1, 0>(u[0], lut, btbl, copy4, raw_c, sx_c);
     v4f acc[kGRT][CT];
 #pragma unroll
     for (int r = 0; r < kGRT; ++r)
@@ -865,17 +868,17 @@ __global__ void __launch_bounds__(kGT, GTile<CT>::kLight ? 4 : 1) grouped_gemm_k
                        more ? rt_of(r) * nst + s + 1 : cont ? rt_of(r) * nst : 0u, lane);
       }
       __builtin_amdgcn_sched_barrier(0);
-      // The step is 12 groups, one per B column tile: the tile's two fragment reads go out two
-      // groups ahead, its MFMAs (one per row tile) are each followed by a share of the VALU work of
-      // the next step (groups 4-5: code addresses and table reads of unit g - 4; groups 8-9: the
-      // sign/scale finish of unit g - 8, whose reads were issued four groups earlier). The VALU of
-      // one wave runs while the matrix core works through the other wave's MFMAs. The groups are
-      // placed so that the table reads and the next A fragments are live for a third of the step
-      // only: with two waves per SIMD a wave has 256 registers, accumulators included. (Step 0 of
-      // the next 1024 columns after step 7: the ring has reloaded every register those reads use.)
+      // (heavy tiles) The step is four quarters. Each looks up one block (four codes: addresses and table
+      // reads) of the next step's A fragments, the last quarter the first block of the step after, and
+      // finishes (sign and scale) the block that the quarter before looked up, between its share of
+      // the MFMAs, whose B fragments are read two column tiles ahead: about three VALU operations an
+      // MFMA all along the step. (A unit's eight codes in one of twelve groups, finished four groups
+      // later, left most MFMAs without and some with fifteen: C4 2044 -> 2028 us, the same
+      // process.) The VALU of one wave runs while the matrix core works through the other wave's
+      // MFMAs. Few table reads and next A fragments are live at a time: with two waves per SIMD a wave
+      // has 256 registers, accumulators included. (Step 0 of the next 1024 columns after step 7: the
+      // ring has reloaded every register those reads use.)
       constexpr int mn = (m + 1) & 7;
-      constexpr int kLook = CT >= 12 ? 4 : CT >= 8 ? 2 : 0, kFin = CT >= 12 ? 8 : CT >= 8 ? 5 : 2;
-      uint32_t rawn[kGRT][8], sxn[kGRT][GTile<CT>::kLight ? 2 : 4];
       v8i a_next[kGRT];
       auto bread = [&](int ct) -> v8i {
         const u32x4 lo = *reinterpret_cast<const u32x4*>(bcur + ct * 2048 + bo0);
@@ -887,6 +890,7 @@ __global__ void __launch_bounds__(kGT, GTile<CT>::kLight ? 4 : 1) grouped_gemm_k
       };
       if constexpr (GTile<CT>::kLight) {
         // (four waves a SIMD: the other waves' work covers the table reads' and MFMAs' latency)
+        uint32_t rawn[kGRT][8], sxn[kGRT][2];
         static_for<0, CT>([&](auto cc) {
           constexpr int ct = decltype(cc)::value;
           if (ct > 0 && n_cur <= (uint32_t)(ct * TPG)) return;  // no token there (the same for the whole workgroup)
@@ -907,31 +911,37 @@ __global__ void __launch_bounds__(kGT, GTile<CT>::kLight ? 4 : 1) grouped_gemm_k
         }
       } else {
       v8i bq0 = bread(0), bq1 = bread(1);
-      static_for<0, CT>([&](auto cc) {
-        constexpr int ct = decltype(cc)::value;
-        v8i bq2;
-        if constexpr (ct + 2 < CT) bq2 = bread(ct + 2);
+      static_for<0, 4>([&](auto gc) {
+        constexpr int g = decltype(gc)::value;
+        constexpr int q = (g + 1) & 3;  // the quarter looked up: block q & 1 of unit q >> 1
+        uint32_t rawl[4];
+        uint2 sxl;
+        lut_lookup_block<kGKC, g == 3 ? (m + 2) & 7 : mn, q & 1>(u[q >> 1], lut, btbl, copy4, rawl, sxl);
+        static_for<0, CT / 4>([&](auto cc) {
+          constexpr int ct = g * (CT / 4) + decltype(cc)::value;
+          v8i bq2;
+          if constexpr (ct + 2 < CT) bq2 = bread(ct + 2);
 #pragma unroll
-        for (int r = 0; r < kGRT; ++r) acc[r][ct] = mfma(a_cur[r], bq0, acc[r][ct]);
-        if constexpr (ct >= kLook && ct < kLook + kGRT) {
-          pin_step<mn>(u[ct - kLook]);
-          lut_lookup<kGKC, mn, true>(u[ct - kLook], lut, btbl, copy4, rawn[ct - kLook], sxn[ct - kLook]);
-        } else if constexpr (ct >= kFin && ct < kFin + kGRT) {
-          a_next[ct - kFin] = lut_finish(rawn[ct - kFin], sxn[ct - kFin]);
-          AFFX_PIN(a_next[ct - kFin]);  // computed here, not sunk into the next step
+          for (int r = 0; r < kGRT; ++r) acc[r][ct] = mfma(a_cur[r], bq0, acc[r][ct]);
+          bq0 = bq1;
+          if constexpr (ct + 2 < CT) bq1 = bq2;
+        });
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a_next[g >> 1][4 * (g & 1) + i] = (int)((raw_c[i] ^ sx_c.x) + sx_c.y);
+          raw_c[i] = rawl[i];
         }
-        // {one MFMA, then up to 12 VALU} per row tile, then the LDS reads (8, 12, 16, 24 and no
-        // pattern measured within about 1 % of each other)
+        sx_c = sxl;
 #pragma unroll
-        for (int i = 0; i < kGRT; ++i) {
+        for (int i = 0; i < kGRT * CT / 4; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x100, 10, 0);
         __builtin_amdgcn_sched_barrier(0);
-        bq0 = bq1;
-        if constexpr (ct + 2 < CT) bq1 = bq2;
       });
+#pragma unroll
+      for (int r = 0; r < kGRT; ++r) AFFX_PIN(a_next[r]);  // computed here, not sunk into the next step
       }
       // the accumulators are materialised here (else the compiler sinks every MFMA below all
       // eight steps' table reads and holds those in registers). They stay in VGPRs: a kernel that

@@ -112,6 +112,26 @@ __device__ __forceinline__ void lut_lookup(const Unit& u, const uint8_t* lds, co
   }
 }
 
+// One block's half of lut_lookup (block 2 MSTEP + B): four table reads, the sign mask and exponent add from
+// the block table. Pins the registers it reads, as pin_step does for the whole step.
+template <int KC, int MSTEP, int B>
+__device__ __forceinline__ void lut_lookup_block(Unit& u, const uint8_t* lds, const uint8_t* btbl, uint32_t copy4,
+                                                 uint32_t (&raw)[4], uint2& sx) {
+  constexpr int I = 8 * MSTEP + 4 * B, F = 12 * MSTEP + 6 * B;
+  constexpr int k0 = (10 * I - 6) < 0 ? 0 : (10 * I - 6) >> 5, k1 = (10 * I + 39) >> 5 > 19 ? 19 : (10 * I + 39) >> 5;
+#pragma unroll
+  for (int k = k0; k <= k1; ++k) AFFX_PIN(u.c[k]);
+  AFFX_PIN(u.f[F >> 5]);
+  if constexpr (((F + 5) >> 5) != (F >> 5)) AFFX_PIN(u.f[(F + 5) >> 5]);
+  const uint32_t fb = stream_bits<3>(u.f, F, 6);
+  const uint32_t vb = (((fb >> 4) & 3u) << Lut<KC>::kVarSh) | copy4;
+  raw[0] = *reinterpret_cast<const uint32_t*>(lds + code_addr<KC, I + 0>(u.c, vb));
+  raw[1] = *reinterpret_cast<const uint32_t*>(lds + code_addr<KC, I + 1>(u.c, vb));
+  raw[2] = *reinterpret_cast<const uint32_t*>(lds + code_addr<KC, I + 2>(u.c, vb));
+  raw[3] = *reinterpret_cast<const uint32_t*>(lds + code_addr<KC, I + 3>(u.c, vb));
+  sx = *reinterpret_cast<const uint2*>(btbl + ((fb << 3) & 0x78u));
+}
+
 // A fragment from the table reads: sign flip, exponent add, one v_xad per dword
 // (src/gpu/expert_kernel.hip:594-617; the rotation, src/quant/blockquant.cpp:826-828, is in the
 // table).
