@@ -116,16 +116,65 @@ __device__ __forceinline__ uint32_t n_cls_of(uint32_t c, uint32_t tt, uint32_t t
   const uint32_t r = c % tt;
   return (k == k0 ? c / tt : 0u) + (r != 0u && tile_cls(r, tpg) == k ? 1u : 0u);
 }
-// Writes the tiles of one expert (slots b0 .. b0 + c - 1): the full ones from tiles[at[k0]], the
-// partial one at tiles[at[its class]] (past the full ones where that is k0).
-__device__ __forceinline__ void put_tiles(Tile* tiles, uint32_t e, uint32_t b0, uint32_t c, uint32_t tt, uint32_t tpg,
-                                          uint32_t k0, const uint32_t (&at)[kNCls]) {
+// The wide tiles that are split into a class 1 and a class 2 tile each (12 column tiles = 8 + 4). A class
+// runs in rounds of a tile's row blocks over the grid (the tiles dealt to the 8 XCDs in turn), so a
+// few tiles past a whole round cost a round in which most of the device idles: 194 wide gate/up
+// tiles over 256 workgroups took 13 rounds for 12.1 rounds' work. They are split where the round saved
+// is worth more than those that the narrower classes grow by; cost: an item's time in each
+// class (gate/up with two terms 49, 36 and 26 us; the other forms' ratios are within a tenth).
+__device__ __forceinline__ uint32_t split_wide(const uint32_t (&n)[kNCls], uint32_t nrb, uint32_t grid, uint32_t room) {
+  static_assert(kClsCT[0] == kClsCT[1] + kClsCT[2], "a wide tile is one of each");
+  constexpr uint32_t cost[3] = {49, 36, 26};
+  auto rounds = [&](uint32_t t) { return ((t + 7u) / 8u * 8u * nrb + grid - 1u) / grid; };
+  const uint32_t r = rounds(n[0]);
+  if (r == 0) return 0u;
+  const uint32_t left = n[0] - min(n[0], (r - 1u) * grid / nrb / 8u * 8u);
+  if (left > room) return 0u;
+  const uint32_t more = (rounds(n[1] + left) - rounds(n[1])) * cost[1] + (rounds(n[2] + left) - rounds(n[2])) * cost[2];
+  return more < cost[0] ? left : 0u;
+}
+// One GEMM's tiles: class k's n[k] tiles from tiles[base[k]]; the wide ones from index keep on are split,
+// their parts following the other tiles of classes 1 and 2.
+struct TileSet {
+  uint32_t base[kNCls], n[kNCls], keep;
+};
+__device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, uint32_t nrb, uint32_t grid,
+                                            uint32_t max_tiles) {
+  TileSet t;
+  uint32_t need = 0;
+#pragma unroll
+  for (int k = 0; k < kNCls; ++k) {
+    t.n[k] = tot[k];
+    need += tot[k];
+  }
+  const uint32_t split = k0 == 0 && need <= max_tiles ? split_wide(t.n, nrb, grid, max_tiles - need) : 0u;
+  t.keep = t.n[0] - split;
+  t.base[0] = 0;
+  t.base[1] = t.keep;
+  t.base[2] = t.base[1] + t.n[1] + split;
+#pragma unroll
+  for (int k = 3; k < kNCls; ++k) t.base[k] = t.base[k - 1] + t.n[k - 1] + (k == 3 ? split : 0u);
+  return t;
+}
+// Writes the tiles of one expert (slots b0 .. b0 + c - 1), whose first of class k is the class's at[k]-th:
+// the full ones of class k0, the partial one of its class (past the full ones where that is k0).
+__device__ __forceinline__ void put_tiles(Tile* tiles, const TileSet& t, uint32_t e, uint32_t b0, uint32_t c, uint32_t tt,
+                                          uint32_t tpg, uint32_t k0, const uint32_t* at) {
   const uint32_t full = c / tt, r = c % tt, kr = r ? tile_cls(r, tpg) : kNCls;
+  auto put = [&](int k, uint32_t i, uint32_t s0, uint32_t n) {
+    if (k == 0 && i >= t.keep) {
+      const uint32_t d = i - t.keep, n1 = (uint32_t)kClsCT[1] * tpg;  // (a wide tile has more tokens than that)
+      tiles[t.base[1] + t.n[1] + d] = Tile{e, s0, n1};
+      tiles[t.base[2] + t.n[2] + d] = Tile{e, s0 + n1, n - n1};
+    } else {
+      tiles[t.base[k] + i] = Tile{e, s0, n};
+    }
+  };
 #pragma unroll
   for (int k = 0; k < kNCls; ++k) {
     if ((uint32_t)k == k0)
-      for (uint32_t i = 0; i < full; ++i) tiles[at[k] + i] = Tile{e, b0 + i * tt, tt};
-    if ((uint32_t)k == kr) tiles[at[k] + ((uint32_t)k == k0 ? full : 0u)] = Tile{e, b0 + full * tt, r};
+      for (uint32_t i = 0; i < full; ++i) put(k, at[k] + i, b0 + i * tt, tt);
+    if ((uint32_t)k == kr) put(k, at[k] + ((uint32_t)k == k0 ? full : 0u), b0 + full * tt, r);
   }
 }
 
@@ -140,6 +189,7 @@ struct PlanOut {
   Tile* tiles1;
   Tile* tiles2;
   uint32_t max_tiles1, max_tiles2;
+  uint32_t nrb1, nrb2, grid;  // row blocks of a tile of each GEMM, workgroups of a GEMM's launch at most
 };
 constexpr uint32_t kPlanSums = (1 + 2 * kNCls) * (kPlanThreads / 64 + 1);
 __device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own_slots, uint32_t n_slots_in,
@@ -164,26 +214,21 @@ __device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own
   for (int k = 0; k < kNCls; ++k) { need1 += tot[1 + k]; need2 += tot[1 + kNCls + k]; }
   // a caller's overlapping ranges could ask for more tiles than the workspace holds: then no tile
   const bool fits = need1 <= o.max_tiles1 && need2 <= o.max_tiles2;
+  const TileSet t1 = tile_set(tot + 1, k01, o.nrb1, o.grid, o.max_tiles1);
+  const TileSet t2 = tile_set(tot + 1 + kNCls, k02, o.nrb2, o.grid, o.max_tiles2);
   if (fits && tid < n_experts) {
     if (!own_slots) o.offsets[tid] = b0;
-    uint32_t at1[kNCls], at2[kNCls], base1 = 0, base2 = 0;
-#pragma unroll
-    for (int k = 0; k < kNCls; ++k) {
-      at1[k] = base1 + v[1 + k];
-      at2[k] = base2 + v[1 + kNCls + k];
-      base1 += tot[1 + k];
-      base2 += tot[1 + kNCls + k];
-    }
-    put_tiles(o.tiles1, tid, b0, c, tt1, tpg1, k01, at1);
-    put_tiles(o.tiles2, tid, b0, c, tt2, tpg2, k02, at2);
+    put_tiles(o.tiles1, t1, tid, b0, c, tt1, tpg1, k01, v + 1);
+    put_tiles(o.tiles2, t2, tid, b0, c, tt2, tpg2, k02, v + 1 + kNCls);
   }
   if (tid == 0) {
     if (!own_slots) o.offsets[n_experts] = tot[0];
     o.hdr->n_slots = own_slots ? n_slots_in : tot[0];
 #pragma unroll
     for (int k = 0; k < kNCls; ++k) {
-      o.hdr->n_cls[0][k] = fits ? tot[1 + k] : 0u;
-      o.hdr->n_cls[1][k] = fits ? tot[1 + kNCls + k] : 0u;
+      const uint32_t s1 = t1.n[0] - t1.keep, s2 = t2.n[0] - t2.keep;
+      o.hdr->n_cls[0][k] = fits ? (k == 0 ? t1.keep : t1.n[k] + (k <= 2 ? s1 : 0u)) : 0u;
+      o.hdr->n_cls[1][k] = fits ? (k == 0 ? t2.keep : t2.n[k] + (k <= 2 ? s2 : 0u)) : 0u;
     }
     o.hdr->tx = tx;
     o.hdr->bad = fits ? 0u : 1u;
@@ -1197,6 +1242,7 @@ using namespace affx;
 namespace {
 
 
+constexpr uint32_t kSplitRoom = 64;
 struct GroupedWs {
   uint64_t hdr, offsets, run, slot_tok, slot_w, ord, hist, tiles1, tiles2, sigma, tok_sigma, zeros, xq, aq, z, total;
   uint32_t max_tiles1, max_tiles2;
@@ -1224,8 +1270,9 @@ uint64_t place_chunks(uint32_t T, uint64_t P) {
 GroupedWs grouped_ws(uint32_t T, uint64_t P, uint32_t E, uint32_t hidden, uint32_t inter, uint32_t tx) {
   GroupedWs w;
   const uint32_t tt1 = tile_tokens(T, tx), tt2 = tile_tokens(T, 3);
-  w.max_tiles1 = (uint32_t)(P / tt1 + E + 1);
-  w.max_tiles2 = (uint32_t)(P / tt2 + E + 1);
+  // (room for a round of wide tiles split in two, see split_wide)
+  w.max_tiles1 = (uint32_t)(P / tt1 + E + 1) + kSplitRoom;
+  w.max_tiles2 = (uint32_t)(P / tt2 + E + 1) + kSplitRoom;
   uint64_t o = 0;
   w.hdr = o; o += a256(sizeof(GroupedHdr));
   w.offsets = o; o += a256(4ull * (AFFX_MAX_EXPERTS + 1));
@@ -1310,8 +1357,14 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
                      (uint32_t*)(b + lay.zeros), zmax / 4);
   int rc = check_launch("grouped_prep_x_kernel");
   if (rc) return rc;
+  // the GEMMs' grid: one workgroup per CU, a multiple of the 8 XCDs (the light class: two)
+  int dev = 0, cus = 0;
+  if ((rc = check_hip(hipGetDevice(&dev), "hipGetDevice"))) return rc;
+  if ((rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
+    return rc;
+  const uint32_t gmax = cus >= 8 ? (uint32_t)cus / 8u * 8u : 8u;
   const PlanOut po{(GroupedHdr*)(b + lay.hdr), (uint32_t*)(b + lay.offsets), (Tile*)(b + lay.tiles1),
-                   (Tile*)(b + lay.tiles2), lay.max_tiles1, lay.max_tiles2};
+                   (Tile*)(b + lay.tiles2), lay.max_tiles1, lay.max_tiles2, L->inter / 128, L->hidden / 256, gmax};
   uint32_t* hist = (uint32_t*)(b + lay.hist);
   if (sel && Pp <= kSmallPairs) {
     // one workgroup instead of three launches: 7.1 us against 5.4 + 8.2 + 5.0 at 144 pairs, 11.6 against
@@ -1340,12 +1393,7 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   // gate/up: 128 gate + 128 up rows per item; down: 256 rows. Items (row block, tile), the tile
   // count rounded up to a multiple of the 8 XCDs (see the kernel's order), run by a persistent
   // grid of one workgroup per CU (a multiple of 8), or fewer when there are fewer items
-  int dev = 0, cus = 0;
-  if ((rc = check_hip(hipGetDevice(&dev), "hipGetDevice"))) return rc;
-  if ((rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
-    return rc;
-  const uint32_t gmax = cus >= 8 ? (uint32_t)cus / 8u * 8u : 8u;
-  // (the classes below the widest: at most one tile per expert)
+  // (the classes below the widest: at most one tile per expert, and the parts of split wide tiles)
   auto grid = [&](uint32_t row_blocks, uint32_t tiles, uint32_t per_cu) {
     const uint32_t items = row_blocks * ((tiles + 7) / 8 * 8);
     return items < per_cu * gmax ? items : per_cu * gmax;
@@ -1355,7 +1403,7 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   A.b_off = lay.xq;
   auto each_cls = [&](auto ph, auto txc, uint32_t k0, uint32_t row_blocks, uint32_t max_tiles) {
     constexpr int PH = decltype(ph)::value, TX = decltype(txc)::value;
-    const uint32_t part = L->n_experts < max_tiles ? L->n_experts : max_tiles;
+    const uint32_t part = L->n_experts + kSplitRoom < max_tiles ? L->n_experts + kSplitRoom : max_tiles;
     static_for<0, kNCls>([&](auto kc) {
       constexpr int k = decltype(kc)::value, CT = kClsCT[k];
       if ((uint32_t)k < k0) return;
