@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     ent[i] = e;
     const float n = ((e.x * e.x + e.y * e.y) + e.z * e.z) + e.w * e.w;
     half[i] = 0.5f * n;
-    e2max = e2max >= n ? e2max : n;  // (a NaN is kept)
+    e2max = fmaxf(e2max, n < 1e30f ? n : INFINITY);  // (an entry past the bound, or a NaN, leaves no bound)
   }
   for (uint32_t i = tid; i < kQuantChunk * 10 / 128; i += 256) cbits[i] = 0;
   if (tid < kQuantChunk * 6 / 512 + 1) fbits[tid] = 0;
@@ -183,14 +183,13 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   rmax = -wave_min(-rmax);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    const float x = __shfl_xor(e2max, o);
-    e2max = e2max >= x ? e2max : x;
+    e2max = fmaxf(e2max, __shfl_xor(e2max, o));
   }
   if (lane == 0) { red[wv] = rmax; red[4 + wv] = e2max; }
   __syncthreads();
   rmax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 #pragma unroll
-  for (int q = 0; q < 4; ++q) e2max = e2max >= red[4 + q] ? e2max : red[4 + q];
+  for (int q = 0; q < 4; ++q) e2max = fmaxf(e2max, red[4 + q]);
   float rscale = rmax > 0.f ? ldexpf(rmax, -7) : 0.f;
   const uint16_t h = f32_to_bf16_rne(rscale);
   rscale = __uint_as_float((uint32_t)h << 16);
@@ -393,12 +392,18 @@ int affx_quantize_matrix(const void* w, uint32_t rows, uint32_t cols, const void
     return set_error(AFFX_ERR_ARG, "quantize_matrix: cols must be a multiple of 64 and <= %d",
                      kQuantMaxCols);
   const uint32_t chunks = (cols + kQuantChunk - 1) / kQuantChunk;
-  if (rows > 0x7FFFFFFFu / chunks) return set_error(AFFX_ERR_ARG, "quantize_matrix: too many rows");
-  hipLaunchKernelGGL(quantize_rows_kernel, dim3(rows * chunks), dim3(256), 0, (hipStream_t)stream,
-                     (const float*)w, cols, chunks, (const float4*)codebook_f32,
-                     (const float*)importance, (uint8_t*)codes, (uint8_t*)fields,
-                     (uint16_t*)rscales);
-  return check_launch("quantize_rows_kernel");
+  // (a launch holds at most 2^32 threads: a matrix of millions of long rows takes several)
+  const uint32_t slab = (1u << 23) / chunks;
+  for (uint32_t r0 = 0; r0 < rows;) {
+    const uint32_t n = rows - r0 < slab ? rows - r0 : slab;
+    hipLaunchKernelGGL(quantize_rows_kernel, dim3(n * chunks), dim3(256), 0, (hipStream_t)stream,
+                       (const float*)w + (uint64_t)r0 * cols, cols, chunks, (const float4*)codebook_f32,
+                       (const float*)importance, (uint8_t*)codes + (uint64_t)r0 * (cols / 32u * 10u),
+                       (uint8_t*)fields + (uint64_t)r0 * (cols / 64u * 3u), (uint16_t*)rscales + r0);
+    if (int rc = check_launch("quantize_rows_kernel")) return rc;
+    r0 += n;
+  }
+  return AFFX_OK;
 }
 
 // One synthetic expert in container layout: gate/up/down = bf16(0.02 * N(0,1)) with seeds

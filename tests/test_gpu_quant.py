@@ -65,11 +65,11 @@ def test_quantizer_matches_reference_config1(ax, c1_codebook):
 
 
 @pytest.mark.parametrize("rows,cols", [(3, 64), (2, 448), (5, 1088), (2, 8192)])
-@pytest.mark.parametrize("kind", ["normal", "ties", "scales", "importance", "nonfinite"])
+@pytest.mark.parametrize("kind", ["normal", "ties", "scales", "importance", "nonfinite", "codebook"])
 def test_quantizer_edges_match_oracle(ax, orc, c1_codebook, rows, cols, kind):
     """Bit for bit against the oracle where the setting's choice is hard: a codebook whose settings tie
     (its second variant the first one negated, entries repeated), rows from 1e-42 to 1e38 with zero
-    blocks, importances that are zero or negative, infinities and NaN; partial chunks and a whole row of
+    blocks, importances that are zero or negative, infinities and NaN in the rows or the codebook; partial chunks and a whole row of
     8192."""
     rng = np.random.default_rng(rows * cols + len(kind))
     w = (0.02 * rng.standard_normal((rows, cols))).astype(np.float32)
@@ -93,6 +93,8 @@ def test_quantizer_edges_match_oracle(ax, orc, c1_codebook, rows, cols, kind):
         w[0, 7] = np.inf
         w[1, 20] = np.nan
         w[-1, 33] = -np.inf
+    elif kind == "codebook":
+        cb[0, 5], cb[0, 261, 2], cb[1, 900, 0] = 1e10, np.nan, -np.inf
     want = orc.quantize(w, cb.reshape(-1), imp)
     codes, fields, rs = ax.quantize_matrix(torch.from_numpy(w).cuda(), torch.from_numpy(cb).cuda(),
                                            None if imp is None else torch.from_numpy(imp).cuda())
