@@ -145,6 +145,9 @@ __device__ uint32_t search_block(const float4* ent, uint32_t lane, const float* 
 // (E + |t|^2) (E = the largest |e|^2), are within 12u of that, twice it 24u; |t|^2 in f32 within 8u |t|^2;
 // the sums over four quads with their weights (>= 0, else the block is searched in full) within
 // 16u of themselves on either side. The code takes 44u (E + |t|^2) a quad and 64u of the sum.
+// These are relative: a value below the normal range may be off by 2^-126 (2^-149 outside the matrix
+// core) instead. With E > 1e-20 that is nothing beside 44u E, and a block whose weighted bound is not above
+// 1e-30 (importances all but zero) is searched in full.
 constexpr int kQuantMaxCols = 8192;
 constexpr uint32_t kQuantChunk = 1024;
 constexpr float kU = 5.9604645e-8f;
@@ -208,15 +211,12 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     wr[q] = __shfl_xor(wq[q], 32);  // dimension (kg + 2) % 4
     const float a = fabsf(wq[q]);
     bmax = bmax < a ? a : bmax;
-    S[q] = wq[q] * wq[q];
     if (bimp) wt[q] = (((bimp[4 * q] + bimp[4 * q + 1]) + bimp[4 * q + 2]) + bimp[4 * q + 3]) * 0.25f;
   }
 #pragma unroll
   for (int o = 16; o <= 32; o <<= 1) {
     const float a = __shfl_xor(bmax, o);
     bmax = bmax < a ? a : bmax;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) S[q] = S[q] + __shfl_xor(S[q], o);
   }
   const bool need = live && bmax > 0.f && rscale > 0.f;
   int mid = 0;
@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   }
   float inv[3], er[3];
   uint32_t valid = 0;  // settings there are (scale 0..7), as in search_block
-  bool sane = e2max < 1e30f;
+  bool sane = e2max > 1e-20f && e2max < 1e30f;
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int s = mid - 1 + j;
@@ -238,11 +238,25 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     const float bs = rscale * (float)(1u << (in ? s : 0));
     inv[j] = in && need ? 1.0f / bs : 0.f;
     if (in) valid |= 0xF00Fu << (4 * j);
+    sane = sane && (!in || (bs > 1e-30f && bs < 1e30f));
+  }
+  // |t|^2 of the quads at the middle scale, of the scaled targets (the weights' own squares underflow);
+  // four times that at the scale below, a quarter at the one above
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float t = wq[q] * inv[1];
+    S[q] = t * t;
+    S[q] = S[q] + __shfl_xor(S[q], 16);
+    S[q] = S[q] + __shfl_xor(S[q], 32);
+  }
+  constexpr float kT2[3] = {4.f, 1.f, 0.25f};
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
     er[j] = 0.f;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) er[j] = er[j] + wt[q] * (44.f * kU * (e2max + S[q] * inv[j] * inv[j]));
+    for (int q = 0; q < 4; ++q) er[j] = er[j] + wt[q] * (44.f * kU * (e2max + S[q] * kT2[j]));
     er[j] = er[j] * (float)(1u << (2 * j));
-    sane = sane && (!in || (bs > 1e-30f && bs < 1e30f)) && er[j] < 1e30f;
+    sane = sane && (!((valid >> (4 * j)) & 1u) || (er[j] > 1e-30f && er[j] < 1e30f));
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) sane = sane && wt[q] >= 0.f;
@@ -295,7 +309,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
           float e = 0.f;
 #pragma unroll
           for (int q = 0; q < 4; ++q)
-            e = e + wt[q] * (2.f * m[8 * j + 4 * (g >> 1) + q][g & 1] + S[q] * inv[j] * inv[j]);
+            e = e + wt[q] * (2.f * m[8 * j + 4 * (g >> 1) + q][g & 1] + S[q] * kT2[j]);
           e = e * (float)(1u << (2 * j));
           if (v == 0) ea[4 * j + g] = e;
           else ea[12 + 4 * j + g] = e;

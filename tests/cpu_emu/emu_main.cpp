@@ -4,7 +4,10 @@
 //   emu_main decode  hidden inter n_experts M K seed [staged|allpad|dm<nb>] -> rel_l2 of the decode FFN (the
 //                    fused launch, also checked equal to the staged launches; `staged` alone)
 //   emu_main grouped hidden inter n_experts T K seed lo   -> rel_l2 of the grouped FFN
-//   emu_main quant   rows cols seed                       -> planes bit-exact vs the oracle
+//   emu_main quant   rows cols seed [wscale cscale iscale spike] -> planes bit-exact vs the oracle; wscale and
+//                    cscale multiply the weights and the codebook, whose second variant is then the
+//                    first one negated; iscale: column importances of that size (0: none); spike:
+//                    the last weight of each row (0: as drawn)
 //   emu_main dequant hidden inter seed                    -> dequant bit-exact vs the oracle
 //   emu_main slots   hidden inter n_experts T K seed      -> the slot-list grouped entry vs the
 //                    routes entry (bit for bit) and, with a reordered list, vs the oracle
@@ -712,13 +715,26 @@ int run_quant(int argc, char** argv) {
   for (auto& v : w) v = 0.02f * nd(rng);
   for (uint32_t c = 0; c < 16 && c < cols; ++c) w[c] = 0.f;  // an all-zero block
   const auto cb = load_codebook();
-  std::vector<float> cbf(8192);
+  std::vector<float> cbf(8192), imp;
   orc_unpack_codebook(cb.data(), cbf.data());
+  if (argc >= 9) {
+    const float ws = strtof(argv[5], nullptr), cs = strtof(argv[6], nullptr), is = strtof(argv[7], nullptr);
+    const float spike = strtof(argv[8], nullptr);
+    for (auto& v : w) v *= ws;
+    for (uint32_t r = 0; r < rows && spike != 0.f; ++r) w[(r + 1) * cols - 1] = spike;
+    for (uint32_t i = 0; i < 4096; ++i) {
+      cbf[i] *= cs;
+      cbf[4096 + i] = -cbf[i];
+    }
+    if (is != 0.f) imp.resize(cols);
+    for (auto& v : imp) v = is * (0.1f + (float)(rng() % 1000) / 1000.f);
+  }
+  const float* im = imp.empty() ? nullptr : imp.data();
   const uint64_t nc = rows * cols * 10 / 32, nf = rows * cols * 6 / 128;
   std::vector<uint8_t> c1(nc), f1(nf), c2(nc), f2(nf);
   std::vector<uint16_t> r1(rows), r2(rows);
-  int rc = affx_quantize_matrix(w.data(), rows, cols, cbf.data(), nullptr, c1.data(), f1.data(), r1.data(), nullptr);
-  orc_quantize_matrix(w.data(), rows, cols, cbf.data(), nullptr, c2.data(), f2.data(), r2.data());
+  int rc = affx_quantize_matrix(w.data(), rows, cols, cbf.data(), im, c1.data(), f1.data(), r1.data(), nullptr);
+  orc_quantize_matrix(w.data(), rows, cols, cbf.data(), im, c2.data(), f2.data(), r2.data());
   const bool ok = c1 == c2 && f1 == f2 && r1 == r2;
   printf("quant rc=%d exact=%d\n", rc, (int)ok);
   return rc == 0 && ok ? 0 : 1;

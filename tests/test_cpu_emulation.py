@@ -77,6 +77,10 @@ CASES = {
     # serves seven or eight tokens, so each one takes two passes of the compacted column group
     "decode_m8_full": (("decode", 1024, 1024, 3, 8, 3, 7), 3),
     "quant": (("quant", 4, 256, 3), 4),
+    # squares of the weights underflow, entries far below the targets; entries and blocks whose
+    # distances underflow, beside one weight that sets the row's scale
+    "quant_tiny": (("quant", 3, 1024, 5, 1e-24, 1e-5, 0, 0), 4),
+    "quant_tiny_blocks": (("quant", 3, 1024, 5, 1e-21, 1e-21, 0, 1), 4),
     "grouped": (("grouped", 1024, 1024, 5, 12, 3, 4, 1), 4),
     "timeout": (("timeout", 1024, 1024, 6, 2, 3, 8), 4),
     # batch 1 in one pass (6 workgroups hold the 64 gate/up items): per-workgroup publish flags
@@ -96,7 +100,7 @@ CASES = {
 }
 # longest first, so the three lanes finish together
 ORDER = ["decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "slots", "shared", "decode_m1_single", "grouped",
-         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "timeout", "timeout_m1", "route", "gemv", "w8a8", "steps", "decode_allpad",
+         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "timeout", "timeout_m1", "route", "gemv", "w8a8", "steps", "decode_allpad",
          "dequant"]
 
 
@@ -160,6 +164,11 @@ def test_decode_emulated_m8_two_passes(runs):
 
 def test_quantizer_emulated(runs):
     assert "exact=1" in result(runs, "quant")
+
+
+@pytest.mark.parametrize("case", ["quant_tiny", "quant_tiny_blocks"])
+def test_quantizer_emulated_underflow(runs, case):
+    assert "exact=1" in result(runs, case)
 
 
 def test_grouped_emulated(runs):

@@ -101,3 +101,29 @@ def test_quantizer_edges_match_oracle(ax, orc, c1_codebook, rows, cols, kind):
     np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
     np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
     np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
+
+
+@pytest.mark.parametrize("tied", [False, True])
+@pytest.mark.parametrize("wscale,cscale,iscale,spike", [
+    (1e-20, 1e-5, 0, 0), (1e-22, 1e-3, 0, 0), (1e-24, 1e-5, 0, 0), (1e-26, 1e-5, 0, 0), (1e-28, 1.0, 0, 0),
+    (1.0, 0.0039, 0, 0), (1e-21, 1e-21, 0, 1), (1e-19, 1e-19, 0, 1), (1.0, 1e-12, 0, 0), (1.0, 1.0, 1e-40, 0),
+    (1.0, 1.0, 1e-28, 0), (1.0, 1.0, 1e12, 0)])
+def test_quantizer_underflow_matches_oracle(ax, orc, c1_codebook, wscale, cscale, iscale, spike, tied):
+    """Bit for bit against the oracle where squares, distances or weighted sums underflow: rows and
+    codebooks scaled down together and apart (tied: the second variant the first one negated),
+    blocks far below the row's scale (spike: its last weight), importances near zero."""
+    rng = np.random.default_rng(77)
+    rows, cols = 24, 1024
+    w = (np.float32(wscale) * (0.02 * rng.standard_normal((rows, cols)))).astype(np.float32)
+    if spike:
+        w[:, -1] = spike
+    cb = (ax.codebook_floats(c1_codebook) * np.float32(cscale)).astype(np.float32)
+    if tied:
+        cb[1] = -cb[0]
+    imp = (np.float32(iscale) * rng.uniform(0.1, 1.1, cols)).astype(np.float32) if iscale else None
+    want = orc.quantize(w, cb.reshape(-1), imp)
+    codes, fields, rs = ax.quantize_matrix(torch.from_numpy(w).cuda(), torch.from_numpy(cb).cuda(),
+                                           None if imp is None else torch.from_numpy(imp).cuda())
+    np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
+    np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
+    np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
