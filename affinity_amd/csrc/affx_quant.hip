@@ -85,6 +85,25 @@ __device__ __forceinline__ float quad_min(const float4* __restrict__ ent, uint32
   return wave_min(m);
 }
 
+// The scan's code of one quad: the lowest index among equal minima (wave-uniform result).
+__device__ __forceinline__ uint32_t quad_argmin(const float4* __restrict__ ent, uint32_t lane, float t0, float t1,
+                                                float t2, float t3) {
+  float m = 3.402823466e38f;
+  uint32_t bi = 0xFFFFFFFFu;
+#pragma unroll 4
+  for (int j = 0; j < 16; ++j) {
+    const float s = qdist(ent[lane + 64 * j], t0, t1, t2, t3);
+    if (s < m) { m = s; bi = lane + 64u * j; }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(m, o);
+    const uint32_t oi = __shfl_xor(bi, o);
+    if (ov < m || (ov == m && oi < bi)) { m = ov; bi = oi; }
+  }
+  return bi == 0xFFFFFFFFu ? 0u : bi;  // nothing below FLT_MAX: the scan's default, code 0
+}
+
 // The reference's setting search of one block (blockquant.cpp:706-762) among the settings of `open`
 // (bit 12 v + 4 j + g: variant v, scale mid - 1 + j, g: bit 0 sign, bit 1 rotation), all lanes of
 // the wave on one block: the first strict minimum in the order v, scale, g.
@@ -150,9 +169,19 @@ __device__ uint32_t search_block(const float4* ent, uint32_t lane, const float* 
 // 1e-30 (importances all but zero) is searched in full.
 constexpr int kQuantMaxCols = 8192;
 constexpr uint32_t kQuantChunk = 1024;
+// A chunk of 64 columns (four blocks of a product's 16 columns, and one wave of the four) is searched in
+// full: rows of 64 columns, 512 of them 186 us by products and 85 so, 2048 of them 521 and 267; of 128
+// columns 154 by products and 192 so, 521 and 518.
+constexpr uint32_t kShort = 4;
 constexpr float kU = 5.9604645e-8f;
 typedef float qv4f __attribute__((ext_vector_type(4)));
 
+// Code i of a chunk into its stream (zeroed; the codes' bits are disjoint).
+__device__ __forceinline__ void put_code(uint32_t* cbits, uint32_t i, uint32_t code) {
+  const uint32_t at = i * 10;
+  atomicOr(&cbits[at >> 5], code << (at & 31));
+  if ((at & 31) > 22) atomicOr(&cbits[(at >> 5) + 1], code >> (32 - (at & 31)));
+}
 __device__ __forceinline__ float low_of(float a, float b) { return __builtin_fminf(a, b); }
 
 __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
@@ -166,6 +195,8 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   __shared__ uint32_t cbits[kQuantChunk * 10 / 128];            // the chunk's code stream
   __shared__ uint32_t fbits[kQuantChunk * 6 / 512 + 1];         // the chunk's field stream
   __shared__ float red[8];
+  __shared__ uint2 todo[kQuantChunk / kBlock];                  // blocks left open: block | middle scale << 8, open settings
+  __shared__ uint32_t n_todo, field_s[kQuantChunk / kBlock];
   float e2max = 0.f;
   for (uint32_t i = tid; i < kVariants * kLut; i += 256) {
     const float4 e = cb[i];
@@ -176,6 +207,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   }
   for (uint32_t i = tid; i < kQuantChunk * 10 / 128; i += 256) cbits[i] = 0;
   if (tid < kQuantChunk * 6 / 512 + 1) fbits[tid] = 0;
+  if (tid == 0) n_todo = 0;
 
   const float* row = w + (uint64_t)r * cols;
   float rmax = 0.f;
@@ -230,7 +262,8 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   }
   float inv[3], er[3];
   uint32_t valid = 0;  // settings there are (scale 0..7), as in search_block
-  bool sane = e2max > 1e-20f && e2max < 1e30f;
+  const bool direct = nblk <= kShort;
+  bool sane = !direct && e2max > 1e-20f && e2max < 1e30f;
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int s = mid - 1 + j;
@@ -329,16 +362,32 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     const uint32_t k = (uint32_t)__builtin_ctz(open), j = (k % 12u) / 4u;
     field = ((k / 12u) << 5) | ((k & 3u) << 3) | (uint32_t)(mid - 1 + (int)j);
   }
-  // the blocks left open, one at a time
-  uint64_t todo = __ballot(need && kg == 0u && (open & (open - 1u)) != 0u);
-  while (todo) {
-    const uint32_t src = (uint32_t)__builtin_ctzll(todo);
-    todo &= todo - 1;
-    const uint32_t bb = (16u * wv + src) * kBlock;
-    const uint32_t f = search_block(ent, lane, row + c0 + bb, imp ? imp + c0 + bb : nullptr, rscale,
-                                    __shfl(mid, (int)src), __shfl(open, (int)src));
-    if (c == src) field = f;
+  // the blocks left open (of a short chunk all), a wave each in turn: in any order and of the whole chunk,
+  // so that the waves whose blocks are decided, or which have none, share the work (512 x 512 with
+  // negative importances, every block open: 1272 us with each wave at its own blocks, now 741)
+  const bool listed = live && (direct || (need && (open & (open - 1u)) != 0u));
+  if (listed && kg == 0u) todo[atomicAdd(&n_todo, 1u)] = make_uint2(b | ((uint32_t)mid << 8), need ? open : 0u);
+  __syncthreads();
+  for (uint32_t i = wv; i < n_todo; i += 4) {
+    uint2 q = todo[i];
+    q.x = __builtin_amdgcn_readfirstlane(q.x);
+    q.y = __builtin_amdgcn_readfirstlane(q.y);
+    const uint32_t bq = q.x & 255u, at = c0 + bq * kBlock;
+    const uint32_t f = search_block(ent, lane, row + at, imp ? imp + at : nullptr, rscale, (int)(q.x >> 8), q.y);
+    if (lane == 0) field_s[bq] = f;
+    const float mag = rscale * (float)(1u << (f & 7u)), bs = (f & 8u) ? -mag : mag;
+    if (!direct || !(mag > 0.f)) continue;
+    // (a short chunk's codes too: the scan below would have most lanes idle)
+    const uint32_t rh = (f & 16u) ? 2u : 0u;
+#pragma unroll
+    for (uint32_t p = 0; p < 4; ++p) {
+      const float* x = row + at + 4 * p;
+      const uint32_t code = quad_argmin(ent + (f >> 5) * kLut, lane, x[rh] / bs, x[1 + rh] / bs, x[2 - rh] / bs, x[3 - rh] / bs);
+      if (lane == 0) put_code(cbits, bq * 4 + p, code);
+    }
   }
+  __syncthreads();
+  if (listed) field = field_s[b];
 
   // ---- the codes: lane (c, kg) takes quad kg of block c --------------------------------------------
   if (live) {
@@ -346,7 +395,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     const float bs = (field & 8u) ? -mag : mag;
     const bool rot = (field & 16u) != 0u;
     uint32_t code = 0;
-    if (mag > 0.f) {
+    if (mag > 0.f && !direct) {
       float x[4];
 #pragma unroll
       for (int p = 0; p < 4; ++p) x[p] = blk[4 * kg + p];
@@ -365,9 +414,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
       atomicOr(&fbits[fpos >> 5], field << (fpos & 31));
       if ((fpos & 31) > 26) atomicOr(&fbits[(fpos >> 5) + 1], field >> (32 - (fpos & 31)));
     }
-    const uint32_t cpos = (b * 4 + kg) * 10;
-    atomicOr(&cbits[cpos >> 5], code << (cpos & 31));
-    if ((cpos & 31) > 22) atomicOr(&cbits[(cpos >> 5) + 1], code >> (32 - (cpos & 31)));
+    if (!direct) put_code(cbits, b * 4 + kg, code);
   }
   __syncthreads();
   // 64 columns are whole bytes of both streams (20 and 3), and cols % 64 == 0

@@ -81,6 +81,8 @@ CASES = {
     # distances underflow, beside one weight that sets the row's scale
     "quant_tiny": (("quant", 3, 1024, 5, 1e-24, 1e-5, 0, 0), 4),
     "quant_tiny_blocks": (("quant", 3, 1024, 5, 1e-21, 1e-21, 0, 1), 4),
+    # a chunk of 1024 columns and one of 64, whose four blocks are searched in full
+    "quant_short": (("quant", 2, 1088, 6), 4),
     "grouped": (("grouped", 1024, 1024, 5, 12, 3, 4, 1), 4),
     "timeout": (("timeout", 1024, 1024, 6, 2, 3, 8), 4),
     # batch 1 in one pass (6 workgroups hold the 64 gate/up items): per-workgroup publish flags
@@ -100,7 +102,7 @@ CASES = {
 }
 # longest first, so the three lanes finish together
 ORDER = ["decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "slots", "shared", "decode_m1_single", "grouped",
-         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "timeout", "timeout_m1", "route", "gemv", "w8a8", "steps", "decode_allpad",
+         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "timeout", "timeout_m1", "route", "gemv", "w8a8", "steps", "decode_allpad",
          "dequant"]
 
 
@@ -166,8 +168,8 @@ def test_quantizer_emulated(runs):
     assert "exact=1" in result(runs, "quant")
 
 
-@pytest.mark.parametrize("case", ["quant_tiny", "quant_tiny_blocks"])
-def test_quantizer_emulated_underflow(runs, case):
+@pytest.mark.parametrize("case", ["quant_tiny", "quant_tiny_blocks", "quant_short"])
+def test_quantizer_emulated_edges(runs, case):
     assert "exact=1" in result(runs, case)
 
 

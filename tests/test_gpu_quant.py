@@ -127,3 +127,22 @@ def test_quantizer_underflow_matches_oracle(ax, orc, c1_codebook, wscale, cscale
     np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
     np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
     np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
+
+
+@pytest.mark.parametrize("cols", [64, 128, 512, 1088])
+def test_quantizer_open_blocks_match_oracle(ax, orc, c1_codebook, cols):
+    """Every block left to the full search, shared among a workgroup's waves: importances below zero,
+    all zero, and (with importances) blocks of zeros between; rows of one short chunk."""
+    rng = np.random.default_rng(cols)
+    rows = 12
+    w = (0.02 * rng.standard_normal((rows, cols))).astype(np.float32)
+    w[1, 16:32] = 0
+    w[2] = 0
+    cb = ax.codebook_floats(c1_codebook)
+    gw, gc = torch.from_numpy(w).cuda(), torch.from_numpy(cb).cuda()
+    for imp in (rng.uniform(-1.0, 0.2, cols).astype(np.float32), np.zeros(cols, np.float32)):
+        want = orc.quantize(w, cb.reshape(-1), imp)
+        codes, fields, rs = ax.quantize_matrix(gw, gc, torch.from_numpy(imp).cuda())
+        np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
+        np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
+        np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
