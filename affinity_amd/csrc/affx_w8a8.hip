@@ -18,7 +18,8 @@
 // quad of tokens, its B zero outside the group: four times the MFMAs, and a fold through DPP quad
 // broadcasts: 256 tokens' steps over 256 experts 1092 us, now 672.)
 //
-// An item is 128 rows by at most 16 tokens (one MFMA column tile) of a tile, eight waves: most tiles of
+// An item is 128 rows (64 where the launch has few) by at most 16 tokens (one MFMA column tile) of a
+// tile, a wave for 16 rows: most tiles of
 // a batch of a few hundred tokens over 256 experts have no more, and the weights' stream and the
 // decode are the bound, so a persistent workgroup requests its next column tile's or next item's
 // weights and token rows before it decodes the current ones, two workgroups (16 waves) a CU. A tile
@@ -30,8 +31,7 @@
 
 namespace affx {
 
-constexpr int kW8Waves = 8;
-constexpr int kW8T = kW8Waves * 64;
+constexpr int kW8Waves = 8;           // waves of a workgroup (half of them in launches of few items)
 constexpr int kW8KC = 2;              // codebook copies
 constexpr uint32_t kW8MaxTok = 64;    // the reference's kExpertWmmaTok (expert_kernel_hip.h:195)
 constexpr uint32_t kW8Row = kTileCols + 16u;  // LDS bytes of one staged token row (padded)
@@ -122,7 +122,7 @@ __device__ __forceinline__ void w8_store(const W8a8Args& A, void* y, uint32_t ld
   }
 }
 
-// An item: eight row tiles (one a wave) of a tile's tokens j0 .. j0 + n - 1.
+// An item: NW row tiles (one a wave) of a tile's tokens j0 .. j0 + n - 1.
 struct W8Item {
   const uint8_t* codes;
   const uint8_t* fields;
@@ -137,15 +137,41 @@ constexpr uint32_t kW8Cols = 16;
 struct W8Order {
   uint32_t nrb, nch, items;
 };
-// The first item in use from round r on (advanced); false past the last.
+// (the lane is counted where it is used: lane values held across the steps were spilled, and a
+// reload, a vector memory load, waits for every load in flight)
+__device__ __forceinline__ uint32_t w8_lane() {
+  uint32_t z = 0u;
+  AFFX_PIN(z);
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
+}
+// The first item in use from round r on (advanced); false past the last. Four rounds (a tile's token groups) are looked at by
+// scalar loads, from there 64 at a time, a lane each: a list of mostly pads has hundreds of rounds without
+// an item (4096 pads, 2048 rows: 282 us by scalar loads alone, now 7.4).
+template <int NW>
 __device__ __forceinline__ bool w8_seek(const W8a8Args& A, const W8Order& o, uint32_t& r, uint32_t wv, W8Item& I) {
-  for (; (uint64_t)r * gridDim.x < o.items; ++r) {
-    const uint32_t it = r * gridDim.x + (blockIdx.x + r) % gridDim.x;
-    if (it >= o.items) continue;
-    const uint32_t q = it / o.nch, j0 = (it - q * o.nch) * kW8Cols, tile = q / o.nrb;
-    const uint32_t nt = w8_tokens(A.tiles, tile, A.cap);
-    if (j0 >= nt) continue;
+  for (uint32_t tries = 0; (uint64_t)r * gridDim.x < o.items; ++tries) {
+    if (tries >= 4u) {
+      const uint32_t rl = r + w8_lane(), il = rl * gridDim.x + (blockIdx.x + rl) % gridDim.x;
+      bool used = il < o.items;
+      if (used) {
+        const uint32_t ql = il / o.nch;
+        used = (il - ql * o.nch) * kW8Cols < min(A.tiles[ql / o.nrb].nt, A.cap);
+      }
+      const uint64_t m = __ballot(used);
+      if (m == 0u) {
+        r += 64u;
+        continue;
+      }
+      r += (uint32_t)__builtin_ctzll(m);
+    }
     r = __builtin_amdgcn_readfirstlane(r);
+    const uint32_t it = r * gridDim.x + (blockIdx.x + r) % gridDim.x;
+    const uint32_t q = it / o.nch, j0 = (it - q * o.nch) * kW8Cols, tile = q / o.nrb;
+    const uint32_t nt = it < o.items ? w8_tokens(A.tiles, tile, A.cap) : 0u;
+    if (j0 >= nt) {
+      ++r;
+      continue;
+    }
     I.tile = __builtin_amdgcn_readfirstlane(tile);
     I.j0 = __builtin_amdgcn_readfirstlane(j0);
     const affx_expert_tile* T = A.tiles + I.tile;
@@ -153,7 +179,7 @@ __device__ __forceinline__ bool w8_seek(const W8a8Args& A, const W8Order& o, uin
     I.fields = reinterpret_cast<const uint8_t*>(*AFFX_CONST_PTR(uint64_t, &T->fields));
     I.tok = reinterpret_cast<const uint32_t*>(*AFFX_CONST_PTR(uint64_t, &T->tok));
     I.n = __builtin_amdgcn_readfirstlane(min(nt - j0, kW8Cols));
-    I.rt = __builtin_amdgcn_readfirstlane((q - tile * o.nrb) * kW8Waves + wv);
+    I.rt = __builtin_amdgcn_readfirstlane((q - tile * o.nrb) * NW + wv);
     return true;
   }
   return false;
@@ -179,19 +205,13 @@ __device__ __forceinline__ void w8_stage(const W8a8Args& A, const W8Item& I, uin
   const __amdgpu_buffer_rsrc_t q = buffer_rsrc(A.xs + (uint64_t)t * (A.cols / 128u) + ct * 8u, 32u);
   if (lane < 8u) __builtin_amdgcn_raw_ptr_buffer_load_lds(q, AFFX_LDS_PTR(sc), 4, lane * 4u, 0, 0, 0);
 }
-// (the lane is counted where it is used: lane values held across the steps were spilled, and a
-// reload, a vector memory load, waits for every load in flight)
-__device__ __forceinline__ uint32_t w8_lane() {
-  uint32_t z = 0u;
-  AFFX_PIN(z);
-  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
-}
-
 // LDS: the codebook and two buffers of a column tile's token rows and scales, so two workgroups a CU (at
 // most 128 registers a wave). The steps of a workgroup are (item, column tile) pairs in order; each
 // step first requests the next step's unit and token rows, then decodes and multiplies its own, and
 // ends in one barrier.
-__global__ void __launch_bounds__(kW8T, 4) w8a8_gemm_kernel(W8a8Args A) {
+template <int NW>
+__global__ void __launch_bounds__(NW * 64, NW / 2) w8a8_gemm_kernel(W8a8Args A) {
+  constexpr int kW8T = NW * 64;
   __shared__ __align__(16) uint32_t lut_s[Lut<kW8KC, true>::kDwords];
   // (two arrays a kind: the compiler can tell the buffer being read from the one being written)
   __shared__ __align__(16) uint8_t xb0[kW8Cols * kW8Row], xb1[kW8Cols * kW8Row];
@@ -200,13 +220,13 @@ __global__ void __launch_bounds__(kW8T, 4) w8a8_gemm_kernel(W8a8Args A) {
   const uint32_t tid = threadIdx.x;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t nct = A.cols / kTileCols, nrt = A.rows / kTileRows;
-  const W8Order o{(nrt + kW8Waves - 1) / kW8Waves, A.cap > kW8Cols ? A.cap / kW8Cols : 1u, A.items};
+  const W8Order o{(nrt + NW - 1) / NW, A.cap > kW8Cols ? A.cap / kW8Cols : 1u, A.items};
   uint32_t r = 0;
   W8Item I;
-  if (!w8_seek(A, o, r, wv, I)) return;  // (the whole workgroup)
+  if (!w8_seek<NW>(A, o, r, wv, I)) return;  // (the whole workgroup)
   auto stage = [&](const W8Item& J, uint32_t ct, uint8_t* xb, float* xs) {
 #pragma unroll
-    for (uint32_t j = wv; j < kW8Cols; j += kW8Waves)
+    for (uint32_t j = wv; j < kW8Cols; j += NW)
       if (j < J.n) w8_stage(A, J, ct, J.j0 + j, w8_lane(), xb + j * kW8Row, xs + j * 8u);
   };
   auto load = [&](Unit& u, const W8Item& J, uint32_t ct) {
@@ -217,10 +237,11 @@ __global__ void __launch_bounds__(kW8T, 4) w8a8_gemm_kernel(W8a8Args A) {
   load(ua, I, 0);
   stage(I, 0, xb0, xs0);
   {
-    uint32_t cbv[4];
+    constexpr int kPer = 2048 / kW8T;
+    uint32_t cbv[kPer];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8T];
-    build_lut<kW8KC, kW8T, 4, true>(lut_s, cbv, tid);
+    for (int i = 0; i < kPer; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8T];
+    build_lut<kW8KC, kW8T, kPer, true>(lut_s, cbv, tid);
   }
   __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(0));
   __syncthreads();
@@ -233,7 +254,7 @@ __global__ void __launch_bounds__(kW8T, 4) w8a8_gemm_kernel(W8a8Args A) {
     const bool last = ct + 1 == nct;
     W8Item N = I;
     bool more = true;
-    if (last) more = w8_seek(A, o, ++r, wv, N);
+    if (last) more = w8_seek<NW>(A, o, ++r, wv, N);
     const bool rows_ok = I.rt < nrt;
     const uint32_t lane = w8_lane(), c = lane & 15, kg = lane >> 4, copy4 = ((lane >> 1) & (kW8KC - 1)) * 4u;
     // (requested here, used after the last column tile's products)
@@ -315,14 +336,21 @@ extern "C" int affx_expert_gemm_w8a8(const affx_expert_tile* tiles, uint32_t n_t
     return rc ? rc : affx_expert_gemm_w8a8(tiles + n_tiles / 2, n_tiles - n_tiles / 2, max_nt, x8, xs, codebook, rows,
                                            cols, wscale, y_bf16, stream);
   }
-  A.items = (uint32_t)items;
   int dev = 0, cus = 0, rc;
   if ((rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) ||
       (rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
     return rc;
+  // A launch of few items is bound by one item's latency: where there is a CU for each half of them, items
+  // of 64 rows (a wave a SIMD: one token, 2048 x 4096, 14.1 us in items of 128 rows, 11.0 so).
+  const uint64_t half = (uint64_t)n_tiles * ((rows / kTileRows + kW8Waves / 2 - 1) / (kW8Waves / 2)) * nch;
+  const bool few = half <= (uint64_t)(cus > 0 ? cus : 1) && half > items;
+  A.items = (uint32_t)(few ? half : items);
   // persistent: as many workgroups as the device holds at once, a multiple of the token groups
   const uint32_t most = 2u * (uint32_t)(cus > 1 ? cus / 2 * 2 : 2);
   const uint32_t grid = A.items < most ? A.items : most;
-  hipLaunchKernelGGL(w8a8_gemm_kernel, dim3(grid), dim3(kW8T), 0, (hipStream_t)stream, A);
+  if (few)
+    hipLaunchKernelGGL((w8a8_gemm_kernel<kW8Waves / 2>), dim3(grid), dim3(kW8Waves * 32), 0, (hipStream_t)stream, A);
+  else
+    hipLaunchKernelGGL((w8a8_gemm_kernel<kW8Waves>), dim3(grid), dim3(kW8Waves * 64), 0, (hipStream_t)stream, A);
   return check_launch("w8a8_gemm_kernel");
 }

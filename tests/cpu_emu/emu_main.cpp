@@ -393,7 +393,8 @@ int run_gemv(int argc, char** argv) {
 
 // The single-matrix W8A8 GEMM against the oracle: one launch of three tiles (each a different
 // expert's down matrix: 64 tokens by identity into a compact block, 13 listed tokens into a strided
-// arena, a pad), then a bf16 launch of 5 tokens; the other columns of the strided arena untouched.
+// arena, a pad), then a bf16 launch of 5 tokens, then a list of mostly pads; the other columns of the
+// strided arena untouched.
 int run_w8a8(int argc, char** argv) {
   const uint32_t hidden = atoi(argv[2]), inter = atoi(argv[3]);
   std::mt19937_64 rng(atoi(argv[4]));
@@ -426,7 +427,14 @@ int run_w8a8(int argc, char** argv) {
   int rc = affx_expert_gemm_w8a8(t3, 3, 64, x8.data(), xs.data(), L.cb.data(), rows, cols, 0.5f, 0, nullptr);
   affx_expert_tile tb = tile(2, tok1.data() + 3, yb.data(), 5, 0);
   if (rc == 0) rc = affx_expert_gemm_w8a8(&tb, 1, 5, x8.data(), xs.data(), L.cb.data(), rows, cols, 0.5f, 1, nullptr);
+  // mostly pads: 13 tokens at entry 130 of 200, five at the last
+  std::vector<affx_expert_tile> tp(200, tile(2, nullptr, nullptr, 0, 0));
+  std::vector<float> p1((size_t)rows * 13), p2((size_t)rows * 5), q2(p2.size());
+  tp[130] = tile(1, tok1.data(), p1.data(), 13, 0);
+  tp[199] = tile(2, tok1.data() + 3, p2.data(), 5, 0);
+  if (rc == 0) rc = affx_expert_gemm_w8a8(tp.data(), 200, 64, x8.data(), xs.data(), L.cb.data(), rows, cols, 0.5f, 0, nullptr);
   oracle(0, nullptr, r0.data(), 64, 0, 0);
+  oracle(2, tok1.data() + 3, q2.data(), 5, 0, 0);
   oracle(1, tok1.data(), r1.data(), 13, ld1, 0);
   oracle(2, tok1.data() + 3, rb.data(), 5, 0, 1);
   // the worst error over each output's scale (its largest magnitude), and the relative L2
@@ -448,6 +456,8 @@ int run_w8a8(int argc, char** argv) {
     emax = std::max(emax, (double)std::fabs(y1[i] - r1[i]));
     rmax = std::max(rmax, (double)std::fabs(r1[i]));
   }
+  for (size_t i = 0; i < p1.size(); ++i) ok = ok && p1[i] == y1[i / 13 * ld1 + i % 13];
+  for (size_t i = 0; i < p2.size(); ++i) emax = std::max(emax, (double)std::fabs(p2[i] - q2[i]));
   const double worst = emax / rmax, l2 = std::sqrt(num / den);
   int bf_off = 0;
   for (size_t i = 0; i < yb.size(); ++i) bf_off = std::max(bf_off, std::abs((int)(int16_t)yb[i] - (int)(int16_t)rb[i]));

@@ -98,11 +98,13 @@ CASES = {
     "steps": (("steps", 256, 40, 3), 4),
     # the single-matrix W8A8 GEMM: three tiles of down matrices (f32, strided arena, pad), one bf16
     "w8a8": (("w8a8", 1024, 1024, 7), 4),
+    # the same with a CU for every item of 64 rows: the launches of few items' form
+    "w8a8_few": (("w8a8", 1024, 1024, 7), 300),
     "shared": (("shared", 1024, 1024, 6, 40, 5), 4),
 }
 # longest first, so the three lanes finish together
 ORDER = ["decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "slots", "shared", "decode_m1_single", "grouped",
-         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "timeout", "timeout_m1", "route", "gemv", "w8a8", "steps", "decode_allpad",
+         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
          "dequant"]
 
 
@@ -213,10 +215,11 @@ def test_gemv_emulated(runs):
     assert "gemv rc=0" in out, out
 
 
-def test_w8a8_gemm_emulated(runs):
+@pytest.mark.parametrize("case", ["w8a8", "w8a8_few"])
+def test_w8a8_gemm_emulated(runs, case):
     """affx_expert_gemm_w8a8 within 1e-5 of the oracle (f32 outputs) and 1 bf16 ulp (bf16 output),
     the strided arena's other columns untouched."""
-    out = result(runs, "w8a8")
+    out = result(runs, case)
     assert "w8a8 rc=0" in out and "others_kept=1" in out, out
 
 

@@ -158,3 +158,44 @@ def test_expert_gemm_w8a8_tile_edges(ax, orc, c1_codebook, rows, cols, max_nt):
         if nt:
             ref = orc.expert_gemm_w8a8(c, f, r, tok, nt, x8, xs, cbf, rows, cols, 0.5, y_bf16=False)
             assert rel_l2(y[:, :nt], ref) <= 2e-4, nt
+
+
+@pytest.mark.parametrize("cols", [1024, 3072])
+@pytest.mark.parametrize("max_nt", [16, 33, 64])
+def test_expert_gemm_w8a8_mostly_pads(ax, orc, c1_codebook, cols, max_nt):
+    """A list of 3000 tiles of which a dozen have tokens (each end, neighbours, and hundreds of pads
+    apart): workgroups of eight waves that pass over whole stretches of it; nine row tiles."""
+    from affinity_amd._lib import AffxExpertTile, check, lib
+    rng = np.random.default_rng(cols + max_nt)
+    rows, n = 144, 3000
+    cbf = orc.unpack_codebook(c1_codebook)
+    x8 = rng.integers(0, 256, (80, cols), dtype=np.uint8)
+    x8[(x8 & 0x7F) == 0x7F] ^= 1
+    xs = rng.uniform(0.01, 2.0, (80, cols // 128)).astype(np.float32)
+    c = rng.integers(0, 256, rows * cols * 10 // 32, dtype=np.uint8)
+    f = rng.integers(0, 256, rows * cols * 6 // 128, dtype=np.uint8)
+    r = (rng.uniform(4e-4, 2e-3, rows).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    dc, df = np.zeros_like(c), np.zeros_like(f)
+    check(lib().affx_matrix_to_device_layout(c.ctypes.data, f.ctypes.data, dc.ctypes.data, df.ctypes.data, rows, cols),
+          "layout")
+    d = [torch.from_numpy(a).cuda() for a in (dc, df, r.view(np.int16))]
+    at = [0, 1, 255, 256, 257, 700, 1023, 1024, 1777, 2500, 2998, 2999]
+    counts = [int(v) for v in rng.integers(1, max_nt + 1, len(at))]
+    counts[0], counts[-1] = max_nt, 1
+    tok = [rng.integers(0, 80, nt).astype(np.uint32) for nt in counts]
+    td = [torch.from_numpy(t.view(np.int32)).cuda() for t in tok]
+    ys = [torch.full((rows, 70), 7.0, device="cuda") for _ in at]
+    tiles = (AffxExpertTile * n)()
+    for q, nt, t, y in zip(at, counts, td, ys):
+        tiles[q] = AffxExpertTile(d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), t.data_ptr(), y.data_ptr(), nt, 70)
+    g = torch.from_numpy(np.frombuffer(bytes(tiles), np.uint8).copy()).cuda()
+    gx, gs = torch.from_numpy(x8).cuda(), torch.from_numpy(xs).cuda()
+    cb = torch.from_numpy(c1_codebook.view(np.int32)).cuda()
+    check(lib().affx_expert_gemm_w8a8(g.data_ptr(), n, max_nt, gx.data_ptr(), gs.data_ptr(), cb.data_ptr(), rows, cols,
+                                      0.5, 0, None), "gemm_w8a8")
+    torch.cuda.synchronize()
+    for nt, t, y in zip(counts, tok, ys):
+        y = y.cpu().numpy()
+        assert (y[:, nt:] == 7.0).all()
+        ref = orc.expert_gemm_w8a8(c, f, r, t, nt, x8, xs, cbf, rows, cols, 0.5, y_bf16=False)
+        assert rel_l2(y[:, :nt], ref) <= 2e-4, nt
