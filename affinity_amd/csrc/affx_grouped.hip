@@ -116,27 +116,44 @@ __device__ __forceinline__ uint32_t n_cls_of(uint32_t c, uint32_t tt, uint32_t t
   const uint32_t r = c % tt;
   return (k == k0 ? c / tt : 0u) + (r != 0u && tile_cls(r, tpg) == k ? 1u : 0u);
 }
-// The wide tiles that are split into a class 1 and a class 2 tile each (12 column tiles = 8 + 4). A class
-// runs in rounds of a tile's row blocks over the grid (the tiles dealt to the 8 XCDs in turn), so a
-// few tiles past a whole round cost a round in which most of the device idles: 194 wide gate/up
-// tiles over 256 workgroups took 13 rounds for 12.1 rounds' work. They are split where the round saved
-// is worth more than those that the narrower classes grow by; cost: an item's time in each
-// class (gate/up with two terms 49, 36 and 26 us; the other forms' ratios are within a tenth).
+// A class runs in rounds of a tile's row blocks over the grid (the tiles dealt to the 8 XCDs in turn), so a
+// few tiles past a whole round cost a round in which most of the device idles, and a class with any
+// tile costs its launch's start (kClsStart more than an empty launch). kClsCost: a round of a class (256
+// items; the light class's two halves of 512), by kernel trace at 1 to 8 rounds: gate/up with two terms
+// 47, 34, 26 and 21 us, with three 49, 36, 26.5 and 21, down 25, 18.5, 13.4 and 11 (hidden 4096, inter
+// 2048); at 2048 and 1024 27, 20, 15 and 12, and 28, 21, 15 and 12, and down 19, 15, 11.5 and 8.7: the
+// same ratios within a seventh. A launch's first round takes 8 to 10 us more, an empty launch 2 to 5.
+constexpr uint32_t kClsCost[kNCls] = {49, 36, 26, 21}, kClsStart = 5;
+__device__ __forceinline__ uint32_t cls_rounds(uint32_t tiles, uint32_t nrb, uint32_t grid) {
+  return ((tiles + 7u) / 8u * 8u * nrb + grid - 1u) / grid;
+}
+// The wide tiles that are split into a class 1 and a class 2 tile each (12 column tiles = 8 + 4): 194 wide
+// gate/up tiles over 256 workgroups took 13 rounds for 12.1 rounds' work. They are split where the
+// round saved is worth more than those that the narrower classes grow by.
 __device__ __forceinline__ uint32_t split_wide(const uint32_t (&n)[kNCls], uint32_t nrb, uint32_t grid, uint32_t room) {
   static_assert(kClsCT[0] == kClsCT[1] + kClsCT[2], "a wide tile is one of each");
-  constexpr uint32_t cost[3] = {49, 36, 26};
-  auto rounds = [&](uint32_t t) { return ((t + 7u) / 8u * 8u * nrb + grid - 1u) / grid; };
+  auto rounds = [&](uint32_t t) { return cls_rounds(t, nrb, grid); };
   const uint32_t r = rounds(n[0]);
   if (r == 0) return 0u;
   const uint32_t left = n[0] - min(n[0], (r - 1u) * grid / nrb / 8u * 8u);
   if (left > room) return 0u;
-  const uint32_t more = (rounds(n[1] + left) - rounds(n[1])) * cost[1] + (rounds(n[2] + left) - rounds(n[2])) * cost[2];
-  return more < cost[0] ? left : 0u;
+  const uint32_t more =
+      (rounds(n[1] + left) - rounds(n[1])) * kClsCost[1] + (rounds(n[2] + left) - rounds(n[2])) * kClsCost[2];
+  return more < kClsCost[0] ? left : 0u;
+}
+// Whether the light tiles run in the class before them (n2 tiles) instead: where the rounds they add there
+// cost less than theirs here, as with the few experts of a small layer, whose tiles of both classes
+// fill a round together (8 experts, two of them a token, 64 tokens: the layer 83 us with two launches a
+// GEMM, 61 with one).
+__device__ __forceinline__ bool merge_light(uint32_t n2, uint32_t n3, uint32_t nrb, uint32_t grid) {
+  auto cost = [&](uint32_t n, uint32_t c) { return n ? cls_rounds(n, nrb, grid) * c + kClsStart : 0u; };
+  return n3 != 0u && cost(n2 + n3, kClsCost[2]) < cost(n2, kClsCost[2]) + cost(n3, kClsCost[3]);
 }
 // One GEMM's tiles: class k's n[k] tiles from tiles[base[k]]; the wide ones from index keep on are split,
-// their parts following the other tiles of classes 1 and 2.
+// their parts following the other tiles of classes 1 and 2; the light tiles follow class 2's, to which
+// they belong if merged (cls[k]: what class k runs).
 struct TileSet {
-  uint32_t base[kNCls], n[kNCls], keep;
+  uint32_t base[kNCls], n[kNCls], keep, cls[kNCls];
 };
 __device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, uint32_t nrb, uint32_t grid,
                                             uint32_t max_tiles) {
@@ -154,6 +171,13 @@ __device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, ui
   t.base[2] = t.base[1] + t.n[1] + split;
 #pragma unroll
   for (int k = 3; k < kNCls; ++k) t.base[k] = t.base[k - 1] + t.n[k - 1] + (k == 3 ? split : 0u);
+#pragma unroll
+  for (int k = 0; k < kNCls; ++k) t.cls[k] = k == 0 ? t.keep : t.n[k] + (k <= 2 ? split : 0u);
+  static_assert(kNCls == 4, "the light class is the one after class 2");
+  if (k0 <= 2 && merge_light(t.cls[2], t.cls[3], nrb, grid)) {
+    t.cls[2] += t.cls[3];
+    t.cls[3] = 0u;
+  }
   return t;
 }
 // Writes the tiles of one expert (slots b0 .. b0 + c - 1), whose first of class k is the class's at[k]-th:
@@ -226,9 +250,8 @@ __device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own
     o.hdr->n_slots = own_slots ? n_slots_in : tot[0];
 #pragma unroll
     for (int k = 0; k < kNCls; ++k) {
-      const uint32_t s1 = t1.n[0] - t1.keep, s2 = t2.n[0] - t2.keep;
-      o.hdr->n_cls[0][k] = fits ? (k == 0 ? t1.keep : t1.n[k] + (k <= 2 ? s1 : 0u)) : 0u;
-      o.hdr->n_cls[1][k] = fits ? (k == 0 ? t2.keep : t2.n[k] + (k <= 2 ? s2 : 0u)) : 0u;
+      o.hdr->n_cls[0][k] = fits ? t1.cls[k] : 0u;
+      o.hdr->n_cls[1][k] = fits ? t2.cls[k] : 0u;
     }
     o.hdr->tx = tx;
     o.hdr->bad = fits ? 0u : 1u;
@@ -1248,17 +1271,29 @@ struct GroupedWs {
   uint32_t max_tiles1, max_tiles2;
 };
 
-// The widest class of a batch of T tokens (tokens are `terms` columns each): the narrowest two of whose
-// tiles hold the batch. An expert with more tokens than one tile is cut into more of them, of which
-// a batch this small has few (24 tokens over 256 experts: none at uniform routes), and the wider
-// classes, whose launches would find no tile, are not launched (4-5 us each).
-uint32_t widest_cls(uint32_t T, uint32_t terms) {
+// The widest class of a batch of T tokens and P slots over E experts (a token is `terms` columns): of those
+// two of whose tiles hold the batch, the one whose rounds cost least if every expert has the mean's
+// tokens. An expert with more tokens than one tile is cut into more of them, each of which decodes
+// its weights again; a batch this small has few such (24 tokens over 256 experts: none at uniform
+// routes), so that is the narrowest, and the wider classes, whose launches would find no tile, are
+// not launched (4-5 us each). Where most experts would be cut it is the narrowest only if the device has
+// room for the tiles (32 tokens that all take 8 experts: 63 us in two light tiles each, 69 in one of
+// four columns; all 16 experts: 100 and 79).
+uint32_t widest_cls(uint32_t T, uint64_t P, uint32_t E, uint32_t terms, uint32_t nrb, uint32_t grid) {
   uint32_t k = 0;
-  for (int q = 1; q < kNCls; ++q)
-    if (T <= 2u * (uint32_t)kClsCT[q] * (16 / terms)) k = (uint32_t)q;
+  uint64_t least = ~0ull;
+  for (int q = 0; q < kNCls; ++q) {
+    const uint64_t cap = (uint64_t)kClsCT[q] * (16 / terms);
+    if (q > 0 && T > 2u * cap) break;
+    const uint64_t tiles = (P + E * cap - 1) / (E * cap) * E;
+    const uint64_t cost = ((tiles + 7) / 8 * 8 * nrb + grid - 1) / grid * kClsCost[q];
+    if (cost <= least) {
+      least = cost;
+      k = (uint32_t)q;
+    }
+  }
   return k;
 }
-uint32_t tile_tokens(uint32_t T, uint32_t terms) { return cls_ct(widest_cls(T, terms)) * (16 / terms); }
 
 // chunks of the routes form's placement: they cover the routes and the run entries 0 .. T
 uint64_t place_chunks(uint32_t T, uint64_t P) {
@@ -1269,8 +1304,9 @@ uint64_t place_chunks(uint32_t T, uint64_t P) {
 // T tokens, room for P slots (the routes form: T * top_k)
 GroupedWs grouped_ws(uint32_t T, uint64_t P, uint32_t E, uint32_t hidden, uint32_t inter, uint32_t tx) {
   GroupedWs w;
-  const uint32_t tt1 = tile_tokens(T, tx), tt2 = tile_tokens(T, 3);
-  // (room for a round of wide tiles split in two, see split_wide)
+  // tiles of the narrowest class (which class a batch's full tiles are of depends on its T, P and E, and a
+  // workspace serves every batch of no more slots), and a round of wide tiles split in two
+  const uint32_t tt1 = (uint32_t)kClsCT[kNCls - 1] * (16 / tx), tt2 = (uint32_t)kClsCT[kNCls - 1] * (16 / 3);
   w.max_tiles1 = (uint32_t)(P / tt1 + E + 1) + kSplitRoom;
   w.max_tiles2 = (uint32_t)(P / tt2 + E + 1) + kSplitRoom;
   uint64_t o = 0;
@@ -1281,14 +1317,16 @@ GroupedWs grouped_ws(uint32_t T, uint64_t P, uint32_t E, uint32_t hidden, uint32
   w.slot_w = o; o += a256(4 * P);
   w.ord = o; o += a256(4 * P);
   w.hist = o; o += a256(4ull * place_chunks(T, P) * E);
-  w.tiles1 = o; o += a256(sizeof(Tile) * w.max_tiles1);
-  w.tiles2 = o; o += a256(sizeof(Tile) * w.max_tiles2);
   w.sigma = o; o += a256(4 * P);  // per slot
-  w.tok_sigma = o; o += a256(4ull * T);
   w.zeros = o; o += a256(hidden > inter ? hidden : inter);
   w.xq = o; o += a256((uint64_t)T * tx * hidden);
   w.aq = o; o += a256(P * 3 * inter);
   w.z = o; o += a256(P * 4 * hidden);
+  // (these last: what comes before the B rows counts towards their 32-bit offsets, and so to the
+  // largest batch accepted)
+  w.tiles1 = o; o += a256(sizeof(Tile) * w.max_tiles1);
+  w.tiles2 = o; o += a256(sizeof(Tile) * w.max_tiles2);
+  w.tok_sigma = o; o += a256(4ull * T);
   w.total = o;
   return w;
 }
@@ -1347,7 +1385,6 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   A.limit = L->swiglu_limit;
   A.sigma_a = 7 - ilogbf(L->swiglu_limit * L->swiglu_limit);
 
-  const uint32_t k01 = widest_cls(T, tx), k02 = widest_cls(T, 3);
   const uint32_t Pp = sel ? T * K : 0u;
   const uint32_t n_sl = (uint32_t)P;  // slot indices are below this (the routes form's taken slots too)
   const uint32_t zmax = L->hidden > L->inter ? L->hidden : L->inter;
@@ -1363,6 +1400,8 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   if ((rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
     return rc;
   const uint32_t gmax = cus >= 8 ? (uint32_t)cus / 8u * 8u : 8u;
+  const uint32_t k01 = widest_cls(T, P, L->n_experts, tx, L->inter / 128, gmax);
+  const uint32_t k02 = widest_cls(T, P, L->n_experts, 3, L->hidden / 256, gmax);
   const PlanOut po{(GroupedHdr*)(b + lay.hdr), (uint32_t*)(b + lay.offsets), (Tile*)(b + lay.tiles1),
                    (Tile*)(b + lay.tiles2), lay.max_tiles1, lay.max_tiles2, L->inter / 128, L->hidden / 256, gmax};
   uint32_t* hist = (uint32_t*)(b + lay.hist);

@@ -3,7 +3,9 @@
 //
 //   emu_main decode  hidden inter n_experts M K seed [staged|allpad|dm<nb>] -> rel_l2 of the decode FFN (the
 //                    fused launch, also checked equal to the staged launches; `staged` alone)
-//   emu_main grouped hidden inter n_experts T K seed lo   -> rel_l2 of the grouped FFN
+//   emu_main grouped hidden inter n_experts T K seed lo [counts] -> rel_l2 of the grouped FFN, the tiles of
+//                    each width class (gate/up, down) and the plan kernels launched; counts "a-b-..":
+//                    the first a tokens' first route names expert 0, and so on, every other route padding
 //   emu_main quant   rows cols seed [wscale cscale iscale spike] -> planes bit-exact vs the oracle; wscale and
 //                    cscale multiply the weights and the codebook, whose second variant is then the
 //                    first one negated; iscale: column importances of that size (0: none); spike:
@@ -229,7 +231,17 @@ int run_grouped(int argc, char** argv) {
     x[i] = lo ? hi + __uint_as_float((uint32_t)xl[i] << 16) : hi;
   }
   routes(rng, T, K, n, sel, w);
-  sel[K] = n + 1;  // a padding id
+  if (argc > 9) {
+    std::fill(sel.begin(), sel.end(), n + 1);
+    uint32_t t = 0, e = 0;
+    for (const char* c = argv[9]; *c; ++e) {
+      char* end;
+      for (uint32_t m = (uint32_t)strtoul(c, &end, 10); m > 0 && t < T; --m, ++t) sel[t * K] = e;
+      c = *end == '-' ? end + 1 : end;
+    }
+  } else {
+    sel[K] = n + 1;  // a padding id
+  }
   affx_layer abi = L.abi();
   const size_t wsb = affx_grouped_workspace_size(T, K, n, hidden, inter);
   std::vector<uint8_t> ws(wsb);
@@ -237,7 +249,12 @@ int run_grouped(int argc, char** argv) {
                                          K, y.data(), 0, ws.data(), wsb, nullptr);
   L.oracle(x.data(), sel.data(), w.data(), T, K, yref.data());
   const double e = rel_l2(y, yref);
-  printf("grouped rc=%d rel_l2=%.3e %s\n", rc, e, affx_last_error());
+  // the workspace starts with the plan's header: slots, terms, a flag, tiles of each class
+  uint32_t h[11];
+  memcpy(h, ws.data(), sizeof(h));
+  printf("grouped rc=%d rel_l2=%.3e classes %u,%u,%u,%u %u,%u,%u,%u small=%d chunks=%d %s\n", rc, e, h[3], h[4], h[5],
+         h[6], h[7], h[8], h[9], h[10], emu_launched()["grouped_plan_small_kernel"],
+         emu_launched()["grouped_place_kernel"], affx_last_error());
   return rc == 0 && e <= 1e-3 ? 0 : 1;
 }
 

@@ -17,6 +17,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <map>
+#include <string>
 #include <thread>
 #include <vector>
 #include <algorithm>
@@ -390,4 +392,10 @@ void emu_launch(F kernel, dim3 grid, dim3 block, size_t shm, Args... args) {
   if (shm) emu_launch_all(kernel, grid, shm, block, args...);
   else emu_launch_seq(kernel, grid, block, args...);
 }
-#define hipLaunchKernelGGL(k, g, b, shm, s, ...) emu_launch(k, dim3(g), dim3(b), (size_t)(shm), __VA_ARGS__)
+// launches by the kernel's name as its launch writes it
+inline std::map<std::string, int>& emu_launched() {
+  static std::map<std::string, int> n;
+  return n;
+}
+#define hipLaunchKernelGGL(k, g, b, shm, s, ...) \
+  (++emu_launched()[#k], emu_launch(k, dim3(g), dim3(b), (size_t)(shm), __VA_ARGS__))

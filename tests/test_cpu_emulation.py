@@ -84,6 +84,8 @@ CASES = {
     # a chunk of 1024 columns and one of 64, whose four blocks are searched in full
     "quant_short": (("quant", 2, 1088, 6), 4),
     "grouped": (("grouped", 1024, 1024, 5, 12, 3, 4, 1), 4),
+    # tokens per expert; a class of its own for the ten tokens' light tiles would cost more than it saves
+    "grouped_merged": (("grouped", 2048, 1024, 2, 40, 1, 7, 0, "30-10"), 8),
     "timeout": (("timeout", 1024, 1024, 6, 2, 3, 8), 4),
     # batch 1 in one pass (6 workgroups hold the 64 gate/up items): per-workgroup publish flags
     "timeout_m1": (("timeout", 1024, 1024, 6, 1, 1, 8), 6),
@@ -104,7 +106,7 @@ CASES = {
 }
 # longest first, so the three lanes finish together
 ORDER = ["decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "slots", "shared", "decode_m1_single", "grouped",
-         "decode_m1", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
+         "decode_m1", "grouped_merged", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
          "dequant"]
 
 
@@ -177,6 +179,17 @@ def test_quantizer_emulated_edges(runs, case):
 
 def test_grouped_emulated(runs):
     assert "rel_l2" in result(runs, "grouped")
+
+
+# tiles of each width class (12, 8, 4 and 2 column tiles), gate/up then down, and the plan's form
+GROUPED = {
+    "grouped_merged": "classes 0,0,2,0 0,0,3,0 small=1 chunks=0",
+}
+
+
+@pytest.mark.parametrize("case", GROUPED)
+def test_grouped_classes_emulated(runs, case):
+    assert GROUPED[case] in result(runs, case)
 
 
 def test_decode_wait_give_up_fails_loudly(runs):

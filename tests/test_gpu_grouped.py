@@ -228,3 +228,36 @@ def test_grouped_tile_class_edges(ax, orc, c1_codebook, layer, counts, lo):
     assert np.isfinite(y).all()
     for i, t in enumerate(pick):
         assert rel_l2(y[t], ref[i]) <= TOL, (t, rel_l2(y[t], ref[i]))
+
+
+@pytest.mark.parametrize("lo", [False, True])
+@pytest.mark.parametrize("E,T,k", [(2, 16, 2), (2, 33, 2), (8, 32, 8), (8, 65, 2), (10, 21, 10), (10, 48, 10), (10, 100, 10)])
+def test_grouped_few_experts(ax, orc, c1_codebook, layer, E, T, k, lo):
+    """Few experts that take most tokens each, so that the widest class of the batch is not the narrowest
+    that could hold it, and light tiles run with the class before: every token's output the same bit for bit
+    as the token's alone, and a dozen against the oracle."""
+    ex, pool, hidden, inter = layer
+    small = ax.ExpertPool(pool.data, pool.codebook, E, hidden, inter)
+    rng = np.random.default_rng(E * T + k + lo)
+    sel, w = _routes(rng, T, k, E)
+    xf = rng.standard_normal((T, hidden)).astype(np.float32)
+    hi = torch.from_numpy(xf).cuda().to(torch.bfloat16)
+    xlo = (torch.from_numpy(xf).cuda() - hi.float()).to(torch.bfloat16) if lo else None
+    gs, gw = torch.from_numpy(sel.view(np.int32)).cuda(), torch.from_numpy(w).cuda()
+    y = ax.expert_ffn_grouped(small, hi, gs, gw, x_lo=xlo)
+    for t in range(T):
+        one = ax.expert_ffn_grouped(small, hi[t:t + 1], gs[t:t + 1], gw[t:t + 1], x_lo=None if xlo is None else xlo[t:t + 1])
+        assert torch.equal(one[0].view(torch.int32), y[t].view(torch.int32)), t
+    xr = (hi.float() + (xlo.float() if lo else 0)).cpu().numpy()
+    pick = rng.permutation(T)[:12]
+    ref = _oracle(orc, ex[:E], orc.unpack_codebook(c1_codebook), xr[pick], sel[pick], w[pick], hidden, inter)
+    assert rel_l2(y.cpu().numpy()[pick], ref) <= TOL
+
+
+@pytest.mark.parametrize("E,k", [(10, 1), (512, 16), (8, 8)])
+def test_grouped_workspace_serves_smaller_batches(ax, E, k):
+    """A workspace of a batch holds every batch of fewer tokens, whatever its widest class."""
+    from affinity_amd._lib import lib
+    for T in (1, 2, 5, 8, 10, 16, 20, 21, 32, 33, 40, 41, 64, 65, 80, 96, 128, 129, 4096):
+        size = lib().affx_grouped_workspace_size(T, k, E, 1024, 1024)
+        assert size > lib().affx_grouped_workspace_size(T - 1, k, E, 1024, 1024) or T == 1
