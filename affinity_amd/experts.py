@@ -22,11 +22,16 @@ from ._lib import AffxLayer, AffxMatrix, check, lib
 HIDDEN, INTER, N_EXPERTS, TOP_K, SWIGLU_LIMIT = 4096, 2048, 256, 6, 10.0   # src/engine/model.h:23-53
 
 
+# the current stream's handle without the Stream object around it (0.3 us against 2.9: a layer's token is
+# four calls of 3-4 us of launching each); not a public name, so a build without it takes the object
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream) -> int:
     if stream is None:
-        # the current stream's handle without the Stream object around it (0.3 us against 2.9: a layer's
-        # token is four calls of 3-4 us of launching each)
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        if _raw_stream is None:
+            return torch.cuda.current_stream().cuda_stream
+        return _raw_stream(torch.cuda.current_device())
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 

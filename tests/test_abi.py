@@ -147,3 +147,18 @@ def test_decode_workspace_grows_with_batch(L):
     a = L.affx_decode_workspace_size(1, 6, 4096, 2048)
     b = L.affx_decode_workspace_size(8, 6, 4096, 2048)
     assert 0 < a < b
+
+
+def test_stream_without_the_raw_handle(monkeypatch):
+    """A torch build that lacks the raw handle's private name falls back to the public stream object."""
+    import affinity_amd.experts as ax
+
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(ax, "_raw_stream", None)
+    monkeypatch.setattr(ax.torch.cuda, "current_stream", lambda: Stream())
+    assert ax._stream(None) == 77 and ax._stream(Stream()) == 77 and ax._stream(5) == 5
+    monkeypatch.setattr(ax, "_raw_stream", lambda device: 1000 + device)
+    monkeypatch.setattr(ax.torch.cuda, "current_device", lambda: 3)
+    assert ax._stream(None) == 1003

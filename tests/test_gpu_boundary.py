@@ -161,3 +161,14 @@ def test_grouped_slot_list(ax, orc, c1_codebook):
     err = rel_l2(y2, ref)
     print(f"slot list reordered rel_l2={err:.3e}")
     assert err <= TOL
+
+
+def test_default_stream_is_the_current_one(ax, monkeypatch):
+    """The handle a call without a stream runs on, by the raw handle and by the stream object."""
+    side = torch.cuda.Stream()
+    for fallback in (False, True):
+        if fallback:
+            monkeypatch.setattr(ax, "_raw_stream", None)
+        assert ax._stream(None) == torch.cuda.current_stream().cuda_stream
+        with torch.cuda.stream(side):
+            assert ax._stream(None) == side.cuda_stream
