@@ -209,7 +209,6 @@ __device__ __forceinline__ void put_tiles(Tile* tiles, const TileSet& t, uint32_
 // the expert's first slot.
 struct PlanOut {
   GroupedHdr* hdr;
-  uint32_t* offsets;
   Tile* tiles1;
   Tile* tiles2;
   uint32_t max_tiles1, max_tiles2;
@@ -241,12 +240,10 @@ __device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own
   const TileSet t1 = tile_set(tot + 1, k01, o.nrb1, o.grid, o.max_tiles1);
   const TileSet t2 = tile_set(tot + 1 + kNCls, k02, o.nrb2, o.grid, o.max_tiles2);
   if (fits && tid < n_experts) {
-    if (!own_slots) o.offsets[tid] = b0;
     put_tiles(o.tiles1, t1, tid, b0, c, tt1, tpg1, k01, v + 1);
     put_tiles(o.tiles2, t2, tid, b0, c, tt2, tpg2, k02, v + 1 + kNCls);
   }
   if (tid == 0) {
-    if (!own_slots) o.offsets[n_experts] = tot[0];
     o.hdr->n_slots = own_slots ? n_slots_in : tot[0];
 #pragma unroll
     for (int k = 0; k < kNCls; ++k) {
@@ -1267,7 +1264,7 @@ namespace {
 
 constexpr uint32_t kSplitRoom = 64;
 struct GroupedWs {
-  uint64_t hdr, offsets, run, slot_tok, slot_w, ord, hist, tiles1, tiles2, sigma, tok_sigma, zeros, xq, aq, z, total;
+  uint64_t hdr, run, slot_tok, slot_w, ord, hist, tiles1, tiles2, sigma, tok_sigma, zeros, xq, aq, z, total;
   uint32_t max_tiles1, max_tiles2;
 };
 
@@ -1311,7 +1308,6 @@ GroupedWs grouped_ws(uint32_t T, uint64_t P, uint32_t E, uint32_t hidden, uint32
   w.max_tiles2 = (uint32_t)(P / tt2 + E + 1) + kSplitRoom;
   uint64_t o = 0;
   w.hdr = o; o += a256(sizeof(GroupedHdr));
-  w.offsets = o; o += a256(4ull * (AFFX_MAX_EXPERTS + 1));
   w.run = o; o += a256(4ull * ((uint64_t)T + 1));
   w.slot_tok = o; o += a256(4 * P);
   w.slot_w = o; o += a256(4 * P);
@@ -1402,12 +1398,13 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   const uint32_t gmax = cus >= 8 ? (uint32_t)cus / 8u * 8u : 8u;
   const uint32_t k01 = widest_cls(T, P, L->n_experts, tx, L->inter / 128, gmax);
   const uint32_t k02 = widest_cls(T, P, L->n_experts, 3, L->hidden / 256, gmax);
-  const PlanOut po{(GroupedHdr*)(b + lay.hdr), (uint32_t*)(b + lay.offsets), (Tile*)(b + lay.tiles1),
-                   (Tile*)(b + lay.tiles2), lay.max_tiles1, lay.max_tiles2, L->inter / 128, L->hidden / 256, gmax};
+  const PlanOut po{(GroupedHdr*)(b + lay.hdr), (Tile*)(b + lay.tiles1), (Tile*)(b + lay.tiles2),
+                   lay.max_tiles1, lay.max_tiles2, L->inter / 128, L->hidden / 256, gmax};
   uint32_t* hist = (uint32_t*)(b + lay.hist);
   if (sel && Pp <= kSmallPairs) {
     // one workgroup instead of three launches: 7.1 us against 5.4 + 8.2 + 5.0 at 144 pairs, 11.6 against
-    // 5.2 + 8.4 + 5.4 at 1998 (kernel trace; the gaps between launches come on top)
+    // 5.2 + 8.4 + 5.4 at 1998, 13 to 15 from 3072 to 4096 against 4.8 + 8.1 + 6.2 at 5120 (kernel trace; the
+    // gaps between launches come on top)
     hipLaunchKernelGGL(grouped_plan_small_kernel, dim3(1), dim3(kPlanThreads), 0, s, sel, w, Pp, T, K, L->n_experts,
                        k01, k02, tx, tok_sigma, (uint32_t*)(b + lay.slot_tok), (float*)(b + lay.slot_w),
                        (int32_t*)(b + lay.sigma), (uint32_t*)(b + lay.ord), (uint32_t*)(b + lay.run), po);
