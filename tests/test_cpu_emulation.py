@@ -86,6 +86,14 @@ CASES = {
     "grouped": (("grouped", 1024, 1024, 5, 12, 3, 4, 1), 4),
     # tokens per expert; a class of its own for the ten tokens' light tiles would cost more than it saves
     "grouped_merged": (("grouped", 2048, 1024, 2, 40, 1, 7, 0, "30-10"), 8),
+    # every width class of both GEMMs, with two and with three terms; two sets of 1024 columns, and one
+    "grouped_wide": (("grouped", 2048, 1024, 1, 130, 1, 4, 0, "130"), 8),
+    "grouped_wide_lo": (("grouped", 1024, 1024, 1, 90, 1, 5, 1, "90"), 8),
+    # a wide tile split in an 8- and a 4-column one, with two terms (gate/up) and three (both)
+    "grouped_split": (("grouped", 1024, 1024, 3, 186, 1, 5, 0, "96-60-30"), 8),
+    "grouped_split_lo": (("grouped", 1024, 1024, 3, 105, 1, 5, 1, "60-15-30"), 8),
+    # 4800 routes: the plan and the placement in chunks
+    "grouped_chunks": (("grouped", 1024, 1024, 4, 300, 16, 6, 0, "12-5-34-70"), 8),
     "timeout": (("timeout", 1024, 1024, 6, 2, 3, 8), 4),
     # batch 1 in one pass (6 workgroups hold the 64 gate/up items): per-workgroup publish flags
     "timeout_m1": (("timeout", 1024, 1024, 6, 1, 1, 8), 6),
@@ -105,7 +113,7 @@ CASES = {
     "shared": (("shared", 1024, 1024, 6, 40, 5), 4),
 }
 # longest first, so the three lanes finish together
-ORDER = ["decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "slots", "shared", "decode_m1_single", "grouped",
+ORDER = ["grouped_wide", "grouped_wide_lo", "grouped_split", "decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "grouped_split_lo", "grouped_chunks", "slots", "shared", "decode_m1_single", "grouped",
          "decode_m1", "grouped_merged", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
          "dequant"]
 
@@ -183,7 +191,13 @@ def test_grouped_emulated(runs):
 
 # tiles of each width class (12, 8, 4 and 2 column tiles), gate/up then down, and the plan's form
 GROUPED = {
+    "grouped": "classes 0,0,0,5 0,0,0,5 small=1 chunks=0",
     "grouped_merged": "classes 0,0,2,0 0,0,3,0 small=1 chunks=0",
+    "grouped_wide": "classes 1,1,0,0 2,0,0,1 small=1 chunks=0",
+    "grouped_wide_lo": "classes 1,1,0,0 1,1,0,0 small=1 chunks=0",
+    "grouped_split": "classes 0,2,2,0 2,2,0,0 small=1 chunks=0",
+    "grouped_split_lo": "classes 0,2,2,0 0,2,2,0 small=1 chunks=0",
+    "grouped_chunks": "classes 1,1,0,2 0,2,4,0 small=0 chunks=1",
 }
 
 

@@ -261,3 +261,37 @@ def test_grouped_workspace_serves_smaller_batches(ax, E, k):
     for T in (1, 2, 5, 8, 10, 16, 20, 21, 32, 33, 40, 41, 64, 65, 80, 96, 128, 129, 4096):
         size = lib().affx_grouped_workspace_size(T, k, E, 1024, 1024)
         assert size > lib().affx_grouped_workspace_size(T - 1, k, E, 1024, 1024) or T == 1
+
+
+@pytest.mark.parametrize("lo", [False, True])
+def test_grouped_split_wide_tiles(ax, orc, c1_codebook, layer, lo):
+    """One wide tile more than a whole round of 32 (2048 x 1024: 8 row blocks over 256 workgroups), which
+    the plan splits into an 8- and a 4-column tile: every token's output the same bit for bit as in a
+    batch that is not split, the last expert's tokens against the oracle."""
+    ex, pool, hidden, inter = layer
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the round is that of 256 CUs")
+    tile = 60 if lo else 96
+    counts = [4 * tile] * 8 + [tile + (tile // 2 + 5)]
+    rng = np.random.default_rng(9 + lo)
+    T = sum(counts)
+    sel = rng.permutation(np.repeat(np.arange(9), counts)).astype(np.uint32).reshape(T, 1)
+    w = rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32)
+    xf = rng.standard_normal((T, hidden)).astype(np.float32)
+    hi = torch.from_numpy(xf).cuda().to(torch.bfloat16)
+    xlo = (torch.from_numpy(xf).cuda() - hi.float()).to(torch.bfloat16) if lo else None
+    gs, gw = torch.from_numpy(sel.view(np.int32)).cuda(), torch.from_numpy(w).cuda()
+    ws = ax.GroupedWorkspace(T, 1, pool.n_experts, hidden, inter)
+    y = ax.expert_ffn_grouped(pool, hi, gs, gw, x_lo=xlo, workspace=ws)
+    # the plan's header: slots, terms, a flag, then the tiles of each class of gate/up and of down
+    assert ws.buf[:28].view(torch.int32).tolist() == [T, 3 if lo else 2, 0, 32, 2, 1, 0]
+    if lo:
+        assert ws.buf[28:44].view(torch.int32).tolist() == [32, 2, 1, 0]
+    for a in range(0, T, 100):
+        b = min(a + 100, T)
+        part = ax.expert_ffn_grouped(pool, hi[a:b], gs[a:b], gw[a:b], x_lo=None if xlo is None else xlo[a:b])
+        assert torch.equal(part.view(torch.int32), y[a:b].view(torch.int32)), a
+    pick = np.nonzero(sel[:, 0] == 8)[0]
+    xr = (hi.float() + (xlo.float() if lo else 0)).cpu().numpy()
+    ref = _oracle(orc, ex, orc.unpack_codebook(c1_codebook), xr[pick], sel[pick], w[pick], hidden, inter)
+    assert rel_l2(y.cpu().numpy()[pick], ref) <= TOL
