@@ -170,13 +170,21 @@ __device__ uint32_t search_block(const float4* ent, uint32_t lane, const float* 
 constexpr int kQuantMaxCols = 8192;
 constexpr uint32_t kQuantChunk = 1024;
 // A chunk of 64 columns (four blocks of a product's 16 columns, and one wave of the four) is searched in
-// full: rows of 64 columns, 512 of them 186 us by products and 85 so, 2048 of them 521 and 267; of 128
+// full: rows of 64 columns, 512 of them 186 us by products and 86 so, 2048 of them 521 and 271; of 128
 // columns 154 by products and 192 so, 521 and 518.
 constexpr uint32_t kShort = 4;
+// Open settings of a wave's undecided blocks that it searches by itself: near ties leave two or three
+// of a block's 24 open in a few percent of the blocks, a codebook of tied entries two in all 16.
+constexpr uint32_t kOwnSettings = 64;
 constexpr float kU = 5.9604645e-8f;
 typedef float qv4f __attribute__((ext_vector_type(4)));
 
-// Code i of a chunk into its stream (zeroed; the codes' bits are disjoint).
+// Field i and code i of a chunk into their streams (zeroed; the bits are disjoint).
+__device__ __forceinline__ void put_field(uint32_t* fbits, uint32_t i, uint32_t field) {
+  const uint32_t at = i * 6;
+  atomicOr(&fbits[at >> 5], field << (at & 31));
+  if ((at & 31) > 26) atomicOr(&fbits[(at >> 5) + 1], field >> (32 - (at & 31)));
+}
 __device__ __forceinline__ void put_code(uint32_t* cbits, uint32_t i, uint32_t code) {
   const uint32_t at = i * 10;
   atomicOr(&cbits[at >> 5], code << (at & 31));
@@ -195,8 +203,8 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   __shared__ uint32_t cbits[kQuantChunk * 10 / 128];            // the chunk's code stream
   __shared__ uint32_t fbits[kQuantChunk * 6 / 512 + 1];         // the chunk's field stream
   __shared__ float red[8];
-  __shared__ uint2 todo[kQuantChunk / kBlock];                  // blocks left open: block | middle scale << 8, open settings
-  __shared__ uint32_t n_todo, field_s[kQuantChunk / kBlock];
+  __shared__ uint2 listed[kQuantChunk / kBlock];                // block | middle scale << 8, open settings
+  __shared__ uint32_t n_listed;
   float e2max = 0.f;
   for (uint32_t i = tid; i < kVariants * kLut; i += 256) {
     const float4 e = cb[i];
@@ -207,7 +215,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   }
   for (uint32_t i = tid; i < kQuantChunk * 10 / 128; i += 256) cbits[i] = 0;
   if (tid < kQuantChunk * 6 / 512 + 1) fbits[tid] = 0;
-  if (tid == 0) n_todo = 0;
+  if (tid == 0) n_listed = 0;
 
   const float* row = w + (uint64_t)r * cols;
   float rmax = 0.f;
@@ -362,61 +370,87 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     const uint32_t k = (uint32_t)__builtin_ctz(open), j = (k % 12u) / 4u;
     field = ((k / 12u) << 5) | ((k & 3u) << 3) | (uint32_t)(mid - 1 + (int)j);
   }
-  // the blocks left open (of a short chunk all), a wave each in turn: in any order and of the whole chunk,
-  // so that the waves whose blocks are decided, or which have none, share the work (512 x 512 with
-  // negative importances, every block open: 1272 us with each wave at its own blocks, now 741)
-  const bool listed = live && (direct || (need && (open & (open - 1u)) != 0u));
-  if (listed && kg == 0u) todo[atomicAdd(&n_todo, 1u)] = make_uint2(b | ((uint32_t)mid << 8), need ? open : 0u);
-  __syncthreads();
-  for (uint32_t i = wv; i < n_todo; i += 4) {
-    uint2 q = todo[i];
-    q.x = __builtin_amdgcn_readfirstlane(q.x);
-    q.y = __builtin_amdgcn_readfirstlane(q.y);
-    const uint32_t bq = q.x & 255u, at = c0 + bq * kBlock;
-    const uint32_t f = search_block(ent, lane, row + at, imp ? imp + at : nullptr, rscale, (int)(q.x >> 8), q.y);
-    if (lane == 0) field_s[bq] = f;
-    const float mag = rscale * (float)(1u << (f & 7u)), bs = (f & 8u) ? -mag : mag;
-    if (!direct || !(mag > 0.f)) continue;
-    // (a short chunk's codes too: the scan below would have most lanes idle)
-    const uint32_t rh = (f & 16u) ? 2u : 0u;
+  // the blocks left open, one at a time; where the chunk leaves a wave without blocks, a wave with many
+  // settings open (not near ties, but blocks that the bound does not cover) lists its for the whole workgroup
+  // instead, as a short chunk does all: in any order, a wave each in turn (512 x 512 with negative
+  // importances, every block open: 1267 us with each wave at its own, 810 so; near ties listed too cost the
+  // usual rows 2 %, as the waves then wait for each other twice)
+  const bool undecided = need && (open & (open - 1u)) != 0u;
+  uint64_t todo = __ballot(undecided && kg == 0u);
+  bool shared = direct;
+  if (todo && nblk <= 3u * kQuantChunk / kBlock / 4u) {
+    uint32_t n = undecided && kg == 0u ? (uint32_t)__popc(open) : 0u;
 #pragma unroll
-    for (uint32_t p = 0; p < 4; ++p) {
-      const float* x = row + at + 4 * p;
-      const uint32_t code = quad_argmin(ent + (f >> 5) * kLut, lane, x[rh] / bs, x[1 + rh] / bs, x[2 - rh] / bs, x[3 - rh] / bs);
-      if (lane == 0) put_code(cbits, bq * 4 + p, code);
-    }
+    for (int o = 1; o < 64; o <<= 1) n += __shfl_xor(n, o);
+    shared = shared || n > kOwnSettings;
   }
-  __syncthreads();
-  if (listed) field = field_s[b];
-
-  // ---- the codes: lane (c, kg) takes quad kg of block c --------------------------------------------
-  if (live) {
-    const float mag = rscale * (float)(1u << (field & 7u));
-    const float bs = (field & 8u) ? -mag : mag;
-    const bool rot = (field & 16u) != 0u;
-    uint32_t code = 0;
-    if (mag > 0.f && !direct) {
-      float x[4];
+  const bool is_listed = live && shared && (direct || undecided);
+  if (shared) {
+    if (is_listed && kg == 0u) listed[atomicAdd(&n_listed, 1u)] = make_uint2(b | ((uint32_t)mid << 8), need ? open : 0u);
+    todo = 0;
+  }
+  // (one loop over both: with a second call of the search in the kernel the search is slower by a third)
+#pragma clang loop unroll(disable)
+  for (int pass = 0;; ++pass) {
+    for (uint32_t i = wv;; i += 4) {
+      uint32_t bq, md, op;
+      if (pass == 0) {
+        if (!todo) break;
+        const int src = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        bq = 16u * wv + (uint32_t)src;
+        md = (uint32_t)__shfl(mid, src);
+        op = __shfl(open, src);
+      } else {
+        if (i >= n_listed) break;
+        const uint2 q = listed[i];
+        bq = __builtin_amdgcn_readfirstlane(q.x) & 255u;
+        md = __builtin_amdgcn_readfirstlane(q.x) >> 8;
+        op = __builtin_amdgcn_readfirstlane(q.y);
+      }
+      const uint32_t at = c0 + bq * kBlock;
+      const uint32_t f = search_block(ent, lane, row + at, imp ? imp + at : nullptr, rscale, (int)md, op);
+      if (pass == 0) {
+        if (b == bq) field = f;
+        continue;
+      }
+      if (lane == 0) put_field(fbits, bq, f);
+      const float mag = rscale * (float)(1u << (f & 7u)), bs = (f & 8u) ? -mag : mag;
+      if (!(mag > 0.f)) continue;
+      const uint32_t rh = (f & 16u) ? 2u : 0u;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) x[p] = blk[4 * kg + p];
-      const float t0 = (rot ? x[2] : x[0]) / bs, t1 = (rot ? x[3] : x[1]) / bs;
-      const float t2 = (rot ? x[0] : x[2]) / bs, t3 = (rot ? x[1] : x[3]) / bs;
-      const float4* ev = ent + (field >> 5) * kLut;
-      float m = 3.402823466e38f;
-#pragma unroll 8
-      for (uint32_t e = 0; e < (uint32_t)kLut; ++e) {
-        const float d = qdist(ev[e], t0, t1, t2, t3);
-        if (d < m) { m = d; code = e; }
+      for (uint32_t p = 0; p < 4; ++p) {
+        const float* x = row + at + 4 * p;
+        const uint32_t code = quad_argmin(ent + (f >> 5) * kLut, lane, x[rh] / bs, x[1 + rh] / bs, x[2 - rh] / bs, x[3 - rh] / bs);
+        if (lane == 0) put_code(cbits, bq * 4 + p, code);
       }
     }
-    if (kg == 0u) {
-      const uint32_t fpos = b * 6;
-      atomicOr(&fbits[fpos >> 5], field << (fpos & 31));
-      if ((fpos & 31) > 26) atomicOr(&fbits[(fpos >> 5) + 1], field >> (32 - (fpos & 31)));
+    if (pass == 0 && live && !is_listed) {
+      // the codes: lane (c, kg) takes quad kg of block c
+      const float mag = rscale * (float)(1u << (field & 7u));
+      const float bs = (field & 8u) ? -mag : mag;
+      const bool rot = (field & 16u) != 0u;
+      uint32_t code = 0;
+      if (mag > 0.f) {
+        float x[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) x[p] = blk[4 * kg + p];
+        const float t0 = (rot ? x[2] : x[0]) / bs, t1 = (rot ? x[3] : x[1]) / bs;
+        const float t2 = (rot ? x[0] : x[2]) / bs, t3 = (rot ? x[1] : x[3]) / bs;
+        const float4* ev = ent + (field >> 5) * kLut;
+        float m = 3.402823466e38f;
+#pragma unroll 8
+        for (uint32_t e = 0; e < (uint32_t)kLut; ++e) {
+          const float d = qdist(ev[e], t0, t1, t2, t3);
+          if (d < m) { m = d; code = e; }
+        }
+      }
+      if (kg == 0u) put_field(fbits, b, field);
+      put_code(cbits, b * 4 + kg, code);
     }
-    if (!direct) put_code(cbits, b * 4 + kg, code);
+    __syncthreads();
+    if (pass == 1 || n_listed == 0) break;  // (the whole workgroup)
   }
-  __syncthreads();
   // 64 columns are whole bytes of both streams (20 and 3), and cols % 64 == 0
   const uint32_t ncb = nblk * 5, nfb = nblk * 3 / 4;
   const uint8_t* cs = reinterpret_cast<const uint8_t*>(cbits);
