@@ -124,18 +124,29 @@ __device__ __forceinline__ uint32_t n_cls_of(uint32_t c, uint32_t tt, uint32_t t
 // 2048); at 2048 and 1024 27, 20, 15 and 12, and 28, 21, 15 and 12, and down 19, 15, 11.5 and 8.7: the
 // same ratios within a seventh. A launch's first round takes 8 to 10 us more, an empty launch 2 to 5.
 constexpr uint32_t kClsCost[kNCls] = {49, 36, 26, 21}, kClsStart = 5;
-__device__ __forceinline__ uint32_t cls_rounds(uint32_t tiles, uint32_t nrb, uint32_t grid) {
-  return ((tiles + 7u) / 8u * 8u * nrb + grid - 1u) / grid;
+// How a GEMM's tiles meet the device: row blocks of a tile, workgroups of a launch at most (and its
+// reciprocal), a light round's cost.
+struct ClsGrid {
+  uint32_t nrb, grid;
+  float inv;
+  uint32_t light;
+};
+// (all 16 waves of a plan compute these, where an integer division is some 35 instructions: by the
+// reciprocal, corrected; the items of a batch are below 2^23, see the B rows' limit)
+__device__ __forceinline__ uint32_t cls_rounds(uint32_t tiles, const ClsGrid& g) {
+  const uint32_t x = (tiles + 7u) / 8u * 8u * g.nrb + g.grid - 1u;
+  const uint32_t q = (uint32_t)((float)x * g.inv), r = x - q * g.grid;  // (q within one of x / grid)
+  return (int32_t)r < 0 ? q - 1u : r >= g.grid ? q + 1u : q;
 }
 // The wide tiles that are split into a class 1 and a class 2 tile each (12 column tiles = 8 + 4): 194 wide
 // gate/up tiles over 256 workgroups took 13 rounds for 12.1 rounds' work. They are split where the
 // round saved is worth more than those that the narrower classes grow by.
-__device__ __forceinline__ uint32_t split_wide(const uint32_t (&n)[kNCls], uint32_t nrb, uint32_t grid, uint32_t room) {
+__device__ __forceinline__ uint32_t split_wide(const uint32_t (&n)[kNCls], const ClsGrid& g, uint32_t room) {
   static_assert(kClsCT[0] == kClsCT[1] + kClsCT[2], "a wide tile is one of each");
-  auto rounds = [&](uint32_t t) { return cls_rounds(t, nrb, grid); };
+  auto rounds = [&](uint32_t t) { return cls_rounds(t, g); };
   const uint32_t r = rounds(n[0]);
   if (r == 0) return 0u;
-  const uint32_t left = n[0] - min(n[0], (r - 1u) * grid / nrb / 8u * 8u);
+  const uint32_t left = n[0] - min(n[0], (r - 1u) * g.grid / g.nrb / 8u * 8u);
   if (left > room) return 0u;
   const uint32_t more =
       (rounds(n[1] + left) - rounds(n[1])) * kClsCost[1] + (rounds(n[2] + left) - rounds(n[2])) * kClsCost[2];
@@ -144,10 +155,17 @@ __device__ __forceinline__ uint32_t split_wide(const uint32_t (&n)[kNCls], uint3
 // Whether the light tiles run in the class before them (n2 tiles) instead: where the rounds they add there
 // cost less than theirs here, as with the few experts of a small layer, whose tiles of both classes
 // fill a round together (8 experts, two of them a token, 64 tokens: the layer 83 us with two launches a
-// GEMM, 61 with one).
-__device__ __forceinline__ bool merge_light(uint32_t n2, uint32_t n3, uint32_t nrb, uint32_t grid) {
-  auto cost = [&](uint32_t n, uint32_t c) { return n ? cls_rounds(n, nrb, grid) * c + kClsStart : 0u; };
-  return n3 != 0u && cost(n2 + n3, kClsCost[2]) < cost(n2, kClsCost[2]) + cost(n3, kClsCost[3]);
+// GEMM, 61 with one). With two workgroups a CU the light class has no whole rounds past the first two
+// halves: 94 narrow and light tiles by 16 row blocks 154 us in one launch, 30 + 115 in two. A light round
+// costs less of a narrow one's where K is 1024 (down, 2 + 62 tiles by 16 row blocks: 44 + 5 us for one launch
+// and an empty one, 11 + 34 for two).
+constexpr uint32_t kLightShort = 18, kMergeGain = 4;
+__device__ __forceinline__ bool merge_light(uint32_t n2, uint32_t n3, const ClsGrid& g) {
+  if (n2 == 0u || n3 == 0u) return false;
+  auto cost2 = [&](uint32_t n) { return g.grid * (cls_rounds(n, g) * kClsCost[2] + kClsStart); };
+  const uint32_t items = (n3 + 7u) / 8u * 8u * g.nrb;
+  const uint32_t full = items <= g.grid ? g.grid : items <= 2u * g.grid ? 2u * g.grid : items;
+  return cost2(n2 + n3) + g.grid * kMergeGain <= cost2(n2) + full * g.light + g.grid * kClsStart;
 }
 // One GEMM's tiles: class k's n[k] tiles from tiles[base[k]]; the wide ones from index keep on are split,
 // their parts following the other tiles of classes 1 and 2; the light tiles follow class 2's, to which
@@ -155,8 +173,7 @@ __device__ __forceinline__ bool merge_light(uint32_t n2, uint32_t n3, uint32_t n
 struct TileSet {
   uint32_t base[kNCls], n[kNCls], keep, cls[kNCls];
 };
-__device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, uint32_t nrb, uint32_t grid,
-                                            uint32_t max_tiles) {
+__device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, const ClsGrid& g, uint32_t max_tiles) {
   TileSet t;
   uint32_t need = 0;
 #pragma unroll
@@ -164,7 +181,7 @@ __device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, ui
     t.n[k] = tot[k];
     need += tot[k];
   }
-  const uint32_t split = k0 == 0 && need <= max_tiles ? split_wide(t.n, nrb, grid, max_tiles - need) : 0u;
+  const uint32_t split = k0 == 0 && need <= max_tiles ? split_wide(t.n, g, max_tiles - need) : 0u;
   t.keep = t.n[0] - split;
   t.base[0] = 0;
   t.base[1] = t.keep;
@@ -174,7 +191,7 @@ __device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, ui
 #pragma unroll
   for (int k = 0; k < kNCls; ++k) t.cls[k] = k == 0 ? t.keep : t.n[k] + (k <= 2 ? split : 0u);
   static_assert(kNCls == 4, "the light class is the one after class 2");
-  if (k0 <= 2 && merge_light(t.cls[2], t.cls[3], nrb, grid)) {
+  if (k0 <= 2 && merge_light(t.cls[2], t.cls[3], g)) {
     t.cls[2] += t.cls[3];
     t.cls[3] = 0u;
   }
@@ -212,7 +229,7 @@ struct PlanOut {
   Tile* tiles1;
   Tile* tiles2;
   uint32_t max_tiles1, max_tiles2;
-  uint32_t nrb1, nrb2, grid;  // row blocks of a tile of each GEMM, workgroups of a GEMM's launch at most
+  ClsGrid g1, g2;
 };
 constexpr uint32_t kPlanSums = (1 + 2 * kNCls) * (kPlanThreads / 64 + 1);
 __device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own_slots, uint32_t n_slots_in,
@@ -237,8 +254,8 @@ __device__ __forceinline__ uint32_t plan_tiles(uint32_t c, uint32_t b0, bool own
   for (int k = 0; k < kNCls; ++k) { need1 += tot[1 + k]; need2 += tot[1 + kNCls + k]; }
   // a caller's overlapping ranges could ask for more tiles than the workspace holds: then no tile
   const bool fits = need1 <= o.max_tiles1 && need2 <= o.max_tiles2;
-  const TileSet t1 = tile_set(tot + 1, k01, o.nrb1, o.grid, o.max_tiles1);
-  const TileSet t2 = tile_set(tot + 1 + kNCls, k02, o.nrb2, o.grid, o.max_tiles2);
+  const TileSet t1 = tile_set(tot + 1, k01, o.g1, o.max_tiles1);
+  const TileSet t2 = tile_set(tot + 1 + kNCls, k02, o.g2, o.max_tiles2);
   if (fits && tid < n_experts) {
     put_tiles(o.tiles1, t1, tid, b0, c, tt1, tpg1, k01, v + 1);
     put_tiles(o.tiles2, t2, tid, b0, c, tt2, tpg2, k02, v + 1 + kNCls);
@@ -1399,7 +1416,9 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   const uint32_t k01 = widest_cls(T, P, L->n_experts, tx, L->inter / 128, gmax);
   const uint32_t k02 = widest_cls(T, P, L->n_experts, 3, L->hidden / 256, gmax);
   const PlanOut po{(GroupedHdr*)(b + lay.hdr), (Tile*)(b + lay.tiles1), (Tile*)(b + lay.tiles2),
-                   lay.max_tiles1, lay.max_tiles2, L->inter / 128, L->hidden / 256, gmax};
+                   lay.max_tiles1, lay.max_tiles2,
+                   ClsGrid{L->inter / 128, gmax, 1.0f / (float)gmax, L->hidden > 1024 ? kClsCost[3] : kLightShort},
+                   ClsGrid{L->hidden / 256, gmax, 1.0f / (float)gmax, L->inter > 1024 ? kClsCost[3] : kLightShort}};
   uint32_t* hist = (uint32_t*)(b + lay.hist);
   if (sel && Pp <= kSmallPairs) {
     // one workgroup instead of three launches: 7.1 us against 5.4 + 8.2 + 5.0 at 144 pairs, 11.6 against
