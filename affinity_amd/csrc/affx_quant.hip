@@ -170,9 +170,12 @@ __device__ uint32_t search_block(const float4* ent, uint32_t lane, const float* 
 constexpr int kQuantMaxCols = 8192;
 constexpr uint32_t kQuantChunk = 1024;
 // A chunk of 64 columns (four blocks of a product's 16 columns, and one wave of the four) is searched in
-// full: rows of 64 columns, 512 of them 186 us by products and 86 so, 2048 of them 521 and 271; of 128
-// columns 154 by products and 192 so, 521 and 518.
+// full, and so are rows of 128 where there are more of them than a device of 256 CUs holds workgroups of
+// the products, three a CU. Both ways, us, products and full search: 64 columns, 512 rows 186 and 85, 2048
+// rows 521 and 228; 128 columns, 512 rows 155 and 165, 768 rows 154 and 196, 1024 rows 300 and 243, 2048
+// rows 521 and 448.
 constexpr uint32_t kShort = 4;
+constexpr uint32_t kAllRows = 3 * 256 + 1;
 // Open settings of a wave's undecided blocks that it searches by itself: near ties leave two or three
 // of a block's 24 open in a few percent of the blocks, a codebook of tied entries two in all 16.
 constexpr uint32_t kOwnSettings = 64;
@@ -192,14 +195,17 @@ __device__ __forceinline__ void put_code(uint32_t* cbits, uint32_t i, uint32_t c
 }
 __device__ __forceinline__ float low_of(float a, float b) { return __builtin_fminf(a, b); }
 
-__global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
+// (kAll: every block is searched in full, which needs neither |e|^2 / 2 nor the products' registers, so a CU
+// holds four workgroups and not three)
+template <bool kAll>
+__global__ void __launch_bounds__(256, kAll ? 4 : 3) quantize_rows_kernel(
     const float* __restrict__ w, uint32_t cols, uint32_t chunks, const float4* __restrict__ cb,
     const float* __restrict__ imp, uint8_t* __restrict__ codes, uint8_t* __restrict__ fields,
     uint16_t* __restrict__ rscales) {
   const uint32_t r = blockIdx.x / chunks, ch = blockIdx.x - r * chunks;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   __shared__ float4 ent[kVariants * kLut];                      // 32 KiB
-  __shared__ __align__(16) float half[kVariants * kLut];        // |e|^2 / 2
+  __shared__ __align__(16) float half[kAll ? 4 : kVariants * kLut];  // |e|^2 / 2
   __shared__ uint32_t cbits[kQuantChunk * 10 / 128];            // the chunk's code stream
   __shared__ uint32_t fbits[kQuantChunk * 6 / 512 + 1];         // the chunk's field stream
   __shared__ float red[8];
@@ -210,7 +216,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
     const float4 e = cb[i];
     ent[i] = e;
     const float n = ((e.x * e.x + e.y * e.y) + e.z * e.z) + e.w * e.w;
-    half[i] = 0.5f * n;
+    if constexpr (!kAll) half[i] = 0.5f * n;
     e2max = fmaxf(e2max, n < 1e30f ? n : INFINITY);  // (an entry past the bound, or a NaN, leaves no bound)
   }
   for (uint32_t i = tid; i < kQuantChunk * 10 / 128; i += 256) cbits[i] = 0;
@@ -270,7 +276,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   }
   float inv[3], er[3];
   uint32_t valid = 0;  // settings there are (scale 0..7), as in search_block
-  const bool direct = nblk <= kShort;
+  const bool direct = kAll || nblk <= kShort;
   bool sane = !direct && e2max > 1e-20f && e2max < 1e30f;
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
@@ -303,7 +309,7 @@ __global__ void __launch_bounds__(256, 3) quantize_rows_kernel(
   for (int q = 0; q < 4; ++q) sane = sane && wt[q] >= 0.f;
 
   uint32_t open = 0;
-  if (__ballot(need && sane)) {  // (the whole wave)
+  if (!kAll && __ballot(need && sane)) {  // (the whole wave)
     float ea[24];  // errors of the settings over bs(j = 0)^2
     for (uint32_t v = 0; v < 2; ++v) {
       float m[24][2];
@@ -487,11 +493,13 @@ int affx_quantize_matrix(const void* w, uint32_t rows, uint32_t cols, const void
     return set_error(AFFX_ERR_ARG, "quantize_matrix: cols must be a multiple of 64 and <= %d",
                      kQuantMaxCols);
   const uint32_t chunks = (cols + kQuantChunk - 1) / kQuantChunk;
+  const bool all = cols <= 64 || (cols <= 128 && rows >= kAllRows);
+  auto* kernel = all ? quantize_rows_kernel<true> : quantize_rows_kernel<false>;
   // (a launch holds at most 2^32 threads: a matrix of millions of long rows takes several)
   const uint32_t slab = (1u << 23) / chunks;
   for (uint32_t r0 = 0; r0 < rows;) {
     const uint32_t n = rows - r0 < slab ? rows - r0 : slab;
-    hipLaunchKernelGGL(quantize_rows_kernel, dim3(n * chunks), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(kernel, dim3(n * chunks), dim3(256), 0, (hipStream_t)stream,
                        (const float*)w + (uint64_t)r0 * cols, cols, chunks, (const float4*)codebook_f32,
                        (const float*)importance, (uint8_t*)codes + (uint64_t)r0 * (cols / 32u * 10u),
                        (uint8_t*)fields + (uint64_t)r0 * (cols / 64u * 3u), (uint16_t*)rscales + r0);

@@ -83,6 +83,8 @@ CASES = {
     "quant_tiny_blocks": (("quant", 3, 1024, 5, 1e-21, 1e-21, 0, 1), 4),
     # a chunk of 1024 columns and one of 64, whose four blocks are searched in full
     "quant_short": (("quant", 2, 1088, 6), 4),
+    # rows of 64 columns: the form without the products
+    "quant_all": (("quant", 3, 64, 8), 4),
     # importances below zero: every block searched in full, by all waves of a half chunk's workgroup
     "quant_listed": (("quant", 2, 512, 4, 1, 1, -1, 0), 4),
     "grouped": (("grouped", 1024, 1024, 5, 12, 3, 4, 1), 4),
@@ -116,7 +118,7 @@ CASES = {
 }
 # longest first, so the three lanes finish together
 ORDER = ["grouped_wide", "grouped_wide_lo", "grouped_split", "decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "grouped_split_lo", "grouped_chunks", "slots", "shared", "decode_m1_single", "grouped",
-         "decode_m1", "grouped_merged", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "quant_listed", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
+         "decode_m1", "grouped_merged", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "quant_all", "quant_listed", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
          "dequant"]
 
 
@@ -182,7 +184,7 @@ def test_quantizer_emulated(runs):
     assert "exact=1" in result(runs, "quant")
 
 
-@pytest.mark.parametrize("case", ["quant_tiny", "quant_tiny_blocks", "quant_short", "quant_listed"])
+@pytest.mark.parametrize("case", ["quant_tiny", "quant_tiny_blocks", "quant_short", "quant_all", "quant_listed"])
 def test_quantizer_emulated_edges(runs, case):
     assert "exact=1" in result(runs, case)
 

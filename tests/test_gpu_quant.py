@@ -146,3 +146,21 @@ def test_quantizer_open_blocks_match_oracle(ax, orc, c1_codebook, cols):
         np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
         np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
         np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 64), (768, 128), (769, 128)])
+def test_quantizer_short_rows_match_oracle(ax, orc, c1_codebook, rows, cols):
+    """Rows of 64 and 128 columns, bit for bit, on both sides of the row count from which those of 128 are
+    searched in full; with and without importances, with rows and blocks of zeros."""
+    rng = np.random.default_rng(rows)
+    w = (0.02 * rng.standard_normal((rows, cols))).astype(np.float32)
+    w[1, 16:32] = 0
+    w[2] = 0
+    cb = ax.codebook_floats(c1_codebook)
+    for imp in (None, rng.uniform(0.1, 1.1, cols).astype(np.float32)):
+        want = orc.quantize(w, cb.reshape(-1), imp)
+        codes, fields, rs = ax.quantize_matrix(torch.from_numpy(w).cuda(), torch.from_numpy(cb).cuda(),
+                                               None if imp is None else torch.from_numpy(imp).cuda())
+        np.testing.assert_array_equal(rs.cpu().numpy().view(np.uint16), np.asarray(want[2]).view(np.uint16))
+        np.testing.assert_array_equal(fields.cpu().numpy(), np.asarray(want[1]).view(np.uint8))
+        np.testing.assert_array_equal(codes.cpu().numpy(), np.asarray(want[0]).view(np.uint8))
