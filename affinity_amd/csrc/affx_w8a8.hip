@@ -221,6 +221,16 @@ __global__ void __launch_bounds__(NW * 64, NW / 2) w8a8_gemm_kernel(W8a8Args A) 
   const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t nct = A.cols / kTileCols, nrt = A.rows / kTileRows;
   const W8Order o{(nrt + NW - 1) / NW, A.cap > kW8Cols ? A.cap / kW8Cols : 1u, A.items};
+  // The codebook: in a launch of few items first, as it waits for no descriptor (one tile of one token, 2048 x
+  // 1024, 5.1 us with it after the weights, 4.7 so; 2048 x 4096 11.0 and 10.7), else after the first weights,
+  // which are the bound (64 tiles of 5 tokens, 4096 x 2048, 49.1 us and 51.2 with it first).
+  constexpr int kPer = 2048 / kW8T;
+  uint32_t cbv[kPer];
+  auto codebook = [&]() {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8T];
+  };
+  if constexpr (NW < kW8Waves) codebook();
   uint32_t r = 0;
   W8Item I;
   if (!w8_seek<NW>(A, o, r, wv, I)) return;  // (the whole workgroup)
@@ -236,13 +246,8 @@ __global__ void __launch_bounds__(NW * 64, NW / 2) w8a8_gemm_kernel(W8a8Args A) 
   Unit ua, ub;
   load(ua, I, 0);
   stage(I, 0, xb0, xs0);
-  {
-    constexpr int kPer = 2048 / kW8T;
-    uint32_t cbv[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) cbv[i] = A.codebook[tid + (uint32_t)i * kW8T];
-    build_lut<kW8KC, kW8T, kPer, true>(lut_s, cbv, tid);
-  }
+  if constexpr (NW == kW8Waves) codebook();
+  build_lut<kW8KC, kW8T, kPer, true>(lut_s, cbv, tid);
   __builtin_amdgcn_s_waitcnt(AFFX_VMCNT(0));
   __syncthreads();
 
@@ -341,7 +346,7 @@ extern "C" int affx_expert_gemm_w8a8(const affx_expert_tile* tiles, uint32_t n_t
       (rc = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute")))
     return rc;
   // A launch of few items is bound by one item's latency: where there is a CU for each half of them, items
-  // of 64 rows (a wave a SIMD: one token, 2048 x 4096, 14.1 us in items of 128 rows, 11.0 so).
+  // of 64 rows (a wave a SIMD: one token, 2048 x 4096, 14.1 us in items of 128 rows, 10.7 so).
   const uint64_t half = (uint64_t)n_tiles * ((rows / kTileRows + kW8Waves / 2 - 1) / (kW8Waves / 2)) * nch;
   const bool few = half <= (uint64_t)(cus > 0 ? cus : 1) && half > items;
   A.items = (uint32_t)(few ? half : items);
