@@ -125,7 +125,7 @@ __device__ __forceinline__ uint32_t n_cls_of(uint32_t c, uint32_t tt, uint32_t t
 // same ratios within a seventh. A launch's first round takes 8 to 10 us more, an empty launch 2 to 5.
 constexpr uint32_t kClsCost[kNCls] = {49, 36, 26, 21}, kClsStart = 5;
 // How a GEMM's tiles meet the device: row blocks of a tile, workgroups of a launch at most (and its
-// reciprocal), a light round's cost.
+// reciprocal), a light round's cost (0: the light class is not launched, see light_cost).
 struct ClsGrid {
   uint32_t nrb, grid;
   float inv;
@@ -191,7 +191,7 @@ __device__ __forceinline__ TileSet tile_set(const uint32_t* tot, uint32_t k0, co
 #pragma unroll
   for (int k = 0; k < kNCls; ++k) t.cls[k] = k == 0 ? t.keep : t.n[k] + (k <= 2 ? split : 0u);
   static_assert(kNCls == 4, "the light class is the one after class 2");
-  if (k0 <= 2 && merge_light(t.cls[2], t.cls[3], g)) {
+  if (k0 <= 2 && (g.light == 0u || merge_light(t.cls[2], t.cls[3], g))) {
     t.cls[2] += t.cls[3];
     t.cls[3] = 0u;
   }
@@ -1309,6 +1309,17 @@ uint32_t widest_cls(uint32_t T, uint64_t P, uint32_t E, uint32_t terms, uint32_t
   return k;
 }
 
+// A light round's cost, 0 where the light tiles join the four-column ones whatever the routes: with at most
+// two rounds of partial tiles (one an expert) and some of them of four columns, a class of their own never
+// pays by merge_light's costs, and an empty launch is 2 us (64 experts of 2048 x 1024, top 4, 1024 tokens:
+// 170.4 us with the launches, 166.9 without the class). The mean of four columns of tokens an expert keeps
+// batches whose tiles are all light out.
+uint32_t light_cost(uint64_t P, uint32_t E, uint32_t k0, uint32_t terms, uint32_t nrb, uint32_t grid, uint32_t k) {
+  const uint64_t items = (uint64_t)(E + 7u) / 8u * 8u * nrb;
+  if (k0 <= 2u && items <= 2u * grid && P >= (uint64_t)E * kClsCT[2] * (16 / terms)) return 0u;
+  return k > 1024 ? kClsCost[3] : kLightShort;
+}
+
 // chunks of the routes form's placement: they cover the routes and the run entries 0 .. T
 uint64_t place_chunks(uint32_t T, uint64_t P) {
   const uint64_t n = P > T ? P : (uint64_t)T + 1;
@@ -1417,8 +1428,10 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   const uint32_t k02 = widest_cls(T, P, L->n_experts, 3, L->hidden / 256, gmax);
   const PlanOut po{(GroupedHdr*)(b + lay.hdr), (Tile*)(b + lay.tiles1), (Tile*)(b + lay.tiles2),
                    lay.max_tiles1, lay.max_tiles2,
-                   ClsGrid{L->inter / 128, gmax, 1.0f / (float)gmax, L->hidden > 1024 ? kClsCost[3] : kLightShort},
-                   ClsGrid{L->hidden / 256, gmax, 1.0f / (float)gmax, L->inter > 1024 ? kClsCost[3] : kLightShort}};
+                   ClsGrid{L->inter / 128, gmax, 1.0f / (float)gmax,
+                           light_cost(P, L->n_experts, k01, tx, L->inter / 128, gmax, L->hidden)},
+                   ClsGrid{L->hidden / 256, gmax, 1.0f / (float)gmax,
+                           light_cost(P, L->n_experts, k02, 3, L->hidden / 256, gmax, L->inter)}};
   uint32_t* hist = (uint32_t*)(b + lay.hist);
   if (sel && Pp <= kSmallPairs) {
     // one workgroup instead of three launches: 7.1 us against 5.4 + 8.2 + 5.0 at 144 pairs, 11.6 against
@@ -1456,25 +1469,25 @@ int grouped_body(const affx_layer* L, const void* x, const void* x_lo, uint32_t 
   A.tiles = (const Tile*)(b + lay.tiles1);
   A.max_tiles = lay.max_tiles1;
   A.b_off = lay.xq;
-  auto each_cls = [&](auto ph, auto txc, uint32_t k0, uint32_t row_blocks, uint32_t max_tiles) {
+  auto each_cls = [&](auto ph, auto txc, uint32_t k0, const ClsGrid& cg, uint32_t max_tiles) {
     constexpr int PH = decltype(ph)::value, TX = decltype(txc)::value;
     const uint32_t part = L->n_experts + kSplitRoom < max_tiles ? L->n_experts + kSplitRoom : max_tiles;
     static_for<0, kNCls>([&](auto kc) {
       constexpr int k = decltype(kc)::value, CT = kClsCT[k];
-      if ((uint32_t)k < k0) return;
-      const dim3 g(grid(row_blocks, (uint32_t)k == k0 ? max_tiles : part, GTile<CT>::kLight ? 2u : 1u));
+      if ((uint32_t)k < k0 || (GTile<CT>::kLight && cg.light == 0u)) return;
+      const dim3 g(grid(cg.nrb, (uint32_t)k == k0 ? max_tiles : part, GTile<CT>::kLight ? 2u : 1u));
       hipLaunchKernelGGL((grouped_gemm_kernel<PH, TX, CT>), g, dim3(kGT), 0, s, A);
     });
   };
   if (tx == 2)
-    each_cls(IConst<0>{}, IConst<2>{}, k01, L->inter / 128, lay.max_tiles1);
+    each_cls(IConst<0>{}, IConst<2>{}, k01, po.g1, lay.max_tiles1);
   else
-    each_cls(IConst<0>{}, IConst<3>{}, k01, L->inter / 128, lay.max_tiles1);
+    each_cls(IConst<0>{}, IConst<3>{}, k01, po.g1, lay.max_tiles1);
   if ((rc = check_launch("grouped_gemm_kernel (gate/up)"))) return rc;
   A.tiles = (const Tile*)(b + lay.tiles2);
   A.max_tiles = lay.max_tiles2;
   A.b_off = lay.aq;
-  each_cls(IConst<1>{}, IConst<3>{}, k02, L->hidden / 256, lay.max_tiles2);
+  each_cls(IConst<1>{}, IConst<3>{}, k02, po.g2, lay.max_tiles2);
   if ((rc = check_launch("grouped_gemm_kernel (down)"))) return rc;
   hipLaunchKernelGGL(grouped_combine_kernel, dim3((L->hidden / 4 + 255) / 256, T), dim3(256), 0, s,
                      (const float*)(b + lay.z), ord_d, run_d, slot_w, n_sl, L->hidden, y, accumulate);
