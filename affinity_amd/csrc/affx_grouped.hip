@@ -1309,11 +1309,12 @@ uint32_t widest_cls(uint32_t T, uint64_t P, uint32_t E, uint32_t terms, uint32_t
   return k;
 }
 
-// A light round's cost, 0 where the light tiles join the four-column ones whatever the routes: with at most
-// two rounds of partial tiles (one an expert) and some of them of four columns, a class of their own never
-// pays by merge_light's costs, and an empty launch is 2 us (64 experts of 2048 x 1024, top 4, 1024 tokens:
-// 170.4 us with the launches, 166.9 without the class). The mean of four columns of tokens an expert keeps
-// batches whose tiles are all light out.
+// A light round's cost, 0 where the light tiles join the four-column ones whatever the routes: where the partial
+// tiles (one an expert) fill at most two rounds, and some of them are of four columns, a class of their own
+// saves at most 3 of kClsCost's units by merge_light's costs, and where the plan merges them its empty launch
+// is 2 us (64 experts of 2048 x 1024, top 4, 1024 tokens: 170.4 us with it in both GEMMs, 167.1 without; 448
+// shapes, none slower). A mean of four columns of tokens an expert keeps out the batches whose tiles are all
+// light.
 uint32_t light_cost(uint64_t P, uint32_t E, uint32_t k0, uint32_t terms, uint32_t nrb, uint32_t grid, uint32_t k) {
   const uint64_t items = (uint64_t)(E + 7u) / 8u * 8u * nrb;
   if (k0 <= 2u && items <= 2u * grid && P >= (uint64_t)E * kClsCT[2] * (16 / terms)) return 0u;

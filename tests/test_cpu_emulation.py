@@ -90,6 +90,8 @@ CASES = {
     "grouped": (("grouped", 1024, 1024, 5, 12, 3, 4, 1), 4),
     # tokens per expert; a class of its own for the ten tokens' light tiles would cost more than it saves
     "grouped_merged": (("grouped", 2048, 1024, 2, 40, 1, 7, 0, "30-10"), 8),
+    # eight tokens' light tile past a full one: without a launch of its own where all tiles fill two rounds
+    "grouped_no_light": (("grouped", 1024, 1024, 1, 48, 1, 9, 1, "48"), 32),
     # every width class of both GEMMs, with two and with three terms; two sets of 1024 columns, and one
     "grouped_wide": (("grouped", 2048, 1024, 1, 130, 1, 4, 0, "130"), 8),
     "grouped_wide_lo": (("grouped", 1024, 1024, 1, 90, 1, 5, 1, "90"), 8),
@@ -118,7 +120,7 @@ CASES = {
 }
 # longest first, so the three lanes finish together
 ORDER = ["grouped_wide", "grouped_wide_lo", "grouped_split", "decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "grouped_split_lo", "grouped_chunks", "slots", "shared", "decode_m1_single", "grouped",
-         "decode_m1", "grouped_merged", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "quant_all", "quant_listed", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
+         "decode_m1", "grouped_merged", "grouped_no_light", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "quant_all", "quant_listed", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
          "dequant"]
 
 
@@ -197,6 +199,7 @@ def test_grouped_emulated(runs):
 GROUPED = {
     "grouped": "classes 0,0,0,5 0,0,0,5 small=1 chunks=0",
     "grouped_merged": "classes 0,0,2,0 0,0,3,0 small=1 chunks=0",
+    "grouped_no_light": "classes 0,1,1,0 0,1,1,0 small=1 chunks=0",
     "grouped_wide": "classes 1,1,0,0 2,0,0,1 small=1 chunks=0",
     "grouped_wide_lo": "classes 1,1,0,0 1,1,0,0 small=1 chunks=0",
     "grouped_split": "classes 0,2,2,0 2,2,0,0 small=1 chunks=0",
