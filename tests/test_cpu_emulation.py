@@ -60,7 +60,7 @@ def run(emu, *args, timeout=900, cus=4):
     return out
 
 
-# Every case's arguments (and emulated CU count). The runs are started together, three at a time,
+# Every case's arguments (and emulated CU count). The runs are started together, five at a time,
 # when the first test asks for one: each is a long single-threaded-per-lane emulation, and
 # running them side by side keeps the module's wall time near the longest few.
 CASES = {
@@ -118,7 +118,7 @@ CASES = {
     "w8a8_few": (("w8a8", 1024, 1024, 7), 300),
     "shared": (("shared", 1024, 1024, 6, 40, 5), 4),
 }
-# longest first, so the three lanes finish together
+# longest first, so the lanes finish together
 ORDER = ["grouped_wide", "grouped_wide_lo", "grouped_split", "decode_m8_wide", "decode_m8_full", "decode_m6_dm16", "decode_m6", "grouped_split_lo", "grouped_chunks", "slots", "shared", "decode_m1_single", "grouped",
          "decode_m1", "grouped_merged", "grouped_no_light", "ffnptr", "ffnptr_n1", "quant", "quant_tiny", "quant_tiny_blocks", "quant_short", "quant_all", "quant_listed", "timeout", "timeout_m1", "route", "gemv", "w8a8", "w8a8_few", "steps", "decode_allpad",
          "dequant"]
@@ -126,7 +126,7 @@ ORDER = ["grouped_wide", "grouped_wide_lo", "grouped_split", "decode_m8_wide", "
 
 @pytest.fixture(scope="module")
 def runs(emu):
-    pool = ThreadPoolExecutor(max_workers=3)
+    pool = ThreadPoolExecutor(max_workers=5)
     futs = {name: pool.submit(run, emu, *CASES[name][0], cus=CASES[name][1]) for name in ORDER}
     yield futs
     for f in futs.values():
